@@ -1,0 +1,88 @@
+"""Context splits of the fused attention: each sequence takes the splits its own
+context needs. Batches of very different lengths (one token beside tens of
+thousands, more splits than one combine pass merges, the split cap, two launches of
+unequal batches), every head's rows against attention over the original words in
+float64 on the GPU. Tolerance: 1e-2 of each output row's largest magnitude (bf16
+output and bf16 softmax weights), as for the kernel's other tests."""
+
+import pytest
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+HEAD_DIM = 128
+TOL = 1e-2
+
+
+@pytest.fixture(scope="module")
+def sz():
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm GPU visible")
+    from unchainkv_amd import splitzip_cuda
+
+    assert splitzip_cuda.available(), splitzip_cuda.load_error()
+    return splitzip_cuda
+
+
+def make_batch(sz, kv_heads, contexts, seed):
+    from unchainkv_amd import workloads
+
+    shape = workloads.Shape(layers=1, kv_heads=kv_heads, head_dim=HEAD_DIM)
+    blocks = [-(-c // 16) for c in contexts]
+    kv = workloads.make_kv_layer(torch, shape, sum(blocks), seed=seed, layer=0, device="cuda",
+                                 outlier_rate=0.001)
+    tables = workloads.random_block_tables(torch, sum(blocks), blocks, seed=seed)
+    books = workloads.fit_codebook(torch, kv, tables)
+    batch = sz.PagedBatch(tables, shape.block_words, "cuda")
+    payloads = batch.new_payload_buffer()
+    assert sz.encode_top16_paged(kv, batch, payloads, batch.new_workspace(), codebooks=books)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    q = torch.randn((len(contexts), 4 * kv_heads, HEAD_DIM), generator=g,
+                    device="cuda").to(torch.bfloat16)
+    return kv, tables, books, batch, payloads, q
+
+
+def reference(kv, ids, tokens, q, kv_heads):
+    index = torch.tensor(ids, dtype=torch.int64, device=kv.device)
+    k, v = kv.index_select(1, index).reshape(2, -1, kv_heads, HEAD_DIM)[:, :tokens].double()
+    rows = q.double().reshape(kv_heads, 4, HEAD_DIM)
+    p = torch.softmax((rows[:, :, None, :] * k.permute(1, 0, 2)[:, None]).sum(-1)
+                      / HEAD_DIM ** 0.5, dim=-1)
+    return (p[..., None] * v.permute(1, 0, 2)[:, None]).sum(2).reshape(4 * kv_heads, HEAD_DIM)
+
+
+@pytest.mark.parametrize("kv_heads,contexts", [
+    (1, [1, 15, 16, 17, 33, 20000]),             # one token beside the longest
+    (1, [40000]),                                # a single sequence: the split cap
+    (2, [2113]),                                 # more splits than one combine pass
+    (3, [700, 5000, 64]),                        # odd head count
+    (8, [1500]),                                 # a single user's decode step
+    (5, [17 + 61 * i for i in range(40)]),       # more workgroups than one round
+    (1, [1 + (i * 977) % 3000 for i in range(67)]),  # two launches, 64 and 3 sequences
+])
+def test_splits_follow_each_context(sz, kv_heads, contexts):
+    print("[case] attention splits", kv_heads, contexts[:8], flush=True)
+    kv, tables, books, batch, payloads, q = make_batch(sz, kv_heads, contexts, 7)
+    out = sz.decode_attention_top16(q, payloads, batch.out_offsets, contexts, kv_heads,
+                                    codebooks=books)
+    torch.cuda.synchronize()
+    assert out is not None
+    got = out.double()
+    for b, (ids, tokens) in enumerate(zip(tables, contexts)):
+        ref = reference(kv, ids, tokens, q[b], kv_heads)
+        err = (got[b] - ref).abs().amax(dim=-1)
+        scale = ref.abs().amax(dim=-1).clamp_min(1e-6)
+        assert (err <= TOL * scale).all(), (b, tokens, float((err / scale).max()))
+
+
+def test_workspace_of_the_largest_batch_serves_smaller_ones(sz):
+    """The workspace size grows with the batch and with the longest context, so one
+    workspace can be kept while a batch shrinks and its contexts grow."""
+    sizes = [[sz.decode_attention_workspace_bytes(b, heads, ctx) for ctx in
+              (1, 17, 500, 1500, 8192, 8193, 40000)] for heads in (1, 8) for b in (1, 3, 32, 64, 90)]
+    for row in sizes:
+        assert row == sorted(row)
+    for heads_rows in (sizes[:5], sizes[5:]):
+        for column in zip(*heads_rows):
+            assert list(column) == sorted(column)

@@ -42,6 +42,7 @@
 // partials) rather than silently wrong.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdint>
 #include <mutex>
@@ -75,7 +76,9 @@ __device__ __forceinline__ constexpr unsigned int row_pos(unsigned int d) {
 constexpr int kWaveLds = 2 * kStep * kKStride;  // u16 per wave: K and V of a step, token-major
 constexpr int kMaxSeqs = 64;                // sequences per launch (kernel arguments)
 constexpr int kPartial = kHeadDim + 2;      // m, l, acc[128] per (split, query head)
-constexpr int kMaxSplits = 64;
+// Context splits of one sequence at most: four batches of kCombineParts *
+// kCombineBatch partials in the combine kernel.
+constexpr unsigned int kMaxSplits = 256;
 constexpr int kCheck = 8;                   // escape-order pairs per thread held through the walk
 // Independent accumulator chains of the PV product: one chain keeps the kernel at
 // 125 VGPRs (4 waves per SIMD); two reached 128 with a spill and ran 1 us slower.
@@ -87,13 +90,18 @@ struct AttnArgs {
   uint16_t* out;                 // [batch][q_heads][128] bf16
   const unsigned char* payloads;
   const unsigned char* tables;   // 544 B; K codebook at +512, V at +528
-  float* partial;                // [batch][kv_heads][splits][kGroup][kPartial]
-  unsigned int batch, q_heads, kv_heads, splits, tokens_per_wave;
+  // [split of the launch][kv_heads][kGroup][kPartial]; sequence b's splits are
+  // first_split[b] .. first_split[b + 1)
+  float* partial;
+  unsigned int batch, q_heads, kv_heads;
+  unsigned int uniform_splits;   // splits of every sequence when all are equal, else 0
   float scale_log2;              // scale * log2(e)
   unsigned int head_magic;       // 2^24 / kv_heads + 1
   unsigned long long offset[kMaxSeqs];  // payload byte offset of each sequence
   unsigned int ctx[kMaxSeqs];           // context tokens of each sequence
   unsigned int span[kMaxSeqs];          // tokens the payload holds (whole blocks, >= ctx)
+  unsigned int tpw[kMaxSeqs];           // tokens per wave range of each sequence
+  unsigned int first_split[kMaxSeqs + 1];
 };
 
 __device__ __forceinline__ unsigned int bf16_bits(float v) {
@@ -437,7 +445,10 @@ top16_attention_split(AttnArgs a) {
 
   const unsigned int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   // work item = (sequence, split, head group) with the group fastest, each XCD
-  // taking a contiguous run of items (xcd_remap). Waves r, r + kRanges, ... serve
+  // taking a contiguous run of items (xcd_remap). Sequences have as many splits as
+  // their own contexts need, so a split's sequence is found by one division when
+  // all have the same count, else by one ballot over the sequences' first splits
+  // (one per lane: a single round trip). Waves r, r + kRanges, ... serve
   // range r of the group's heads: the heads' rows of one token are adjacent in the
   // payload (body kHeads * 128 bytes, codes kHeads * 64), which the group's waves
   // then read together.
@@ -445,8 +456,18 @@ top16_attention_split(AttnArgs a) {
   const unsigned int groups = (hkv + kHeads - 1) / kHeads;
   const unsigned int w_item = xcd_remap(blockIdx.x, gridDim.x);
   const unsigned int hg = w_item % groups;
-  const unsigned int split = (w_item / groups) % a.splits;
-  const unsigned int b = w_item / (groups * a.splits);
+  const unsigned int item = w_item / groups;  // split of the launch
+  unsigned int b;
+  if (a.uniform_splits) {
+    b = item / a.uniform_splits;
+  } else {
+    const unsigned int begin = lane < a.batch ? a.first_split[lane] : 0xFFFFFFFFu;
+    b = uniform((unsigned int)__popcll(__ballot(begin <= item)) - 1u);
+  }
+  const unsigned int split0 = a.first_split[b];
+  const unsigned int splits = a.first_split[b + 1] - split0;
+  const unsigned int split = item - split0;
+  const unsigned int tpw = a.tpw[b];
   const unsigned int h = kHeads * hg + wave / kRanges;
   const unsigned int range = wave % kRanges;
   const bool head_ok = h < hkv;  // the last group may be partly empty
@@ -461,14 +482,14 @@ top16_attention_split(AttnArgs a) {
                                     ((unsigned int)payload[3] << 16) |
                                     ((unsigned int)payload[4] << 24);
   const unsigned int row_words = hkv * kHeadDim;  // payload words per token per plane
-  const unsigned int wb = (split * kRanges + range) * a.tokens_per_wave;
+  const unsigned int wb = (split * kRanges + range) * tpw;
   StepConst c;
   c.entries = entries;
   c.count = min(header_count, cap);
   c.half = (unsigned int)(n / 2);
   c.row_words = row_words;
   c.head = h;
-  c.we = head_ok ? min(ctx, wb + a.tokens_per_wave) : wb;
+  c.we = head_ok ? min(ctx, wb + tpw) : wb;
   c.kv_heads = hkv;
   c.head_magic = a.head_magic;
   c.scale_log2 = a.scale_log2;
@@ -508,7 +529,7 @@ top16_attention_split(AttnArgs a) {
   // + kCheck; their loads go out now and are compared once the walk's first loads
   // are in flight, so they add no round trip of their own (entries past chk_last
   // repeat its position).
-  const unsigned int chk_groups = a.splits * groups, chk_g = split * groups + hg;
+  const unsigned int chk_groups = splits * groups, chk_g = split * groups + hg;
   const unsigned int chk_chunk = (c.count + chk_groups - 1) / chk_groups;
   const unsigned int chk_first = min(chk_g * chk_chunk, c.count);
   const unsigned int chk_last = min(chk_first + chk_chunk, c.count > 0 ? c.count - 1 : 0u);
@@ -526,8 +547,8 @@ top16_attention_split(AttnArgs a) {
   unsigned int steps_max = 0;
 #pragma unroll
   for (int r = 0; r < kRanges; ++r) {
-    const unsigned int s0 = (split * kRanges + r) * a.tokens_per_wave;
-    const unsigned int e0 = min(ctx, s0 + a.tokens_per_wave);
+    const unsigned int s0 = (split * kRanges + r) * tpw;
+    const unsigned int e0 = min(ctx, s0 + tpw);
     steps_max = max(steps_max, e0 > s0 ? (e0 - s0 + kStep - 1) / kStep : 0u);
   }
   const unsigned int steps = wb < c.we ? (c.we - wb + kStep - 1) / kStep : 0u;
@@ -639,7 +660,7 @@ top16_attention_split(AttnArgs a) {
         }
       }
       float* dst = a.partial +
-                   ((((unsigned long long)b * hkv + hm) * a.splits + split) * kGroup + j) * kPartial;
+                   (((unsigned long long)item * hkv + hm) * kGroup + j) * kPartial;
 #pragma unroll
       for (int k = 0; k < kVals; ++k) dst[2 + d0 + k] = bad ? NAN : o[k];
       if (u % kPerRow == 0) {
@@ -656,30 +677,38 @@ top16_attention_split(AttnArgs a) {
 // read in batches of kCombineBatch with every load of a batch issued before any is
 // used (one memory round trip per batch; a loop over the splits waited for each
 // load in turn); with a single batch the sums run in split order against the
-// global max.
+// global max. kParts thread groups of kHeadDim take every kParts-th batch and are
+// merged through LDS, so that a long sequence's many splits still cost few round
+// trips (64 splits: one).
 constexpr int kCombineBatch = 16;
+constexpr int kCombineParts = 4;
 
-__global__ __launch_bounds__(kHeadDim) void top16_attention_combine(AttnArgs a) {
-  const unsigned int qh = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
+template <int kParts>
+__global__ __launch_bounds__(kHeadDim * kParts) void top16_attention_combine(AttnArgs a) {
+  constexpr unsigned int kThreads = kHeadDim * kParts;
+  const unsigned int qh = blockIdx.x, b = blockIdx.y, tid = threadIdx.x;
+  const unsigned int d = tid % kHeadDim, part_id = tid / kHeadDim;
   const unsigned int h = qh / kGroup, g = qh % kGroup;
-  const float* seq = a.partial + (unsigned long long)b * a.kv_heads * a.splits * kGroup * kPartial;
-  // the running max of the sequence's partials d, d + kHeadDim, ... (kv heads x
+  const unsigned int split0 = a.first_split[b], splits = a.first_split[b + 1] - split0;
+  const unsigned long long stride = (unsigned long long)a.kv_heads * kGroup * kPartial;
+  const float* seq = a.partial + split0 * stride;
+  // the running max of the sequence's partials tid, tid + kThreads, ... (kv heads x
   // splits of them): the first four loaded now, tested after the merge
   float flag[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const unsigned int k = d + j * kHeadDim;
-    flag[j] = k < a.kv_heads * a.splits ? seq[(unsigned long long)k * kGroup * kPartial] : 0.f;
+    const unsigned int k = tid + j * kThreads;
+    flag[j] = k < a.kv_heads * splits ? seq[(unsigned long long)k * kGroup * kPartial] : 0.f;
   }
-  const float* part = seq + (unsigned long long)h * a.splits * kGroup * kPartial + g * kPartial;
+  const float* part = seq + (h * kGroup + g) * kPartial;
   float big = -INFINITY, num = 0.f, den = 0.f;
-  for (unsigned int s0 = 0; s0 < a.splits; s0 += kCombineBatch) {
+  for (unsigned int s0 = part_id * kCombineBatch; s0 < splits; s0 += kParts * kCombineBatch) {
     float m[kCombineBatch], l[kCombineBatch], v[kCombineBatch];
 #pragma unroll
     for (int k = 0; k < kCombineBatch; ++k) {
       // splits past the last one load split s0 again and are ignored
-      const bool in = s0 + k < a.splits;
-      const float* p = part + (unsigned long long)(in ? s0 + k : s0) * kGroup * kPartial;
+      const bool in = s0 + k < splits;
+      const float* p = part + (in ? s0 + k : s0) * stride;
       m[k] = p[0];
       l[k] = p[1];
       v[k] = p[2 + d];
@@ -706,11 +735,32 @@ __global__ __launch_bounds__(kHeadDim) void top16_attention_combine(AttnArgs a) 
   int flagged = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) flagged |= isnan(flag[j]) ? 1 : 0;
-  for (unsigned int k = d + 4 * kHeadDim; k < a.kv_heads * a.splits; k += kHeadDim)
+  for (unsigned int k = tid + 4 * kThreads; k < a.kv_heads * splits; k += kThreads)
     flagged |= isnan(seq[(unsigned long long)k * kGroup * kPartial]) ? 1 : 0;
-  const bool bad = __syncthreads_or(flagged) != 0;
-  a.out[((unsigned long long)b * a.q_heads + qh) * kHeadDim + d] =
-      (uint16_t)bf16_bits(bad ? NAN : num / den);
+  if constexpr (kParts > 1) {
+    __shared__ float s_m[kParts][kHeadDim], s_num[kParts][kHeadDim], s_den[kParts][kHeadDim];
+    s_m[part_id][d] = big;
+    s_num[part_id][d] = num;
+    s_den[part_id][d] = den;
+    const bool bad = __syncthreads_or(flagged) != 0;
+    if (part_id != 0) return;
+#pragma unroll
+    for (int k = 1; k < kParts; ++k) big = fmaxf(big, s_m[k][d]);
+    num = den = 0.f;
+#pragma unroll
+    for (int k = 0; k < kParts; ++k) {
+      if (s_m[k][d] == -INFINITY) continue;  // a group with no splits
+      const float wgt = exp2f(s_m[k][d] - big);
+      den += s_den[k][d] * wgt;
+      num += s_num[k][d] * wgt;
+    }
+    a.out[((unsigned long long)b * a.q_heads + qh) * kHeadDim + d] =
+        (uint16_t)bf16_bits(bad ? NAN : num / den);
+  } else {
+    const bool bad = __syncthreads_or(flagged) != 0;
+    a.out[((unsigned long long)b * a.q_heads + qh) * kHeadDim + d] =
+        (uint16_t)bf16_bits(bad ? NAN : num / den);
+  }
 }
 
 }  // namespace
@@ -742,36 +792,91 @@ unsigned long long resident_workgroups() {
   return cached[dev];
 }
 
-struct SplitPlan {
-  unsigned int groups;           // workgroups per (sequence, split)
-  unsigned int splits, tokens_per_wave;
-};
+// Workgroups per context split: every kv head, kHeads of them per workgroup.
+unsigned long long head_groups(unsigned long long kv_heads) {
+  return (kv_heads + kHeads - 1) / kHeads;
+}
 
-// Context splits per (sequence, head group): the count whose workgroups fill whole
-// rounds of the resident slots with the fewest tokens per wave (a wave walks its
-// range serially; a round that is partly empty wastes the rest of the chip). A split
-// gives every head kRanges token ranges of tokens_per_wave.
-SplitPlan plan_splits(unsigned long long sequences, unsigned long long kv_heads,
-                      unsigned long long max_ctx) {
-  SplitPlan best{(unsigned int)((kv_heads + kHeads - 1) / kHeads), 1, 0};
-  const unsigned long long ranges = kRanges;
-  const unsigned long long per_split = sequences * best.groups;
-  const unsigned long long slots = resident_workgroups();
+// Splits of all sequences of a launch together, at most: two rounds of the resident
+// workgroups and one split per sequence, and no more than one step per wave. Grows
+// with each argument, so a workspace made for the largest batch and context serves
+// the smaller ones.
+unsigned long long max_launch_splits(unsigned long long sequences, unsigned long long kv_heads,
+                                     unsigned long long max_ctx) {
+  const unsigned long long per_seq = (max_ctx + kRanges * kStep - 1) / (kRanges * kStep);
+  return std::min(sequences * std::min<unsigned long long>(per_seq, kMaxSplits),
+                  2 * resident_workgroups() / head_groups(kv_heads) + sequences);
+}
+
+// Splits of every sequence with at most `tpw` tokens per wave.
+unsigned long long count_splits(const unsigned long long* ctx, unsigned int count,
+                                unsigned int tpw) {
+  const unsigned int per_split = tpw * kRanges;
+  unsigned long long splits = 0;
+  for (unsigned int r = 0; r < count; ++r) splits += ((unsigned int)ctx[r] + per_split - 1) / per_split;
+  return splits;
+}
+
+// Fills the launch's splits (a.tpw, a.first_split, a.uniform_splits) from the
+// sequences' own context lengths: a split gives every head kRanges token ranges, and
+// a sequence takes as many splits as keep its ranges within the launch's tokens per
+// wave. That number is the smallest whose workgroups fit k rounds of the resident
+// slots, for the k with the least work in a row (a wave walks its range serially, a
+// round lasts as long as its longest range): k rounds of (tpw + kWaveOverhead)
+// token steps. Sized for the longest sequence instead, with equal splits per
+// sequence, a batch of mixed lengths left most of its workgroups empty: 64 sequences
+// of 128 to 32768 tokens, one kv head, 117 -> 43 us per call (185 MB of packed KV);
+// one 1500-token sequence of 8 kv heads, 18.4 -> 12.8 us (8 -> 47 splits); 32 equal
+// sequences of 8192 tokens take the same splits as before (144 us).
+unsigned int plan_splits(AttnArgs& a, const unsigned long long* ctx, unsigned int count,
+                         unsigned long long max_ctx) {
+  const unsigned long long groups = head_groups(a.kv_heads), slots = resident_workgroups();
+  const unsigned long long limit = max_launch_splits(count, a.kv_heads, max_ctx);
   constexpr unsigned long long kWaveOverhead = 32;  // start-up cost in token steps
+  unsigned long long total = 0;
+  for (unsigned int r = 0; r < count; ++r) total += ctx[r];
+  const unsigned int most =
+      (unsigned int)((max_ctx + kRanges * kStep - 1) / (kRanges * kStep));  // steps: one split each
+  // at most kMaxSplits per sequence
+  const unsigned int least = (unsigned int)((max_ctx + (unsigned long long)kRanges * kStep * kMaxSplits - 1) /
+                                            ((unsigned long long)kRanges * kStep * kMaxSplits));
+  unsigned int best = most;
   unsigned long long best_cost = ~0ull;
-  for (unsigned int s = 1; s <= kMaxSplits; ++s) {
-    const unsigned long long per_wave = (max_ctx + ranges * s - 1) / (ranges * s);
-    const unsigned long long tpw = (per_wave + kStep - 1) / kStep * kStep;
-    if (s > 1 && (unsigned long long)(s - 1) * ranges * tpw >= max_ctx) break;  // empty splits
-    const unsigned long long rounds = (per_split * s + slots - 1) / slots;
-    const unsigned long long cost = rounds * (tpw + kWaveOverhead);
+  const unsigned long long k0 = (count * groups + slots - 1) / slots;
+  for (unsigned long long k = k0; k < k0 + 3; ++k) {
+    const unsigned long long fit = std::min(k * slots / groups, std::max<unsigned long long>(limit, count));
+    // smallest number of steps per range whose splits fit
+    unsigned int lo = least, hi = most;
+    const unsigned long long floor_steps = total / (fit * kRanges * kStep);
+    if (floor_steps > lo) lo = (unsigned int)std::min<unsigned long long>(floor_steps, most);
+    while (lo < hi) {
+      const unsigned int mid = lo + (hi - lo) / 2;
+      if (count_splits(ctx, count, mid * kStep) <= fit)
+        hi = mid;
+      else
+        lo = mid + 1;
+    }
+    const unsigned long long cost = k * ((unsigned long long)lo * kStep + kWaveOverhead);
     if (cost < best_cost) {
       best_cost = cost;
-      best.splits = s;
-      best.tokens_per_wave = (unsigned int)tpw;
+      best = lo;
     }
   }
-  return best;
+  // even ranges within each sequence
+  unsigned int splits = 0, largest = 0, smallest = ~0u;
+  for (unsigned int r = 0; r < count; ++r) {
+    const unsigned int c = (unsigned int)ctx[r];
+    const unsigned int want = (c + best * kStep * kRanges - 1) / (best * kStep * kRanges);
+    a.tpw[r] = (c + want * kRanges * kStep - 1) / (want * kRanges * kStep) * kStep;
+    const unsigned int own = (c + a.tpw[r] * kRanges - 1) / (a.tpw[r] * kRanges);
+    a.first_split[r] = splits;
+    splits += own;
+    largest = std::max(largest, own);
+    smallest = std::min(smallest, own);
+  }
+  a.first_split[count] = splits;
+  a.uniform_splits = largest == smallest ? largest : 0;
+  return largest;
 }
 
 }  // namespace
@@ -782,8 +887,8 @@ extern "C" unsigned long long kvq_splitzip_top16_decode_attention_workspace_byte
     unsigned long long batch, unsigned long long kv_heads, unsigned long long max_ctx) {
   if (batch == 0 || kv_heads == 0 || max_ctx == 0) return 0;
   const unsigned long long per_launch = batch < kMaxSeqs ? batch : kMaxSeqs;
-  const SplitPlan plan = plan_splits(per_launch, kv_heads, max_ctx);
-  return per_launch * kv_heads * plan.splits * kGroup * kPartial * sizeof(float);
+  return max_launch_splits(per_launch, kv_heads, max_ctx) * kv_heads * kGroup * kPartial *
+         sizeof(float);
 }
 
 // Decode attention of one query token per sequence over Top-16 packed KV (no
@@ -815,8 +920,6 @@ extern "C" long long kvq_splitzip_top16_decode_attention(
   if (kvq_splitzip_top16_decode_attention_workspace_bytes(batch, kv_heads, max_ctx) >
       workspace_bytes)
     return 0;
-  const unsigned long long per_launch = batch < kMaxSeqs ? batch : kMaxSeqs;
-  const SplitPlan plan = plan_splits(per_launch, kv_heads, max_ctx);
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
   for (unsigned long long first = 0; first < batch; first += kMaxSeqs) {
     const unsigned int count = (unsigned int)(batch - first < kMaxSeqs ? batch - first : kMaxSeqs);
@@ -829,8 +932,6 @@ extern "C" long long kvq_splitzip_top16_decode_attention(
     a.batch = count;
     a.q_heads = (unsigned int)q_heads;
     a.kv_heads = (unsigned int)kv_heads;
-    a.splits = plan.splits;
-    a.tokens_per_wave = plan.tokens_per_wave;
     a.scale_log2 = scale * 1.4426950408889634f;
     a.head_magic = (unsigned int)((1ull << 24) / kv_heads + 1);
     for (unsigned int r = 0; r < count; ++r) {
@@ -839,12 +940,21 @@ extern "C" long long kvq_splitzip_top16_decode_attention(
       a.ctx[r] = (unsigned int)ctx;
       a.span[r] = (unsigned int)((ctx + block_tokens - 1) / block_tokens * block_tokens);
     }
-    hipLaunchKernelGGL(top16_attention_split, dim3(plan.splits * plan.groups * count), dim3(kT),
+    unsigned long long longest = 0;
+    for (unsigned int r = 0; r < count; ++r)
+      longest = std::max(longest, context_tokens[first + r]);
+    const unsigned int splits = plan_splits(a, context_tokens + first, count, longest);
+    hipLaunchKernelGGL(top16_attention_split,
+                       dim3(a.first_split[count] * (unsigned int)head_groups(kv_heads)), dim3(kT),
                        0, stream, a);
     hipError_t st = hipGetLastError();
     if (st != hipSuccess) return fail("top16_attention_split", st);
-    hipLaunchKernelGGL(top16_attention_combine, dim3((unsigned int)q_heads, count),
-                       dim3(kHeadDim), 0, stream, a);
+    const dim3 grid((unsigned int)q_heads, count);
+    if (splits <= kCombineBatch)
+      hipLaunchKernelGGL(top16_attention_combine<1>, grid, dim3(kHeadDim), 0, stream, a);
+    else
+      hipLaunchKernelGGL(top16_attention_combine<kCombineParts>, grid,
+                         dim3(kHeadDim * kCombineParts), 0, stream, a);
     st = hipGetLastError();
     if (st != hipSuccess) return fail("top16_attention_combine", st);
   }
