@@ -432,13 +432,13 @@ __device__ __forceinline__ void attend_step(const RawShare& cur, unsigned int ts
 // and of 8 heads x 1 range in 8-wave workgroups (6 us); 4 waves per SIMD (at most
 // 128 VGPRs) ahead of 3 (6 us): the payload loads alone ran 134 against 152 us.
 constexpr int kWaves = 4;
-constexpr int kHeads = 2;
-constexpr int kRanges = kWaves / kHeads;
 constexpr int kT = 64 * kWaves;
-static_assert(kRanges * kHeads == kWaves, "whole ranges per head");
 
+template <int kHeads>
 __global__ __launch_bounds__(kT) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 top16_attention_split(AttnArgs a) {
+  constexpr int kRanges = kWaves / kHeads;
+  static_assert(kRanges * kHeads == kWaves, "whole ranges per head");
   __shared__ __align__(16) uint16_t lds[kWaves * kWaveLds];
   __shared__ uint32_t sTab[2][256];
   __shared__ unsigned int sBad[kWaves];
@@ -770,31 +770,48 @@ using namespace unchainkv;
 
 namespace {
 
-// Split-kernel workgroups the current device keeps resident at once (CUs x
-// workgroups per CU at the kernel's register and LDS use), cached per device.
-unsigned long long resident_workgroups() {
+// Compute units of the current device and the split-kernel workgroups each keeps
+// resident (at the kernel's register and LDS use; both variants take the same),
+// cached per device.
+struct Residency {
+  unsigned long long cus, per_cu;
+};
+
+Residency residency() {
   static std::mutex mu;
-  static unsigned long long cached[64] = {};
+  static Residency cached[64] = {};
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 512;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return Residency{256, 2};
   std::lock_guard<std::mutex> lock(mu);
-  if (cached[dev] == 0) {
+  if (cached[dev].cus == 0) {
     int cus = 0, per_cu = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
         cus <= 0)
       cus = 256;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &per_cu, reinterpret_cast<const void*>(top16_attention_split), kT, 0) != hipSuccess ||
+            &per_cu, reinterpret_cast<const void*>(top16_attention_split<2>), kT, 0) !=
+            hipSuccess ||
         per_cu <= 0)
       per_cu = 1;
-    cached[dev] = (unsigned long long)cus * (unsigned long long)per_cu;
+    cached[dev] = Residency{(unsigned long long)cus, (unsigned long long)per_cu};
   }
   return cached[dev];
 }
 
-// Workgroups per context split: every kv head, kHeads of them per workgroup.
-unsigned long long head_groups(unsigned long long kv_heads) {
-  return (kv_heads + kHeads - 1) / kHeads;
+// How a context split of a sequence is laid over workgroups of kWaves waves: `groups`
+// workgroups of `heads` kv heads and `ranges` token ranges each. Pairs of heads where
+// they come out even (above); with an odd count the last pair would leave two waves
+// of its workgroups idle, which costs more than reading code lines that two heads
+// share twice: 27 sequences of about 17000 tokens, 3 kv heads, 135 -> 117 us per call;
+// one sequence of 32768 tokens, 1 head, 21.6 -> 19.6 us.
+struct Shape {
+  unsigned long long groups;
+  unsigned int heads, ranges;
+};
+
+Shape group_shape(unsigned long long kv_heads) {
+  const unsigned int heads = kv_heads % 2 == 1 ? 1 : 2;
+  return Shape{(kv_heads + heads - 1) / heads, heads, kWaves / heads};
 }
 
 // Splits of all sequences of a launch together, at most: two rounds of the resident
@@ -803,60 +820,81 @@ unsigned long long head_groups(unsigned long long kv_heads) {
 // the smaller ones.
 unsigned long long max_launch_splits(unsigned long long sequences, unsigned long long kv_heads,
                                      unsigned long long max_ctx) {
-  const unsigned long long per_seq = (max_ctx + kRanges * kStep - 1) / (kRanges * kStep);
+  const Shape sh = group_shape(kv_heads);
+  const unsigned long long per_seq = (max_ctx + sh.ranges * kStep - 1) / (sh.ranges * kStep);
   return std::min(sequences * std::min<unsigned long long>(per_seq, kMaxSplits),
-                  2 * resident_workgroups() / head_groups(kv_heads) + sequences);
+                  2 * residency().cus * residency().per_cu / sh.groups + sequences);
 }
 
-// Splits of every sequence with at most `tpw` tokens per wave.
+// Splits of all sequences together with at most `per_split` tokens in each.
 unsigned long long count_splits(const unsigned long long* ctx, unsigned int count,
-                                unsigned int tpw) {
-  const unsigned int per_split = tpw * kRanges;
+                                unsigned int per_split) {
   unsigned long long splits = 0;
   for (unsigned int r = 0; r < count; ++r) splits += ((unsigned int)ctx[r] + per_split - 1) / per_split;
   return splits;
 }
 
+// Cost of one round of w workgroups per CU whose longest range has s steps, in
+// hundredths of a microsecond: kRoundCost + w * kGroupCost + s * kStepCost[w]. A step
+// of more workgroups takes longer (they share the CU's LDS and the memory), but less
+// than in proportion, and more workgroups pay more start-ups, so that few steps in
+// all are best spread thinly. Fitted to 32 sequences of 8192 tokens, 8 kv heads, at
+// 1, 2, 3 and 4 workgroups per CU: 254, 168, 152 and 146 us per call (128, 64, 43 and
+// 32 steps); one sequence of 32768 tokens: 40, 35, 37 and 41 us (16, 8, 6 and 4); 64
+// sequences of 128 to 32768 tokens, 1 kv head: 68, 45.5, 45 and 47 us.
+constexpr unsigned long long kStepCost[] = {0, 193, 248, 326, 410};
+constexpr unsigned long long kRoundCost = 400, kGroupCost = 350;
+
 // Fills the launch's splits (a.tpw, a.first_split, a.uniform_splits) from the
-// sequences' own context lengths: a split gives every head kRanges token ranges, and
-// a sequence takes as many splits as keep its ranges within the launch's tokens per
-// wave. That number is the smallest whose workgroups fit k rounds of the resident
-// slots, for the k with the least work in a row (a wave walks its range serially, a
-// round lasts as long as its longest range): k rounds of (tpw + kWaveOverhead)
-// token steps. Sized for the longest sequence instead, with equal splits per
-// sequence, a batch of mixed lengths left most of its workgroups empty: 64 sequences
-// of 128 to 32768 tokens, one kv head, 117 -> 43 us per call (185 MB of packed KV);
-// one 1500-token sequence of 8 kv heads, 18.4 -> 12.8 us (8 -> 47 splits); 32 equal
-// sequences of 8192 tokens take the same splits as before (144 us).
-unsigned int plan_splits(AttnArgs& a, const unsigned long long* ctx, unsigned int count,
-                         unsigned long long max_ctx) {
-  const unsigned long long groups = head_groups(a.kv_heads), slots = resident_workgroups();
+// sequences' own context lengths and returns the most of one sequence: a split gives
+// every head `ranges` token ranges, and a sequence takes as many splits as keep its
+// ranges within the launch's number of steps. That number is the smallest whose
+// workgroups fit a round of w workgroups per CU, or several rounds of as many as stay
+// resident, whichever costs least. Sized for the longest sequence instead, with equal
+// splits per sequence, a batch of mixed lengths left most of its workgroups empty: 64
+// sequences of 128 to 32768 tokens, one kv head, 117 -> 45 us per call (185 MB of
+// packed KV); one 1500-token sequence of 8 kv heads, 18.4 -> 12.8 us (8 -> 47 splits).
+unsigned int plan_splits(AttnArgs& a, const Shape& sh, const unsigned long long* ctx,
+                         unsigned int count, unsigned long long max_ctx) {
+  const Residency res = residency();
+  const unsigned long long groups = sh.groups;
   const unsigned long long limit = max_launch_splits(count, a.kv_heads, max_ctx);
-  constexpr unsigned long long kWaveOverhead = 32;  // start-up cost in token steps
+  const unsigned int round = sh.ranges * kStep;  // tokens of a split with one step per range
   unsigned long long total = 0;
   for (unsigned int r = 0; r < count; ++r) total += ctx[r];
-  const unsigned int most =
-      (unsigned int)((max_ctx + kRanges * kStep - 1) / (kRanges * kStep));  // steps: one split each
-  // at most kMaxSplits per sequence
-  const unsigned int least = (unsigned int)((max_ctx + (unsigned long long)kRanges * kStep * kMaxSplits - 1) /
-                                            ((unsigned long long)kRanges * kStep * kMaxSplits));
+  // steps per range: with one split per sequence, and with the most splits
+  const unsigned int most = (unsigned int)((max_ctx + round - 1) / round);
+  const unsigned int least = (most + kMaxSplits - 1) / kMaxSplits;
   unsigned int best = most;
   unsigned long long best_cost = ~0ull;
-  const unsigned long long k0 = (count * groups + slots - 1) / slots;
-  for (unsigned long long k = k0; k < k0 + 3; ++k) {
-    const unsigned long long fit = std::min(k * slots / groups, std::max<unsigned long long>(limit, count));
-    // smallest number of steps per range whose splits fit
-    unsigned int lo = least, hi = most;
-    const unsigned long long floor_steps = total / (fit * kRanges * kStep);
-    if (floor_steps > lo) lo = (unsigned int)std::min<unsigned long long>(floor_steps, most);
+  // k rounds of w workgroups per CU: w = 1, 2, ... for one round, then k = 2, 3
+  for (unsigned long long c = 1; c < res.per_cu + 3; ++c) {
+    const unsigned long long w = std::min(c, res.per_cu);
+    const unsigned long long k0 = std::max<unsigned long long>(
+        1, (count * groups + res.cus * w - 1) / (res.cus * w));
+    const unsigned long long k = k0 + (c - w);
+    if (w < res.per_cu && k > 1) continue;
+    const unsigned long long fit =
+        std::min(k * res.cus * w / groups, std::max<unsigned long long>(limit, count));
+    // smallest number of steps per range whose splits fit: between the even share of
+    // all tokens and that of all but one split per sequence
+    unsigned int lo = std::max<unsigned int>(
+        least, (unsigned int)std::min<unsigned long long>(total / (fit * round), most));
+    unsigned int hi = most;
+    if (fit > count) {
+      const unsigned long long even = total / ((fit - count) * round) + 1;
+      hi = std::max(lo, (unsigned int)std::min<unsigned long long>(even, most));
+    }
     while (lo < hi) {
       const unsigned int mid = lo + (hi - lo) / 2;
-      if (count_splits(ctx, count, mid * kStep) <= fit)
+      if (count_splits(ctx, count, mid * round) <= fit)
         hi = mid;
       else
         lo = mid + 1;
     }
-    const unsigned long long cost = k * ((unsigned long long)lo * kStep + kWaveOverhead);
+    const unsigned long long step_cost =
+        w < sizeof(kStepCost) / sizeof(kStepCost[0]) ? kStepCost[w] : kStepCost[4] * w / 4;
+    const unsigned long long cost = k * (kRoundCost + w * kGroupCost + lo * step_cost);
     if (cost < best_cost) {
       best_cost = cost;
       best = lo;
@@ -866,9 +904,10 @@ unsigned int plan_splits(AttnArgs& a, const unsigned long long* ctx, unsigned in
   unsigned int splits = 0, largest = 0, smallest = ~0u;
   for (unsigned int r = 0; r < count; ++r) {
     const unsigned int c = (unsigned int)ctx[r];
-    const unsigned int want = (c + best * kStep * kRanges - 1) / (best * kStep * kRanges);
-    a.tpw[r] = (c + want * kRanges * kStep - 1) / (want * kRanges * kStep) * kStep;
-    const unsigned int own = (c + a.tpw[r] * kRanges - 1) / (a.tpw[r] * kRanges);
+    const unsigned int want = (c + best * round - 1) / (best * round);
+    const unsigned int steps = (c + want * round - 1) / (want * round);
+    const unsigned int own = (c + steps * round - 1) / (steps * round);
+    a.tpw[r] = steps * kStep;
     a.first_split[r] = splits;
     splits += own;
     largest = std::max(largest, own);
@@ -943,10 +982,13 @@ extern "C" long long kvq_splitzip_top16_decode_attention(
     unsigned long long longest = 0;
     for (unsigned int r = 0; r < count; ++r)
       longest = std::max(longest, context_tokens[first + r]);
-    const unsigned int splits = plan_splits(a, context_tokens + first, count, longest);
-    hipLaunchKernelGGL(top16_attention_split,
-                       dim3(a.first_split[count] * (unsigned int)head_groups(kv_heads)), dim3(kT),
-                       0, stream, a);
+    const Shape sh = group_shape(kv_heads);
+    const unsigned int splits = plan_splits(a, sh, context_tokens + first, count, longest);
+    const dim3 split_grid(a.first_split[count] * (unsigned int)sh.groups);
+    if (sh.heads == 1)
+      hipLaunchKernelGGL(top16_attention_split<1>, split_grid, dim3(kT), 0, stream, a);
+    else
+      hipLaunchKernelGGL(top16_attention_split<2>, split_grid, dim3(kT), 0, stream, a);
     hipError_t st = hipGetLastError();
     if (st != hipSuccess) return fail("top16_attention_split", st);
     const dim3 grid((unsigned int)q_heads, count);
