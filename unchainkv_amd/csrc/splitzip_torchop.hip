@@ -28,8 +28,9 @@
 // launch, XCD-remapped, lanes own two 8-word runs so that every section access of
 // a wave instruction is one contiguous span), `*_generic` for any other geometry
 // (workgroup (x, y): words [4096 x, 4096 x + 4096) of payload y, 16 consecutive
-// words per thread, byte-granular section accesses). A launch covers at most 64
-// payloads; the plan kernel runs once for up to 256 after all presence launches.
+// words per thread, byte-granular section accesses). A launch of the tile kernels
+// covers up to 256 payloads (TileArgs), of the generic ones 64; the plan kernel runs
+// once for up to 256 after all presence launches.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -607,12 +608,65 @@ __device__ __forceinline__ void store_bytes(unsigned char* p, unsigned long long
   if (w & 1) p[at] = (unsigned char)(v >> (8 * at));
 }
 
+// One payload of a tile launch.
+struct TilePayload {
+  unsigned long long buf_offset;  // its first byte in `buf`
+  unsigned long long encoded;     // its encoded bytes
+  unsigned long long ids_offset;  // its first block id in `ids`
+  unsigned int block_count;       // blocks per plane
+  unsigned int tile_begin;        // its first tile within the launch
+};
+static_assert(sizeof(TilePayload) == 32, "one scalar load of eight dwords");
+
+// Arguments of a tile launch of up to kMax payloads. Requests below 1 MiB come by the
+// dozen, and every launch of them pays its own ramp and drain (4 to 5 us each): 136
+// requests of 15 Llama-3-8B blocks took 35.4 us (presence), 52.7 us (encode) and 59.3
+// us (decode) in launches of at most 64, and 27.4, 48.4 and 52.5 us in one (134 MB read;
+// 242 MB moved each way, 4.6 to 5.0 TB/s). The small struct serves calls of at most
+// 64 payloads: the arguments (9.5 KB of them for 256) are copied on each launch.
+template <unsigned int kMax>
+struct TileArgs {
+  uint16_t* kv;
+  const long long* ids;
+  unsigned char* buf;
+  unsigned int* records;  // presence: the launch's first tile record
+  const TorchopPlan* plans;  // encode: the launch's first plan
+  unsigned long long plane_stride;
+  unsigned long long block_stride;
+  EncodeGeom geo;
+  unsigned int total_tiles;
+  unsigned int uniform_tiles;  // tiles of every payload when all are equal, else 0
+  unsigned int begin[kMax];    // tile_begin of each payload, 0xFFFFFFFF past the last
+  TilePayload p[kMax];
+};
+constexpr unsigned int kTilePayloadsSmall = kWave;
+constexpr unsigned int kTilePayloads = 4 * kWave;
+
+// Payload of a (wave-uniform) tile: one division for equal payloads; otherwise lane l
+// holds the first tiles of payloads l * kMax / 64 .. and ballots count the payloads
+// that start at or before the tile. Every lane of the wave must be active.
+template <unsigned int kMax>
+__device__ __forceinline__ unsigned int tile_payload(const TileArgs<kMax>& a, unsigned int tile) {
+  constexpr unsigned int kPer = kMax / kWave;
+  static_assert(kPer * kWave == kMax, "whole payloads per lane");
+  if (a.uniform_tiles) return tile / a.uniform_tiles;
+  const unsigned int lane = __lane_id();
+  unsigned int begin[kPer];
+#pragma unroll
+  for (unsigned int k = 0; k < kPer; ++k) begin[k] = a.begin[lane * kPer + k];
+  unsigned int count = 0;
+#pragma unroll
+  for (unsigned int k = 0; k < kPer; ++k) count += (unsigned int)__popcll(__ballot(begin[k] <= tile));
+  return uniform(count - 1u);
+}
+
 // Element offset in the layer of the wave chunk starting at payload word c.
-__device__ __forceinline__ unsigned long long chunk_source(const LaunchArgs& a,
-                                                           const PayloadDesc& d,
-                                                           const EncodeGeom& geo,
+template <unsigned int kMax>
+__device__ __forceinline__ unsigned long long chunk_source(const TileArgs<kMax>& a,
+                                                           const TilePayload& d,
                                                            unsigned long long n,
                                                            unsigned long long c) {
+  const EncodeGeom& geo = a.geo;
   const unsigned long long half = n >> 1;
   const unsigned int plane = c >= half ? 1u : 0u;
   const unsigned int in_plane = uniform((unsigned int)(c - plane * half));
@@ -628,20 +682,21 @@ __device__ __forceinline__ unsigned int run_code(unsigned long long codes, unsig
   return (unsigned int)(codes >> (width * k)) & ((1u << width) - 1u);
 }
 
-__global__ __launch_bounds__(kThreads) void torchop_presence_tile(LaunchArgs a, EncodeGeom geo,
-                                                                  unsigned int record_base) {
+template <unsigned int kMax>
+__global__ __launch_bounds__(kThreads) void torchop_presence_tile(TileArgs<kMax> a) {
   __shared__ unsigned char s_high[256];
   __shared__ unsigned int s_nib;
   const unsigned int tid = threadIdx.x;
   const unsigned int lane = tid & (kWave - 1), wave = uniform(tid >> 6);
   const unsigned int tile = group_index();
-  const PayloadDesc d = a.p[find_payload(a, tile)];
-  const unsigned long long n = payload_words(a, d);
-  const unsigned long long c = (unsigned long long)(tile - d.tile_begin) * kTorchopTile + wave * 1024ull;
+  const TilePayload d = a.p[tile_payload(a, tile)];
+  const unsigned long long n = 2ull * d.block_count * a.geo.bw;
+  const unsigned long long c =
+      (unsigned long long)(tile - d.tile_begin) * kTorchopTile + wave * 1024ull;
   const bool active = c < n;
   u32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
   if (active) {
-    const uint16_t* src = a.kv + chunk_source(a, d, geo, n, c);
+    const uint16_t* src = a.kv + chunk_source(a, d, n, c);
     v0 = load_stream16(src + 8 * lane);
     v1 = load_stream16(src + 512 + 8 * lane);
   }
@@ -663,7 +718,7 @@ __global__ __launch_bounds__(kThreads) void torchop_presence_tile(LaunchArgs a, 
     if (lane == 0) atomicOr(&s_nib, nib);
   }
   __syncthreads();
-  unsigned int* rec = a.workspace + kTorchopRecordWords * (record_base + tile);
+  unsigned int* rec = a.records + (unsigned long long)kTorchopRecordWords * tile;
   const unsigned long long high = __ballot(s_high[tid] != 0);
   if (lane == 0) {
     rec[2 * wave] = (unsigned int)high;
@@ -672,28 +727,27 @@ __global__ __launch_bounds__(kThreads) void torchop_presence_tile(LaunchArgs a, 
   if (tid == 0) rec[8] = s_nib;
 }
 
-__global__ __launch_bounds__(kThreads) void torchop_encode_tile(LaunchArgs a, EncodeGeom geo,
-                                                                const TorchopPlan* plans,
-                                                                TorchopSizes sizes) {
+template <unsigned int kMax>
+__global__ __launch_bounds__(kThreads) void torchop_encode_tile(TileArgs<kMax> a) {
   __shared__ unsigned char s_rank[256];
   const unsigned int tid = threadIdx.x;
   const unsigned int lane = tid & (kWave - 1), wave = uniform(tid >> 6);
   const unsigned int tile = group_index();
-  const unsigned int r = find_payload(a, tile);
-  const PayloadDesc d = a.p[r];
-  const unsigned long long n = payload_words(a, d);
+  const unsigned int r = tile_payload(a, tile);
+  const TilePayload d = a.p[r];
+  const unsigned long long n = 2ull * d.block_count * a.geo.bw;
   const unsigned int local = tile - d.tile_begin;
   const unsigned long long c = (unsigned long long)local * kTorchopTile + wave * 1024ull;
   const bool active = c < n;
   // the words first: the plan's round trip overlaps with theirs
   u32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
   if (active) {
-    const uint16_t* src = a.kv + chunk_source(a, d, geo, n, c);
+    const uint16_t* src = a.kv + chunk_source(a, d, n, c);
     v0 = load_stream16(src + 8 * lane);
     v1 = load_stream16(src + 512 + 8 * lane);
   }
   unsigned char* out = a.buf + d.buf_offset;
-  const EncodeFields f = encode_prologue(plans + r, n, sizes.encoded[r], out, s_rank, local == 0);
+  const EncodeFields f = encode_prologue(a.plans + r, n, d.encoded, out, s_rank, local == 0);
   if (!f.ok) return;  // the whole workgroup
   __syncthreads();
   if (!active) return;
@@ -748,16 +802,15 @@ __global__ __launch_bounds__(kThreads) void torchop_encode_tile(LaunchArgs a, En
   }
 }
 
-__global__ __launch_bounds__(kThreads) void torchop_decode_tile(LaunchArgs a, EncodeGeom geo,
-                                                                TorchopSizes sizes) {
+template <unsigned int kMax>
+__global__ __launch_bounds__(kThreads) void torchop_decode_tile(TileArgs<kMax> a) {
   __shared__ unsigned char s_pal[256];
   const unsigned int tid = threadIdx.x;
   const unsigned int lane = tid & (kWave - 1), wave = uniform(tid >> 6);
   const unsigned int tile = group_index();
-  const unsigned int r = find_payload(a, tile);
-  const PayloadDesc d = a.p[r];
-  const unsigned long long n = 2ull * d.block_count * a.block_words;
-  const unsigned long long size = sizes.encoded[r];
+  const TilePayload d = a.p[tile_payload(a, tile)];
+  const unsigned long long n = 2ull * d.block_count * a.geo.bw;
+  const unsigned long long size = d.encoded;
   const unsigned char* payload = a.buf + d.buf_offset;
   const unsigned long long c =
       (unsigned long long)(tile - d.tile_begin) * kTorchopTile + wave * 1024ull;
@@ -773,7 +826,7 @@ __global__ __launch_bounds__(kThreads) void torchop_decode_tile(LaunchArgs a, En
   const unsigned long long first8 =
       sh ? (lo64 >> sh) | ((unsigned long long)hw[2] << (64 - sh)) : lo64;
   const bool active = c < n;
-  uint16_t* dst = active ? a.kv + chunk_source(a, d, geo, n, c) : nullptr;
+  uint16_t* dst = active ? a.kv + chunk_source(a, d, n, c) : nullptr;
   const TorchopHeader h = parse_header(first8, size, n);
   if (!h.ok) return;  // the whole workgroup
   // the palette bytes first, then every section load of both runs, so that the
@@ -856,6 +909,69 @@ bool torchop_tile_geometry(unsigned long long kv_ptr, unsigned long long plane_s
          block_stride % 8 == 0;
 }
 
+// Queues a tile kernel over payloads [0, payload_count), at most kMax per launch:
+// launch(a, first, before) with the arguments of the payloads from `first` on filled in
+// (`before` tiles lie in earlier launches); offsets and sizes may be null. The caller
+// has checked that every payload has at most 2^32 - 1 words, so that the tiles of a
+// launch fit 32 bits.
+template <unsigned int kMax, typename Launch>
+hipError_t each_tile_launch(unsigned long long kv_ptr, unsigned long long plane_stride,
+                      unsigned long long block_stride, unsigned long long block_words,
+                      unsigned long long block_ids_ptr, const unsigned long long* block_offsets,
+                      const unsigned long long* offsets, const unsigned long long* sizes,
+                      unsigned long long payload_count, Launch launch) {
+  TileArgs<kMax> a;  // (entries past the last payload are never read)
+  a.kv = reinterpret_cast<uint16_t*>(kv_ptr);
+  a.ids = reinterpret_cast<const long long*>(block_ids_ptr);
+  a.buf = nullptr;
+  a.records = nullptr;
+  a.plans = nullptr;
+  a.plane_stride = plane_stride;
+  a.block_stride = block_stride;
+  a.geo = make_geom(block_words);
+  unsigned long long before = 0;
+  for (unsigned long long first = 0; first < payload_count; first += kMax) {
+    const unsigned int count =
+        (unsigned int)std::min<unsigned long long>(kMax, payload_count - first);
+    unsigned int tiles = 0;
+    bool uniform_size = true;
+    for (unsigned int k = 0; k < count; ++k) {
+      const unsigned long long r = first + k;
+      TilePayload& d = a.p[k];
+      d.buf_offset = offsets ? offsets[r] : 0;
+      d.encoded = sizes ? sizes[r] : 0;
+      d.ids_offset = block_offsets[r];
+      d.block_count = (unsigned int)(block_offsets[r + 1] - block_offsets[r]);
+      d.tile_begin = a.begin[k] = tiles;
+      tiles += (unsigned int)torchop_tiles(2ull * d.block_count * block_words);
+      uniform_size = uniform_size && d.block_count == a.p[0].block_count;
+    }
+    for (unsigned int k = count; k < kMax; ++k) a.begin[k] = 0xFFFFFFFFu;
+    a.total_tiles = tiles;
+    a.uniform_tiles = uniform_size ? tiles / count : 0;
+    launch(a, first, before);
+    const hipError_t st = hipGetLastError();
+    if (st != hipSuccess) return st;
+    before += tiles;
+  }
+  return hipSuccess;
+}
+
+template <typename Launch>
+hipError_t tile_launches(unsigned long long kv_ptr, unsigned long long plane_stride,
+                         unsigned long long block_stride, unsigned long long block_words,
+                         unsigned long long block_ids_ptr, const unsigned long long* block_offsets,
+                         const unsigned long long* offsets, const unsigned long long* sizes,
+                         unsigned long long payload_count, Launch launch) {
+  if (payload_count <= kTilePayloadsSmall)
+    return each_tile_launch<kTilePayloadsSmall>(kv_ptr, plane_stride, block_stride, block_words,
+                                                block_ids_ptr, block_offsets, offsets, sizes,
+                                                payload_count, launch);
+  return each_tile_launch<kTilePayloads>(kv_ptr, plane_stride, block_stride, block_words,
+                                         block_ids_ptr, block_offsets, offsets, sizes,
+                                         payload_count, launch);
+}
+
 }  // namespace
 
 // Decodes payload r (src + src_offsets[r], encoded_bytes[r] long; byte 0 is its
@@ -872,17 +988,23 @@ extern "C" long long kvq_splitzip_bf16_decode_torchop_paged(
       encoded_bytes == nullptr || block_offsets == nullptr || payload_count == 0 ||
       block_words == 0 || block_words > 0xFFFFFFFFULL || kv_ptr % 2 != 0)
     return 0;
-  unsigned long long total = 0, max_n = 0;
+  unsigned long long total = 0;
   for (unsigned long long r = 0; r < payload_count; ++r) {
     if (block_offsets[r + 1] <= block_offsets[r] || encoded_bytes[r] == 0) return 0;
     const unsigned long long n = 2 * (block_offsets[r + 1] - block_offsets[r]) * block_words;
     if (n > 0xFFFFFFFFULL) return 0;
     total += 2 * n;
-    max_n = std::max(max_n, n);
   }
-  const bool tiles = torchop_tile_geometry(kv_ptr, plane_stride, block_stride, block_words);
-  const EncodeGeom geo = make_geom(block_words);
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
+  if (torchop_tile_geometry(kv_ptr, plane_stride, block_stride, block_words)) {
+    const hipError_t st = tile_launches(
+        kv_ptr, plane_stride, block_stride, block_words, block_ids_ptr, block_offsets, src_offsets,
+        encoded_bytes, payload_count, [&](auto& a, unsigned long long, unsigned long long) {
+          a.buf = reinterpret_cast<unsigned char*>(src_ptr);
+          torchop_decode_tile<<<dim3(a.total_tiles), dim3(kThreads), 0, stream>>>(a);
+        });
+    return st != hipSuccess ? fail("torchop_decode", st) : (long long)total;
+  }
   for (unsigned long long first = 0; first < payload_count; first += kMaxPayloads) {
     LaunchArgs a{};
     TorchopSizes sizes{};
@@ -894,29 +1016,18 @@ extern "C" long long kvq_splitzip_bf16_decode_torchop_paged(
     a.block_words = block_words;
     const unsigned int count =
         (unsigned int)std::min<unsigned long long>(kMaxPayloads, payload_count - first);
-    unsigned long long launch_max = 0, launch_tiles = 0;
-    bool uniform_size = true;
+    unsigned long long launch_max = 0;
     for (unsigned int k = 0; k < count; ++k) {
       const unsigned long long r = first + k;
       a.p[k].buf_offset = src_offsets[r];
       a.p[k].ids_offset = block_offsets[r];
       a.p[k].block_count = (unsigned int)(block_offsets[r + 1] - block_offsets[r]);
-      a.p[k].tile_begin = (unsigned int)launch_tiles;
       sizes.encoded[k] = encoded_bytes[r];
-      const unsigned long long n = 2ull * a.p[k].block_count * block_words;
-      launch_max = std::max(launch_max, n);
-      launch_tiles += torchop_tiles(n);
-      uniform_size = uniform_size && a.p[k].block_count == a.p[0].block_count;
+      launch_max = std::max(launch_max, 2ull * a.p[k].block_count * block_words);
     }
     a.payload_count = count;
-    const dim3 grid((unsigned int)((launch_max + kTorchopTile - 1) / kTorchopTile), count);
-    if (tiles && launch_tiles <= 0xFFFFFFFFULL) {
-      a.total_tiles = (unsigned int)launch_tiles;
-      a.uniform_tiles = uniform_size ? (unsigned int)(launch_tiles / count) : 0;
-      hipLaunchKernelGGL(torchop_decode_tile, dim3(a.total_tiles), dim3(kThreads), 0, stream, a,
-                         geo, sizes);
-    } else
-      hipLaunchKernelGGL(torchop_decode_generic, grid, dim3(kThreads), 0, stream, a, sizes);
+    const dim3 grid((unsigned int)torchop_tiles(launch_max), count);
+    hipLaunchKernelGGL(torchop_decode_generic, grid, dim3(kThreads), 0, stream, a, sizes);
     const hipError_t st = hipGetLastError();
     if (st != hipSuccess) return fail("torchop_decode", st);
   }
@@ -926,16 +1037,12 @@ extern "C" long long kvq_splitzip_bf16_decode_torchop_paged(
 namespace {
 
 
-// Fills the launch arguments of payloads [first, first + count): descriptors with
-// their first tile within the launch, the launch's tile count and, when every
-// payload has the same size, its tiles per payload. The launch's tile records
-// start at record tile_prefix. False when a word or tile count is past the
-// kernels' limits.
-bool torchop_args(LaunchArgs& a, unsigned long long kv_ptr, unsigned long long plane_stride,
+// Fills the arguments of a generic launch over payloads [first, first + count):
+// descriptors with their first tile within the launch, and the launch's tile count.
+void torchop_args(LaunchArgs& a, unsigned long long kv_ptr, unsigned long long plane_stride,
                   unsigned long long block_stride, unsigned long long block_words,
                   unsigned long long block_ids_ptr, const unsigned long long* block_offsets,
-                  unsigned long long first, unsigned int count, unsigned long long tile_prefix,
-                  unsigned long long& max_n) {
+                  unsigned long long first, unsigned int count, unsigned long long& max_n) {
   a = LaunchArgs{};
   a.kv = reinterpret_cast<uint16_t*>(kv_ptr);
   a.ids = reinterpret_cast<const long long*>(block_ids_ptr);
@@ -945,23 +1052,17 @@ bool torchop_args(LaunchArgs& a, unsigned long long kv_ptr, unsigned long long p
   a.payload_count = count;
   max_n = 0;
   unsigned long long tile = 0;  // tiles of the launch before payload k
-  bool uniform_size = true;
   for (unsigned int k = 0; k < count; ++k) {
     const unsigned long long r = first + k;
     const unsigned long long blocks = block_offsets[r + 1] - block_offsets[r];
     const unsigned long long n = 2 * blocks * block_words;
-    if (n > 0x7FFFFFFFULL || tile_prefix + tile > 0xFFFFFFFFULL) return false;
     a.p[k].ids_offset = block_offsets[r];
     a.p[k].block_count = (unsigned int)blocks;
     a.p[k].tile_begin = (unsigned int)tile;
     tile += torchop_tiles(n);
     max_n = std::max(max_n, n);
-    uniform_size = uniform_size && blocks == block_offsets[first + 1] - block_offsets[first];
   }
-  if (tile > 0xFFFFFFFFULL) return false;
   a.total_tiles = (unsigned int)tile;
-  a.uniform_tiles = uniform_size ? (unsigned int)(tile / count) : 0;
-  return true;
 }
 
 bool torchop_tables_ok(unsigned long long kv_ptr, unsigned long long block_words,
@@ -970,9 +1071,15 @@ bool torchop_tables_ok(unsigned long long kv_ptr, unsigned long long block_words
   if (kv_ptr == 0 || block_ids_ptr == 0 || block_offsets == nullptr || payload_count == 0 ||
       block_words == 0 || block_words > 0xFFFFFFFFULL || kv_ptr % 2 != 0)
     return false;
-  for (unsigned long long r = 0; r < payload_count; ++r)
+  unsigned long long tiles = 0;
+  for (unsigned long long r = 0; r < payload_count; ++r) {
     if (block_offsets[r + 1] <= block_offsets[r]) return false;
-  return true;
+    const unsigned long long n = 2 * (block_offsets[r + 1] - block_offsets[r]) * block_words;
+    // the encode kernels' limits: 31-bit word counts, 32-bit tile records of a call
+    if (n > 0x7FFFFFFFULL) return false;
+    tiles += torchop_tiles(n);
+  }
+  return tiles <= 0xFFFFFFFFULL;
 }
 
 }  // namespace
@@ -1006,26 +1113,28 @@ extern "C" long long kvq_splitzip_bf16_plan_torchop_paged(
   const unsigned long long need =
       kvq_splitzip_torchop_workspace_bytes(block_words, block_offsets, payload_count);
   if (need == 0 || workspace_bytes < need) return 0;
-  const bool tiles = torchop_tile_geometry(kv_ptr, plane_stride, block_stride, block_words);
-  const EncodeGeom geo = make_geom(block_words);
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
+  const bool tiles = torchop_tile_geometry(kv_ptr, plane_stride, block_stride, block_words);
+  if (tiles) {
+    const hipError_t st = tile_launches(
+        kv_ptr, plane_stride, block_stride, block_words, block_ids_ptr, block_offsets, nullptr,
+        nullptr, payload_count, [&](auto& a, unsigned long long, unsigned long long before) {
+          a.records = reinterpret_cast<unsigned int*>(workspace_ptr) + kTorchopRecordWords * before;
+          torchop_presence_tile<<<dim3(a.total_tiles), dim3(kThreads), 0, stream>>>(a);
+        });
+    if (st != hipSuccess) return fail("torchop_presence", st);
+  }
   unsigned long long tile_prefix = 0;
-  for (unsigned long long first = 0; first < payload_count; first += kMaxPayloads) {
+  for (unsigned long long first = 0; !tiles && first < payload_count; first += kMaxPayloads) {
     const unsigned int count =
         (unsigned int)std::min<unsigned long long>(kMaxPayloads, payload_count - first);
     LaunchArgs a;
     unsigned long long max_n = 0;
-    if (!torchop_args(a, kv_ptr, plane_stride, block_stride, block_words, block_ids_ptr,
-                      block_offsets, first, count, tile_prefix, max_n))
-      return 0;
+    torchop_args(a, kv_ptr, plane_stride, block_stride, block_words, block_ids_ptr, block_offsets,
+                 first, count, max_n);
     a.workspace = reinterpret_cast<unsigned int*>(workspace_ptr);
-    const unsigned int base = (unsigned int)tile_prefix;
-    if (tiles)
-      hipLaunchKernelGGL(torchop_presence_tile, dim3(a.total_tiles), dim3(kThreads), 0, stream, a,
-                         geo, base);
-    else
-      hipLaunchKernelGGL(torchop_presence_generic, dim3((unsigned int)torchop_tiles(max_n), count),
-                         dim3(kThreads), 0, stream, a, base);
+    hipLaunchKernelGGL(torchop_presence_generic, dim3((unsigned int)torchop_tiles(max_n), count),
+                       dim3(kThreads), 0, stream, a, (unsigned int)tile_prefix);
     const hipError_t st = hipGetLastError();
     if (st != hipSuccess) return fail("torchop_presence", st);
     tile_prefix += a.total_tiles;
@@ -1063,8 +1172,6 @@ extern "C" long long kvq_splitzip_bf16_encode_torchop_paged(
       plans_ptr == 0 || plans_ptr % 8 != 0 || out_ptr == 0 || out_offsets == nullptr ||
       encoded_bytes == nullptr)
     return 0;
-  const bool tiles = torchop_tile_geometry(kv_ptr, plane_stride, block_stride, block_words);
-  const EncodeGeom geo = make_geom(block_words);
   unsigned long long total = 0;
   for (unsigned long long r = 0; r < payload_count; ++r) {
     const unsigned long long n = 2 * (block_offsets[r + 1] - block_offsets[r]) * block_words;
@@ -1075,14 +1182,23 @@ extern "C" long long kvq_splitzip_bf16_encode_torchop_paged(
     total += size;
   }
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
+  if (torchop_tile_geometry(kv_ptr, plane_stride, block_stride, block_words)) {
+    const hipError_t st = tile_launches(
+        kv_ptr, plane_stride, block_stride, block_words, block_ids_ptr, block_offsets, out_offsets,
+        encoded_bytes, payload_count, [&](auto& a, unsigned long long first, unsigned long long) {
+          a.buf = reinterpret_cast<unsigned char*>(out_ptr);
+          a.plans = reinterpret_cast<const TorchopPlan*>(plans_ptr) + first;
+          torchop_encode_tile<<<dim3(a.total_tiles), dim3(kThreads), 0, stream>>>(a);
+        });
+    return st != hipSuccess ? fail("torchop_encode", st) : (long long)total;
+  }
   for (unsigned long long first = 0; first < payload_count; first += kMaxPayloads) {
     const unsigned int count =
         (unsigned int)std::min<unsigned long long>(kMaxPayloads, payload_count - first);
     LaunchArgs a;
     unsigned long long max_n = 0;
-    if (!torchop_args(a, kv_ptr, plane_stride, block_stride, block_words, block_ids_ptr,
-                      block_offsets, first, count, 0, max_n))
-      return 0;
+    torchop_args(a, kv_ptr, plane_stride, block_stride, block_words, block_ids_ptr, block_offsets,
+                 first, count, max_n);
     a.buf = reinterpret_cast<unsigned char*>(out_ptr);
     TorchopSizes sizes{};
     for (unsigned int k = 0; k < count; ++k) {
@@ -1091,11 +1207,7 @@ extern "C" long long kvq_splitzip_bf16_encode_torchop_paged(
     }
     const dim3 grid((unsigned int)torchop_tiles(max_n), count);
     const TorchopPlan* plans = reinterpret_cast<const TorchopPlan*>(plans_ptr) + first;
-    if (tiles)
-      hipLaunchKernelGGL(torchop_encode_tile, dim3(a.total_tiles), dim3(kThreads), 0, stream, a,
-                         geo, plans, sizes);
-    else
-      hipLaunchKernelGGL(torchop_encode_generic, grid, dim3(kThreads), 0, stream, a, plans, sizes);
+    hipLaunchKernelGGL(torchop_encode_generic, grid, dim3(kThreads), 0, stream, a, plans, sizes);
     const hipError_t st = hipGetLastError();
     if (st != hipSuccess) return fail("torchop_encode", st);
   }
