@@ -1,0 +1,184 @@
+"""Layers whose block words are a multiple of 8 but not of 1024 (the run geometry of the
+tile kernels): every codec's payloads byte for byte with the oracle's and the decode
+into other blocks word for word. Requests end on both sides of a 512-word run row, a
+1024-word wave and a 4096-word tile; exponents are natural, escape-dense (tiles past
+the staged escapes are scanned again) or overflow the Top-16 capacity. Blocks of the
+layer outside the requests stay untouched."""
+
+import numpy as np
+import pytest
+
+import oracle
+
+torch = pytest.importorskip("torch")
+pytestmark = pytest.mark.gpu
+
+BLOCK_WORDS = [8, 24, 520, 1016, 1032, 1280, 4104, 7680]
+
+
+@pytest.fixture(scope="module")
+def sz():
+    if not torch.cuda.is_available():
+        pytest.skip("no ROCm GPU visible")
+    from unchainkv_amd import splitzip_cuda
+
+    assert splitzip_cuda.available(), splitzip_cuda.load_error()
+    return splitzip_cuda
+
+
+def make(bw, kind, seed):
+    """(layer words, sender tables, receiver tables, codebook)."""
+    rng = np.random.default_rng(seed)
+    counts = [max(3, t // bw) for t in (500, 1024, 4096, 4608, 13000)]
+    pool = sum(counts) + 4
+    values = rng.standard_normal((2, pool, bw)).astype(np.float32)
+    words = (values.view(np.uint32) >> 16).astype(np.uint16)
+    if kind != "natural":
+        # 'dense': one request's words in one tile-long stretch all off the codebook
+        # (still within the payload's capacity only for the long requests)
+        flat = words.reshape(-1)
+        share = 0.003 if kind == "dense" else 0.05
+        hit = rng.random(flat.size) < share
+        flat[hit] = (rng.integers(0x60, 0x7F, hit.sum()) << 8).astype(np.uint16)
+
+    def tables():
+        ids, at, out = rng.permutation(pool).tolist(), 0, []
+        for c in counts:
+            out.append(ids[at:at + c])
+            at += c
+        return out
+
+    send, recv = tables(), tables()
+    if kind == "dense":
+        # 150 escapes in a row in the longest request: more than a tile stages, within
+        # its capacity where the request is long enough
+        words[0, send[-1][0], :min(bw, 150)] = 0x7F00
+    book = b""
+    for plane in range(2):
+        count = np.bincount((words[plane].reshape(-1) >> 7) & 0xFF, minlength=256)
+        count[0xC0:] = 0
+        book += bytes(sorted(range(256), key=lambda e: (-count[e], e))[:16])
+    return words, send, recv, book
+
+
+def to_gpu(words):
+    return torch.from_numpy(words.view(np.int16).copy()).cuda().view(torch.bfloat16)
+
+
+def check_restored(words, send, recv, target, payload_ok):
+    got = target.view(torch.int16).cpu().numpy().view(np.uint16)
+    for r, (t, u) in enumerate(zip(send, recv)):
+        want = words[:, t] if payload_ok[r] else np.zeros_like(words[:, t])
+        assert np.array_equal(got[:, u], want), r
+    rest = sorted(set(range(words.shape[1])) - {b for u in recv for b in u})
+    assert not got[:, rest].any()
+
+
+@pytest.mark.parametrize("kind", ["natural", "dense", "overflow"])
+@pytest.mark.parametrize("bw", BLOCK_WORDS)
+def test_top16(sz, bw, kind):
+    print("[case] runs top16", bw, kind, flush=True)
+    words, send, recv, book = make(bw, kind, bw)
+    layer = to_gpu(words)
+    batch = sz.PagedBatch(send, bw, "cuda")
+    assert batch.directory_bytes() == 0
+    out = batch.new_payload_buffer().fill_(0x5A)
+    assert sz.encode_top16_paged(layer, batch, out, batch.new_workspace(), codebooks=book) == \
+        batch.total_encoded_bytes
+    host = out.cpu().numpy()
+    tab = oracle.top16_tables(book)
+    ok = []
+    for r, t in enumerate(send):
+        a = batch.out_offsets[r]
+        want = oracle.top16_encode(words[:, t].reshape(-1), tab)
+        assert bytes(host[a:a + batch.encoded_bytes[r]]) == bytes(want), r
+        ok.append(want[0] == 5)
+    assert (host[:batch.out_offsets[0]] == 0x5A).all()
+    target = torch.zeros_like(layer)
+    assert sz.decode_top16_paged(out, batch.out_offsets, batch.encoded_bytes, target,
+                                 sz.PagedBatch(recv, bw, "cuda"), codebooks=book) == \
+        batch.total_raw_bytes
+    check_restored(words, send, recv, target, ok)
+    # the drop-in pair over the longest request, a workspace's room past the payload
+    words_r = np.ascontiguousarray(words[:, send[-1]])
+    size = batch.encoded_bytes[-1]
+    buf = torch.zeros(2 * words_r.size + (1 << 20), dtype=torch.uint8, device="cuda")
+    assert sz.encode_top16(to_gpu(words_r), buf, 0, codebooks=book) == size
+    want = oracle.top16_encode(words_r.reshape(-1), tab)
+    assert bytes(buf[:size].cpu().numpy()) == bytes(want)
+    target = torch.zeros_like(layer)
+    assert sz.decode_top16(buf[:size], target, recv[-1], 2 * words_r.size, 0, codebooks=book)
+    got = target.view(torch.int16).cpu().numpy().view(np.uint16)
+    assert np.array_equal(got[:, recv[-1]], words_r if want[0] == 5 else np.zeros_like(words_r))
+
+
+@pytest.mark.parametrize("bits", [6, 5])
+@pytest.mark.parametrize("bw", BLOCK_WORDS)
+def test_palette(sz, bw, bits):
+    print("[case] runs palette", bw, bits, flush=True)
+    words, send, recv, _ = make(bw, "natural", bw + bits)
+    # at most 31 high bytes, so that both palettes hold them; a request needs about
+    # 300 words to be smaller than its raw bytes
+    words = (((words >> 8) % 31 << 8) | (words & 0xFF)).astype(np.uint16)
+    keep = [r for r, t in enumerate(send) if 2 * len(t) * bw >= 512]
+    send, recv = [send[r] for r in keep], [recv[r] for r in keep]
+    layer = to_gpu(words)
+    batch = sz.PagedBatch(send, bw, "cuda")
+    offsets, sizes, _ = batch.palette_layout(bits)
+    out = batch.new_palette_buffer(bits).fill_(0x5A)
+    assert sz.encode_bf16_paged(layer, batch, out, batch.new_palette_workspace(), bits) == \
+        sum(sizes)
+    host = out.cpu().numpy()
+    for r, t in enumerate(send):
+        want = oracle.palette_encode(words[:, t].reshape(-1), bits)
+        assert bytes(host[offsets[r]:offsets[r] + sizes[r]]) == bytes(want), r
+    target = torch.zeros_like(layer)
+    assert sz.decode_bf16_paged(out, offsets, sizes, target, sz.PagedBatch(recv, bw, "cuda"),
+                                bits) == batch.total_raw_bytes
+    check_restored(words, send, recv, target, [True] * len(send))
+
+
+@pytest.mark.parametrize("formats", ["signmag", "mixed"])
+@pytest.mark.parametrize("bw", BLOCK_WORDS)
+def test_torchop(sz, bw, formats):
+    print("[case] runs torchop", bw, formats, flush=True)
+    words, send, recv, _ = make(bw, "natural", bw + 1)
+    if formats == "mixed":
+        rng = np.random.default_rng(bw)
+        # every third request's high bytes over the whole range (palette), another's
+        # with few low nibbles (nibble planes)
+        for r, t in enumerate(send):
+            if r % 3 == 1:
+                high = rng.choice(np.concatenate([[0, 0x7F], np.arange(0x80, 0x98)]),
+                                  (2, len(t), bw))
+                words[:, t] = ((high << 8) | (words[:, t] & 0xFF)).astype(np.uint16)
+            elif r % 3 == 2:
+                words[:, t] = (rng.integers(0, 256, (2, len(t), bw)) << 8 |
+                               rng.integers(0, 2, (2, len(t), bw))).astype(np.uint16)
+    layer = to_gpu(words)
+    batch = sz.PagedBatch(send, bw, "cuda")
+    plans = sz.plan_torchop_paged(layer, batch)
+    fields = sz.read_torchop_plans(plans.cpu().numpy())
+    sizes = [size for _, size in fields]
+    offsets = (np.cumsum([0] + [s + 3 for s in sizes])[:-1] + 1).tolist()  # odd starts
+    out = torch.full((sum(sizes) + 3 * len(sizes) + 8,), 0x5A, dtype=torch.uint8, device="cuda")
+    assert sz.encode_torchop_paged(layer, batch, plans, out, offsets, sizes) == sum(sizes)
+    host = out.cpu().numpy()
+    keep = []
+    for r, t in enumerate(send):
+        want = oracle.encode_torchop(words[:, t].reshape(-1))
+        if want is None:
+            assert fields[r] == (255, 0), r
+            continue
+        keep.append(r)
+        assert fields[r] == (int(want[0]), want.size), r
+        end = offsets[r] + sizes[r]
+        assert bytes(host[offsets[r]:end]) == want.tobytes(), r
+        assert (host[end:end + 3] == 0x5A).all()
+    assert keep
+    target = torch.zeros_like(layer)
+    assert sz.decode_torchop_paged(out, [offsets[r] for r in keep], [sizes[r] for r in keep],
+                                   target, sz.PagedBatch([recv[r] for r in keep], bw, "cuda")) \
+        == sum(batch.raw_bytes[r] for r in keep)
+    check_restored(words, [send[r] for r in keep], [recv[r] for r in keep], target,
+                   [True] * len(keep))

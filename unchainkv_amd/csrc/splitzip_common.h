@@ -299,7 +299,8 @@ struct PlaneTile {
   const long long* ids;   // the payload's block table (when there is one)
   unsigned int plane;
   unsigned int in_plane0;  // first word of the tile within its plane
-  unsigned int words;      // words in the tile: a multiple of 1024, at most the tile size
+  unsigned int words;      // words in the tile: a multiple of 1024 (run geometry: of 8),
+                           // at most the tile size
   unsigned int local_tile;
   unsigned int payload_tiles;
   unsigned int payload_index;  // index of the payload within the launch
@@ -366,6 +367,34 @@ __device__ __forceinline__ unsigned long long wave_source(const LaunchArgs& a, c
   return wave_offset_by(a, t, geo, in_plane, [&](unsigned int j) {
     return kIds ? (unsigned long long)t.ids[j] : a.block_start + j;
   });
+}
+
+// ---------------------------------------------------------------------------
+// run geometry: block words a multiple of 8 but not of 1024 (a head dim of 80 or 96,
+// three kv heads, blocks of 8 tokens). A wave's 1024 words then span several blocks, but
+// each 8-word run still lies in one, so a tile kernel keeps its lane layout (runs at
+// 8 * lane and 512 + 8 * lane of its wave's words, contiguous section accesses) and
+// each lane finds the block of its two runs itself: one multiply-high division and
+// one gathered id load per run, most of a wave's lanes in the same cache line. Tile
+// and plane ends fall anywhere on a multiple of 8 words, so runs, not waves, are
+// active or not.
+
+// The layout's share of the rule: whole 16-byte runs of the layer.
+inline bool run_geometry(unsigned long long kv_ptr, unsigned long long plane_stride,
+                         unsigned long long block_stride, unsigned long long block_words) {
+  return block_words % 8 == 0 && kv_ptr % 16 == 0 && plane_stride % 8 == 0 &&
+         block_stride % 8 == 0;
+}
+
+// Element offset in the layer of the run at in-plane word `in_plane` of tile t.
+template <bool kIds>
+__device__ __forceinline__ unsigned long long run_source(const LaunchArgs& a, const PlaneTile& t,
+                                                         const EncodeGeom& geo,
+                                                         unsigned int in_plane) {
+  const unsigned int j = div_u32(in_plane, geo.bw_magic, geo.bw);
+  const unsigned int within = in_plane - j * geo.bw;
+  const unsigned long long blk = kIds ? (unsigned long long)t.ids[j] : a.block_start + j;
+  return t.plane * a.plane_stride + blk * a.block_stride + within;
 }
 
 // A request's block table of at most kInlineBlocks ids carried in the kernel

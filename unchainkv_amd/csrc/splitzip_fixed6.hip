@@ -19,10 +19,11 @@
 //   palette_encode_tile / _generic     header + palette, low bytes, packed codes
 //   palette_decode_tile / _generic     decode + scatter (no-op unless byte 0 is the
 //       format's mode byte)
-// The tile kernels take block words a multiple of 1024 and a payload at any byte
-// address (global memory takes unaligned vector accesses): waves own 1024 words of
-// one block, lanes two 8-word runs, and the packed codes of a tile are staged in
-// LDS so they move as whole dwords.
+// The tile kernels take a payload at any byte address (global memory takes unaligned
+// vector accesses) and block words a multiple of 8: waves own 1024 words, of one block
+// where block words are a multiple of 1024 (chunk geometry), of several otherwise (run
+// geometry), lanes two 8-word runs, and the packed codes of a tile are staged in LDS
+// so they move as whole dwords.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -69,7 +70,8 @@ __device__ __forceinline__ void seen_clear(unsigned char* s_seen) {
   __syncthreads();
 }
 
-template <bool kIds>
+// kRuns (here and in the encode and decode tile kernels): the run geometry.
+template <bool kIds, bool kRuns>
 __global__ __launch_bounds__(kThreads) void palette_presence_tile(LaunchArgs a, EncodeGeom geo,
                                                                   unsigned int* masks) {
   __shared__ unsigned char s_seen[256];
@@ -78,12 +80,20 @@ __global__ __launch_bounds__(kThreads) void palette_presence_tile(LaunchArgs a, 
   const unsigned int tile = group_index();
   const PlaneTile t = plane_tile<kTileShift>(a, tile);
   const unsigned int in_plane = t.in_plane0 + wave * 1024;
-  const bool active = wave * 1024 < t.words;
+  const bool active = wave * 1024 + (kRuns ? 8 * lane : 0) < t.words;
+  const bool active_b = kRuns ? wave * 1024 + 512 + 8 * lane < t.words : active;
   u32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
   if (active) {
-    const uint16_t* src = a.kv + wave_source<kIds>(a, t, geo, in_plane);
-    v0 = load_stream16(src + 8 * lane);
-    v1 = load_stream16(src + 512 + 8 * lane);
+    if (kRuns) {
+      // (a lane without a second run reads its first one twice: the same mask)
+      v0 = load_stream16(a.kv + run_source<kIds>(a, t, geo, in_plane + 8 * lane));
+      v1 = load_stream16(a.kv + run_source<kIds>(a, t, geo, in_plane + (active_b ? 512 : 0) +
+                                                                8 * lane));
+    } else {
+      const uint16_t* src = a.kv + wave_source<kIds>(a, t, geo, in_plane);
+      v0 = load_stream16(src + 8 * lane);
+      v1 = load_stream16(src + 512 + 8 * lane);
+    }
   }
   seen_clear(s_seen);
   if (active) {
@@ -194,7 +204,7 @@ __device__ __forceinline__ unsigned long long unstage_run(const unsigned char* s
 
 // kIndexed: payload r's palette is info[a.p[r].mask_begin] (palettes computed by a
 // Top-16 probe encode for a larger batch), else info[r].
-template <bool kIds, int kBits, bool kIndexed = false>
+template <bool kIds, int kBits, bool kIndexed = false, bool kRuns = false>
 __global__ __launch_bounds__(kThreads) void palette_encode_tile(LaunchArgs a, EncodeGeom geo,
                                                                 const PaletteInfo* info) {
   using P = Palette<kBits>;
@@ -208,9 +218,17 @@ __global__ __launch_bounds__(kThreads) void palette_encode_tile(LaunchArgs a, En
   const PaletteInfo& pi = info[kIndexed ? a.p[t.payload_index].mask_begin : t.payload_index];
   const unsigned int in_plane = t.in_plane0 + wave * 1024;
   const unsigned long long wstart = t.plane * (t.n >> 1) + in_plane;  // payload word
-  const bool active = wave * 1024 < t.words;
+  const bool active = wave * 1024 + (kRuns ? 8 * lane : 0) < t.words;
+  const bool active_b = kRuns ? wave * 1024 + 512 + 8 * lane < t.words : active;
   uint32_t x[8];
-  if (active) {
+  if (kRuns) {
+    u32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
+    if (active) v0 = load_stream16(a.kv + run_source<kIds>(a, t, geo, in_plane + 8 * lane));
+    if (active_b)
+      v1 = load_stream16(a.kv + run_source<kIds>(a, t, geo, in_plane + 512 + 8 * lane));
+    x[0] = v0.x; x[1] = v0.y; x[2] = v0.z; x[3] = v0.w;
+    x[4] = v1.x; x[5] = v1.y; x[6] = v1.z; x[7] = v1.w;
+  } else if (active) {
     const uint16_t* src = a.kv + wave_source<kIds>(a, t, geo, in_plane);
     const u32x4 v0 = load_stream16(src + 8 * lane);
     const u32x4 v1 = load_stream16(src + 512 + 8 * lane);
@@ -228,21 +246,29 @@ __global__ __launch_bounds__(kThreads) void palette_encode_tile(LaunchArgs a, En
   __syncthreads();  // s_rank ready
   const unsigned char* rank = reinterpret_cast<const unsigned char*>(s_rank);
   unsigned char* stage = reinterpret_cast<unsigned char*>(s_code) + wave * kWaveCodeBytes;
+  unsigned char* low = t.payload + P::kHeader + wstart;
   if (active) {
-    unsigned char* low = t.payload + P::kHeader + wstart;
     store_stream8(low + 8 * lane, low_run(x));
-    store_stream8(low + 512 + 8 * lane, low_run(x + 4));
     stage_run<kBits>(stage, kBits * lane, pack_run<kBits>(x, rank));
+  }
+  if (active_b) {
+    store_stream8(low + 512 + 8 * lane, low_run(x + 4));
     stage_run<kBits>(stage, kBits * (64 + lane), pack_run<kBits>(x + 4, rank));
   }
   __syncthreads();
-  // the tile's code bytes as whole dwords (a tile's share is a multiple of 16
-  // bytes, so no dword reaches into a neighbour tile's share)
+  // the tile's code bytes as whole dwords, and in the run geometry, whose tiles may
+  // end on any run (kBits bytes), the last one to three as bytes: nothing reaches
+  // into a neighbour tile's share
   const unsigned long long tile_word = t.plane * (t.n >> 1) + t.in_plane0;
   uint32_t* codes = reinterpret_cast<uint32_t*>(t.payload + P::kHeader + t.n +
                                                 tile_word * kBits / 8);
   const unsigned int dwords = t.words * kBits / 32;
   for (unsigned int k = tid; k < dwords; k += kThreads) store_stream4(codes + k, s_code[k]);
+  if (kRuns) {
+    const unsigned int k = 4 * dwords + tid;
+    if (k < t.words * kBits / 8)
+      reinterpret_cast<unsigned char*>(codes)[k] = reinterpret_cast<unsigned char*>(s_code)[k];
+  }
 }
 
 // Any geometry: grid = payload_count x kGenericGroups, grid-stride over groups.
@@ -284,7 +310,7 @@ __global__ __launch_bounds__(kThreads) void palette_encode_generic(LaunchArgs a,
 // decode (DecodeFixed6 semantics, kvq_splitzip_cuda.cu:113-144)
 
 // Decode + scatter of one tile; the destination's j-th block from block_of(t, j).
-template <int kBits, typename BlockOf>
+template <int kBits, bool kRuns, typename BlockOf>
 __device__ __forceinline__ void palette_decode_tile_body(const LaunchArgs& a,
                                                          const EncodeGeom& geo,
                                                          BlockOf block_of) {
@@ -300,23 +326,42 @@ __device__ __forceinline__ void palette_decode_tile_body(const LaunchArgs& a,
   const unsigned int mode = t.payload[0];
   const unsigned int in_plane = t.in_plane0 + wave * 1024;
   const unsigned long long wstart = t.plane * (t.n >> 1) + in_plane;
-  const bool active = wave * 1024 < t.words;
+  const bool active = wave * 1024 + (kRuns ? 8 * lane : 0) < t.words;
+  const bool active_b = kRuns ? wave * 1024 + 512 + 8 * lane < t.words : active;
   const unsigned long long tile_word = t.plane * (t.n >> 1) + t.in_plane0;
   const uint32_t* codes = reinterpret_cast<const uint32_t*>(t.payload + P::kHeader + t.n +
                                                             tile_word * kBits / 8);
-  // the tile's code bytes, 16 at a time (a tile's share is a multiple of 16 bytes)
+  // the tile's code bytes, 16 at a time (a tile's share is a multiple of 16 bytes; in
+  // the run geometry of kBits bytes, the last up to 15 of them read singly)
   const unsigned int quads = t.words * kBits / 128;
   for (unsigned int k = tid; k < quads; k += kThreads)
     reinterpret_cast<u32x4*>(s_code)[k] = load_stream16(codes + 4 * k);
+  if (kRuns) {
+    const unsigned int k = 16 * quads + tid;
+    if (k < t.words * kBits / 8)
+      reinterpret_cast<unsigned char*>(s_code)[k] = reinterpret_cast<const unsigned char*>(codes)[k];
+  }
   if (tid < (unsigned int)P::kLimit) s_pal[tid] = t.payload[1 + tid];
   u32x2 low_a = {0, 0}, low_b = {0, 0};
-  uint16_t* dst = nullptr;
+  uint16_t* dst[2] = {nullptr, nullptr};  // of this lane's two runs
   if (active) {
     const unsigned char* low = t.payload + P::kHeader + wstart;
+    const unsigned int second = kRuns && !active_b ? 0u : 512u;  // (not stored then)
     low_a = load_stream8(low + 8 * lane);
-    low_b = load_stream8(low + 512 + 8 * lane);
-    dst = a.kv + wave_offset_by(a, t, geo, in_plane,
-                                [&](unsigned int j) { return block_of(t, j); });
+    low_b = load_stream8(low + second + 8 * lane);
+    if (kRuns) {
+#pragma unroll
+      for (int run = 0; run < 2; ++run) {
+        const unsigned int word = in_plane + (run ? second : 0u) + 8 * lane;
+        const unsigned int j = div_u32(word, geo.bw_magic, geo.bw);
+        dst[run] = a.kv + t.plane * a.plane_stride + block_of(t, j) * a.block_stride +
+                   (word - j * geo.bw);
+      }
+    } else {
+      dst[0] = a.kv + 8 * lane +
+               wave_offset_by(a, t, geo, in_plane, [&](unsigned int j) { return block_of(t, j); });
+      dst[1] = dst[0] + 512;
+    }
   }
   __syncthreads();
   if (mode != P::kMode || !active) return;  // the reference leaves other payloads untouched
@@ -334,13 +379,13 @@ __device__ __forceinline__ void palette_decode_tile_body(const LaunchArgs& a,
       const uint32_t h1 = s_pal[(bits >> (kBits * (2 * k + 1))) & kMask];
       out[k] = (lo & 0xFF) | (h0 << 8) | ((lo >> 8) << 16) | (h1 << 24);
     }
-    store_through16(dst + run * 512 + 8 * lane, u32x4{out[0], out[1], out[2], out[3]});
+    if (run == 0 || active_b) store_through16(dst[run], u32x4{out[0], out[1], out[2], out[3]});
   }
 }
 
-template <bool kIds, int kBits>
+template <bool kIds, int kBits, bool kRuns>
 __global__ __launch_bounds__(kThreads) void palette_decode_tile(LaunchArgs a, EncodeGeom geo) {
-  palette_decode_tile_body<kBits>(a, geo, [&](const PlaneTile& t, unsigned int j) {
+  palette_decode_tile_body<kBits, kRuns>(a, geo, [&](const PlaneTile& t, unsigned int j) {
     return kIds ? (unsigned long long)t.ids[j] : a.block_start + j;
   });
 }
@@ -350,7 +395,7 @@ template <int kBits>
 __global__ __launch_bounds__(kThreads) void palette_decode_tile_inline(LaunchArgs a,
                                                                        EncodeGeom geo,
                                                                        InlineBlocks table) {
-  palette_decode_tile_body<kBits>(a, geo, [&](const PlaneTile&, unsigned int j) {
+  palette_decode_tile_body<kBits, false>(a, geo, [&](const PlaneTile&, unsigned int j) {
     return (unsigned long long)table.id[j];
   });
 }
@@ -389,16 +434,18 @@ long long check(const char* what) {
   return st == hipSuccess ? 0 : fail(what, st);
 }
 
-inline bool tile_geometry(unsigned long long kv_ptr, unsigned long long plane_stride,
-                          unsigned long long block_stride, unsigned long long block_words,
-                          unsigned long long max_plane_words) {
-  return block_words % 1024 == 0 && kv_ptr % 16 == 0 && plane_stride % 8 == 0 &&
-         block_stride % 8 == 0 && max_plane_words < (1ull << 31);
-}
+// The kernels of a layout: tile kernels (chunk or run geometry; a payload's words are
+// then a multiple of 16, its sections at any byte address) or the generic ones.
+enum class Layout { kTile, kRuns, kGeneric };
 
-// A payload of n words suits the tile kernels at any byte address when its
-// sections are whole multiples of 16 bytes.
-inline bool palette_sections(unsigned long long n) { return n % 16 == 0; }
+inline Layout layout_of(unsigned long long kv_ptr, unsigned long long plane_stride,
+                        unsigned long long block_stride, unsigned long long block_words,
+                        unsigned long long max_plane_words) {
+  if (!run_geometry(kv_ptr, plane_stride, block_stride, block_words) ||
+      max_plane_words >= (1ull << 31))
+    return Layout::kGeneric;
+  return block_words % 1024 == 0 ? Layout::kTile : Layout::kRuns;
+}
 
 unsigned int tiles_of(unsigned long long n) {
   return 2u * (unsigned int)(((n >> 1) + kTileWords - 1) >> kTileShift);
@@ -407,19 +454,24 @@ unsigned int tiles_of(unsigned long long n) {
 // masks_given: `masks` already holds one mask per tile of every payload (from the
 // Top-16 encode), at each payload's mask_begin; the presence pass is skipped.
 template <int kBits>
-long long launch_palette_encode(LaunchArgs& a, const EncodeGeom& g, bool tiles,
+long long launch_palette_encode(LaunchArgs& a, const EncodeGeom& g, Layout layout,
                                 unsigned int presence_groups, PaletteInfo* info,
                                 unsigned int* masks, bool masks_given, hipStream_t stream) {
   const dim3 block(kThreads);
+  const bool tiles = layout != Layout::kGeneric;
+  const dim3 grid(a.total_tiles);
   if (masks_given) {
     presence_groups = 0;
+  } else if (layout == Layout::kRuns) {
+    if (a.ids)
+      palette_presence_tile<true, true><<<grid, block, 0, stream>>>(a, g, masks);
+    else
+      palette_presence_tile<false, true><<<grid, block, 0, stream>>>(a, g, masks);
   } else if (tiles) {
     if (a.ids)
-      hipLaunchKernelGGL(palette_presence_tile<true>, dim3(a.total_tiles), block, 0, stream, a, g,
-                         masks);
+      palette_presence_tile<true, false><<<grid, block, 0, stream>>>(a, g, masks);
     else
-      hipLaunchKernelGGL(palette_presence_tile<false>, dim3(a.total_tiles), block, 0, stream, a,
-                         g, masks);
+      palette_presence_tile<false, false><<<grid, block, 0, stream>>>(a, g, masks);
   } else {
     hipLaunchKernelGGL(palette_presence_generic, dim3(a.payload_count * presence_groups), block, 0,
                        stream, a, presence_groups, masks);
@@ -428,13 +480,16 @@ long long launch_palette_encode(LaunchArgs& a, const EncodeGeom& g, bool tiles,
   hipLaunchKernelGGL(palette_reduce<kBits>, dim3(a.payload_count), block, 0, stream, a,
                      tiles || masks_given ? 0u : presence_groups, masks, info);
   if (long long rc = check("palette_reduce")) return rc;
-  if (tiles) {
+  if (layout == Layout::kRuns) {
     if (a.ids)
-      hipLaunchKernelGGL((palette_encode_tile<true, kBits>), dim3(a.total_tiles), block, 0, stream,
-                         a, g, info);
+      palette_encode_tile<true, kBits, false, true><<<grid, block, 0, stream>>>(a, g, info);
     else
-      hipLaunchKernelGGL((palette_encode_tile<false, kBits>), dim3(a.total_tiles), block, 0,
-                         stream, a, g, info);
+      palette_encode_tile<false, kBits, false, true><<<grid, block, 0, stream>>>(a, g, info);
+  } else if (tiles) {
+    if (a.ids)
+      palette_encode_tile<true, kBits><<<grid, block, 0, stream>>>(a, g, info);
+    else
+      palette_encode_tile<false, kBits><<<grid, block, 0, stream>>>(a, g, info);
   } else {
     hipLaunchKernelGGL(palette_encode_generic<kBits>, dim3(a.payload_count * kGenericGroups),
                        block, 0, stream, a, info);
@@ -443,19 +498,21 @@ long long launch_palette_encode(LaunchArgs& a, const EncodeGeom& g, bool tiles,
 }
 
 template <int kBits>
-long long launch_palette_decode(LaunchArgs& a, const EncodeGeom& g, bool tiles,
+long long launch_palette_decode(LaunchArgs& a, const EncodeGeom& g, Layout layout,
                                 hipStream_t stream, const InlineBlocks* table) {
-  const dim3 block(kThreads);
-  if (tiles) {
-    if (table)
-      hipLaunchKernelGGL(palette_decode_tile_inline<kBits>, dim3(a.total_tiles), block, 0, stream,
-                         a, g, *table);
-    else if (a.ids)
-      hipLaunchKernelGGL((palette_decode_tile<true, kBits>), dim3(a.total_tiles), block, 0, stream,
-                         a, g);
+  const dim3 block(kThreads), grid(a.total_tiles);
+  if (layout == Layout::kRuns) {
+    if (a.ids)
+      palette_decode_tile<true, kBits, true><<<grid, block, 0, stream>>>(a, g);
     else
-      hipLaunchKernelGGL((palette_decode_tile<false, kBits>), dim3(a.total_tiles), block, 0,
-                         stream, a, g);
+      palette_decode_tile<false, kBits, true><<<grid, block, 0, stream>>>(a, g);
+  } else if (layout == Layout::kTile) {
+    if (table)
+      palette_decode_tile_inline<kBits><<<grid, block, 0, stream>>>(a, g, *table);
+    else if (a.ids)
+      palette_decode_tile<true, kBits, false><<<grid, block, 0, stream>>>(a, g);
+    else
+      palette_decode_tile<false, kBits, false><<<grid, block, 0, stream>>>(a, g);
   } else {
     hipLaunchKernelGGL(palette_decode_generic<kBits>, dim3(a.payload_count * kGenericGroups),
                        block, 0, stream, a);
@@ -479,20 +536,20 @@ long long launch_palette_encode_info(LaunchArgs& a, const EncodeGeom& g, const P
   return check("palette_encode (probe palettes)");
 }
 
-long long palette_encode(LaunchArgs& a, const EncodeGeom& g, bool tiles,
+long long palette_encode(LaunchArgs& a, const EncodeGeom& g, Layout layout,
                          unsigned int presence_groups, PaletteInfo* info, unsigned int* masks,
                          hipStream_t stream, int bits, bool masks_given = false) {
-  return bits == 6 ? launch_palette_encode<6>(a, g, tiles, presence_groups, info, masks,
+  return bits == 6 ? launch_palette_encode<6>(a, g, layout, presence_groups, info, masks,
                                               masks_given, stream)
-                   : launch_palette_encode<5>(a, g, tiles, presence_groups, info, masks,
+                   : launch_palette_encode<5>(a, g, layout, presence_groups, info, masks,
                                               masks_given, stream);
 }
 
 // `table`: one request's block table in the kernel arguments (tile kernels only).
-long long palette_decode(LaunchArgs& a, const EncodeGeom& g, bool tiles, hipStream_t stream,
+long long palette_decode(LaunchArgs& a, const EncodeGeom& g, Layout layout, hipStream_t stream,
                          int bits, const InlineBlocks* table = nullptr) {
-  return bits == 6 ? launch_palette_decode<6>(a, g, tiles, stream, table)
-                   : launch_palette_decode<5>(a, g, tiles, stream, table);
+  return bits == 6 ? launch_palette_decode<6>(a, g, layout, stream, table)
+                   : launch_palette_decode<5>(a, g, layout, stream, table);
 }
 
 // Fills a.p for payloads [first, first + count) of a batch (tiles of 4096 words
@@ -575,10 +632,10 @@ extern "C" long long kvq_splitzip_bf16_encode_mode(unsigned long long src_ptr,
   a.tile_shift = kTileShift;
   const unsigned long long ws = (dst_ptr + encoded + 15) / 16 * 16;  // 16-byte aligned scratch
   const unsigned long long room = dst_ptr + capacity > ws ? dst_ptr + capacity - ws : 0;
-  const bool tiles = count % 2 == 0 &&
-                     tile_geometry(src_ptr, count / 2, 0, count / 2, count / 2) &&
-                     palette_sections(count) &&
-                     room >= sizeof(PaletteInfo) + 32ull * tiles_of(count);
+  Layout layout = count % 2 == 0 ? layout_of(src_ptr, count / 2, 0, count / 2, count / 2)
+                                 : Layout::kGeneric;
+  if (room < sizeof(PaletteInfo) + 32ull * tiles_of(count)) layout = Layout::kGeneric;
+  const bool tiles = layout != Layout::kGeneric;
   a.total_tiles = tiles ? tiles_of(count) : 0;
   // Generic path: one presence mask per workgroup of the presence pass, as many as
   // the room holds (the reference's minimum capacity leaves room for 15).
@@ -587,7 +644,7 @@ extern "C" long long kvq_splitzip_bf16_encode_mode(unsigned long long src_ptr,
   if (!tiles && presence_groups == 0) return fail_msg("encode_mode: no room for the palette state");
   PaletteInfo* info = reinterpret_cast<PaletteInfo*>(ws);
   unsigned int* masks = reinterpret_cast<unsigned int*>(info + 1);
-  const long long rc = palette_encode(a, make_geom(count / 2), tiles, presence_groups, info, masks,
+  const long long rc = palette_encode(a, make_geom(count / 2), layout, presence_groups, info, masks,
                                       reinterpret_cast<hipStream_t>(stream_ptr), bits);
   return rc < 0 ? rc : (long long)encoded;
 }
@@ -628,20 +685,19 @@ long long decode_blocks(unsigned long long src_ptr, unsigned long long encoded_b
   a.p[0].block_count = (unsigned int)block_count;
   a.tiles_per_plane_mode = 1;
   a.tile_shift = kTileShift;
-  const bool tiles = tile_geometry(dst_ptr, plane_stride, block_stride, block_words,
-                                   count_words / 2) &&
-                     palette_sections(count_words);
+  const Layout layout =
+      layout_of(dst_ptr, plane_stride, block_stride, block_words, count_words / 2);
   a.total_tiles = tiles_of(count_words);
-  // a host block table rides in the kernel arguments (tile kernels only)
+  // a host block table rides in the kernel arguments (chunk geometry only)
   InlineBlocks table{};
   if (host_ids) {
-    if (!tiles || block_count > kInlineBlocks) return 0;
+    if (layout != Layout::kTile || block_count > kInlineBlocks) return 0;
     for (unsigned long long j = 0; j < block_count; ++j) {
       if (host_ids[j] < 0 || host_ids[j] > 0xFFFFFFFFll) return 0;
       table.id[j] = (unsigned int)host_ids[j];
     }
   }
-  const long long rc = palette_decode(a, make_geom(block_words), tiles,
+  const long long rc = palette_decode(a, make_geom(block_words), layout,
                                       reinterpret_cast<hipStream_t>(stream_ptr), bits,
                                       host_ids ? &table : nullptr);
   return rc < 0 ? rc : (long long)(count_words * sizeof(uint16_t));
@@ -718,7 +774,6 @@ long long encode_mode_paged_impl(
     for (unsigned long long r = 0; r < payload_count; ++r)
       if (info_first[r] >= info_count) return 0;
   unsigned long long total = 0, max_plane = 0;
-  bool sections = true;
   std::vector<std::pair<unsigned long long, unsigned long long>> spans;
   for (unsigned long long r = 0; r < payload_count; ++r) {
     if (block_offsets[r + 1] <= block_offsets[r]) return 0;
@@ -728,7 +783,6 @@ long long encode_mode_paged_impl(
     spans.emplace_back(out_offsets[r], out_offsets[r] + e);
     total += e;
     max_plane = std::max(max_plane, n >> 1);
-    sections = sections && palette_sections(n);
   }
   std::sort(spans.begin(), spans.end());
   for (size_t k = 1; k < spans.size(); ++k)
@@ -736,9 +790,8 @@ long long encode_mode_paged_impl(
   if (!with_info && batch_workspace_bytes(block_offsets, payload_count, block_words) >
                         workspace_bytes)
     return 0;
-  const bool tiles =
-      sections && tile_geometry(kv_ptr, plane_stride, block_stride, block_words, max_plane);
-  if (with_info && !tiles) return 0;  // the probe palettes come with the tile geometry
+  const Layout layout = layout_of(kv_ptr, plane_stride, block_stride, block_words, max_plane);
+  if (with_info && layout != Layout::kTile) return 0;  // the probe palettes come with the tile geometry
   const EncodeGeom g = make_geom(block_words);
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
   unsigned char* ws = reinterpret_cast<unsigned char*>(workspace_ptr);
@@ -768,7 +821,7 @@ long long encode_mode_paged_impl(
       for (unsigned int k = 0; k < count; ++k) a.p[k].mask_begin = (unsigned int)presence_first[first + k];
     }
     const long long rc =
-        palette_encode(a, g, tiles, kGenericGroups, info, masks, stream, bits, presence_ptr != 0);
+        palette_encode(a, g, layout, kGenericGroups, info, masks, stream, bits, presence_ptr != 0);
     if (rc < 0) return rc;
     ws += count * sizeof(PaletteInfo) +
           32 * std::max<unsigned long long>(a.total_tiles, (unsigned long long)count * kGenericGroups);
@@ -831,17 +884,14 @@ extern "C" long long kvq_splitzip_bf16_decode_mode_paged(
       block_words == 0 || block_words > 0xFFFFFFFFULL || (bits != 5 && bits != 6))
     return 0;
   unsigned long long total = 0, max_plane = 0;
-  bool sections = true;
   for (unsigned long long r = 0; r < payload_count; ++r) {
     if (block_offsets[r + 1] <= block_offsets[r]) return 0;
     const unsigned long long n = 2 * (block_offsets[r + 1] - block_offsets[r]) * block_words;
     if (encoded_bytes[r] != palette_encoded_size(n, bits) || (n >> 1) > 0xFFFFFFFFULL) return 0;
     total += 2 * n;
     max_plane = std::max(max_plane, n >> 1);
-    sections = sections && palette_sections(n);
   }
-  const bool tiles =
-      sections && tile_geometry(kv_ptr, plane_stride, block_stride, block_words, max_plane);
+  const Layout layout = layout_of(kv_ptr, plane_stride, block_stride, block_words, max_plane);
   const EncodeGeom g = make_geom(block_words);
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
   for (unsigned long long first = 0; first < payload_count; first += kMaxPayloads) {
@@ -855,7 +905,7 @@ extern "C" long long kvq_splitzip_bf16_decode_mode_paged(
     const unsigned int count =
         (unsigned int)std::min<unsigned long long>(kMaxPayloads, payload_count - first);
     fill_batch(a, block_offsets, src_offsets, first, count, block_words);
-    const long long rc = palette_decode(a, g, tiles, stream, bits);
+    const long long rc = palette_decode(a, g, layout, stream, bits);
     if (rc < 0) return rc;
   }
   return (long long)total;

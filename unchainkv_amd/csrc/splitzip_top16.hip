@@ -18,15 +18,20 @@
 //   top16_encode_tile        block words a multiple of 1024, payload at any byte
 //       address: gather through the block table + encode one 4096-word tile per
 //       workgroup, one block per wave so addressing is scalar; escapes are
-//       counted per tile and up to kStageSlots of them staged in the workspace.
+//       counted per tile and up to kStageSlots of them staged in the workspace. The
+//       same kernel takes any block words that are a multiple of 8 (run geometry),
+//       with per-lane addresses.
 //   top16_encode_lanes<fast, sequential>  any geometry: 16 consecutive words per
 //       lane (stores realigned through neighbour-lane shuffles); or one workgroup
-//       walking every tile in order.
+//       walking every tile in order. For what the tile kernels do not take: a layer
+//       off 16-byte alignment, other block words, drop-in encodes without room for a
+//       workspace.
 //   top16_encode_finalize    per payload (8, 16 or 32 workgroups): scan tile counts,
 //       place escapes in ascending order, write the header (the tile kernel
 //       zeroes the escape slots of its span).
-//   top16_decode_tile / top16_decode_lanes / top16_decode_generic
-//       decode + scatter for the tile geometry, 16-word lanes, any geometry.
+//   top16_decode_tile / top16_decode_runs / top16_decode_lanes / top16_decode_generic
+//       decode + scatter for the tile geometry, the run geometry, 16-word lanes (code
+//       tables or planes past the tile kernels' limits), any geometry.
 // Global memory takes unaligned vector accesses (the code object's unaligned
 // access mode), so a payload's sections need no alignment: the reference
 // connector's payloads start at a buffer's first byte, their body at byte 5.
@@ -632,9 +637,11 @@ __device__ __forceinline__ void zero_escape_span(unsigned char* payload, unsigne
 // and its first kInBodySlots escapes are staged in the tile's first 512 body
 // bytes (run A of wave 0, left unwritten here); top16_body_tile writes those
 // body bytes once the finalize has read the staging.
-template <bool kIds, bool kSeen, bool kInBody>
+// kRuns: the run geometry; without presence masks, in-body staging and a directory.
+template <bool kIds, bool kSeen, bool kInBody, bool kRuns = false>
 __global__ __launch_bounds__(kThreads) void top16_encode_tile(LaunchArgs a, EncodeGeom geo) {
   static_assert(!(kSeen && kInBody), "presence masks come with a workspace");
+  static_assert(!(kRuns && (kSeen || kInBody)), "presence and in-body staging: chunk geometry");
   __shared__ uint32_t s_tab[64];  // this tile's plane, 4 code bytes per dword
   __shared__ unsigned int s_wave[kThreads / kWave];
   __shared__ uint32_t s_seen[kSeen ? 64 : 1];  // one byte per high byte value
@@ -646,9 +653,18 @@ __global__ __launch_bounds__(kThreads) void top16_encode_tile(LaunchArgs a, Enco
   const unsigned int in_plane = t.in_plane0 + wave * 1024;
   const unsigned long long wstart = t.plane * (t.n >> 1) + in_plane;  // payload word
   const bool active = wave * 1024 < t.words;  // whole waves
+  const bool active_a = kRuns ? wave * 1024 + 8 * lane < t.words : active;
+  const bool active_b = kRuns ? wave * 1024 + 512 + 8 * lane < t.words : active;
   // source loads first, then the code table, so the table's round trip overlaps them
   uint32_t x[8];
-  if (active) {
+  if (kRuns) {
+    u32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
+    if (active_a) v0 = load_stream16(a.kv + run_source<kIds>(a, t, geo, in_plane + 8 * lane));
+    if (active_b)
+      v1 = load_stream16(a.kv + run_source<kIds>(a, t, geo, in_plane + 512 + 8 * lane));
+    x[0] = v0.x; x[1] = v0.y; x[2] = v0.z; x[3] = v0.w;
+    x[4] = v1.x; x[5] = v1.y; x[6] = v1.z; x[7] = v1.w;
+  } else if (active) {
     const uint16_t* src = a.kv + wave_source<kIds>(a, t, geo, in_plane);
     const u32x4 v0 = load_stream16(src + 8 * lane);
     const u32x4 v1 = load_stream16(src + 512 + 8 * lane);
@@ -680,13 +696,17 @@ __global__ __launch_bounds__(kThreads) void top16_encode_tile(LaunchArgs a, Enco
   if (active) {
     unsigned char* pbody = t.payload + 5 + wstart;
     unsigned char* pcode = t.payload + 5 + t.n + (wstart >> 1);
-    if (!kInBody || wave != 0) store_through8(pbody + 8 * lane, u32x2{body_a[0], body_a[1]});
-    store_through8(pbody + 512 + 8 * lane, u32x2{body_b[0], body_b[1]});
-    store_through4(pcode + 4 * lane, code_a);
-    store_through4(pcode + 256 + 4 * lane, code_b);
-  } else {
-    mask_a = mask_b = 0;
+    if (active_a) {
+      if (!kInBody || wave != 0) store_through8(pbody + 8 * lane, u32x2{body_a[0], body_a[1]});
+      store_through4(pcode + 4 * lane, code_a);
+    }
+    if (active_b) {
+      store_through8(pbody + 512 + 8 * lane, u32x2{body_b[0], body_b[1]});
+      store_through4(pcode + 256 + 4 * lane, code_b);
+    }
   }
+  if (!active_a) mask_a = 0;
+  if (!active_b) mask_b = 0;
 
   // escapes (rare), in ascending word order: run A of every lane of the wave,
   // then run B of every lane, then the next wave. Per-lane counts of both runs are
@@ -839,6 +859,41 @@ __global__ __launch_bounds__(kThreads) void top16_decode_tile_inline(LaunchArgs 
   decode_tile(a, geo, [&](const PlaneTile&, unsigned int j) {
     return (unsigned long long)table.id[j];
   });
+}
+
+// The same over the run geometry, with a destination per lane and run. A 65.6 MB layer
+// of 12 requests with 7680-word blocks (6 heads of 80): the 16-word lanes of the
+// lanes kernels store and load 32-byte strides and realign their sections by
+// shuffles; encode + decode call 68.8 us with those, 61.4 us with runs.
+template <bool kIds>
+__global__ __launch_bounds__(kThreads) void top16_decode_runs(LaunchArgs a, EncodeGeom geo) {
+  const unsigned int lane = threadIdx.x & (kWave - 1);
+  const unsigned int wave = uniform(threadIdx.x >> 6);
+  const PlaneTile t = plane_tile<kTileShift>(a, group_index());
+  const unsigned int in_plane = t.in_plane0 + wave * 1024;
+  const unsigned long long wstart = t.plane * (t.n >> 1) + in_plane;  // payload word
+  const unsigned int at_a = wave * 1024 + 8 * lane, at_b = at_a + 512;
+  if (at_a >= t.words) return;  // no barrier in this kernel
+  const bool active_b = at_b < t.words;
+  const unsigned int mode = t.payload[0];
+  const uint32_t* cbw = reinterpret_cast<const uint32_t*>(a.tables + 512 + t.plane * 16);
+  const uint32_t cb[4] = {cbw[0], cbw[1], cbw[2], cbw[3]};
+  const unsigned char* pbody = t.payload + 5 + wstart;
+  const unsigned char* pcode = t.payload + 5 + t.n + (wstart >> 1);
+  // a lane without a second run reads its first one twice (no branch on the loads)
+  const unsigned int second = active_b ? 512u : 0u;
+  const u32x2 body_a = load_stream8(pbody + 8 * lane);
+  const u32x2 body_b = load_stream8(pbody + second + 8 * lane);
+  const uint32_t code_a = load_stream4(pcode + 4 * lane);
+  const uint32_t code_b = load_stream4(pcode + second / 2 + 4 * lane);
+  uint16_t* dst_a = a.kv + run_source<kIds>(a, t, geo, in_plane + 8 * lane);
+  uint16_t* dst_b = a.kv + run_source<kIds>(a, t, geo, in_plane + second + 8 * lane);
+  const u32x4 out_a = decode_run8(body_a, code_a, cb);
+  const u32x4 out_b = decode_run8(body_b, code_b, cb);
+  asm volatile("" ::"v"(out_a), "v"(out_b), "v"(dst_a), "v"(dst_b));
+  if (mode != 5) return;
+  store_through16(dst_a, out_a);
+  if (active_b) store_through16(dst_b, out_b);
 }
 
 // Replaces the exponent of word w (0..1023) of this wave's chunk, held in run A
@@ -1304,7 +1359,7 @@ constexpr unsigned int kMinTileShift = kTileShift;
 // The tile kernels use 32-bit in-plane word arithmetic.
 constexpr unsigned long long kTilePlaneLimit = 1ull << 31;
 
-enum class Kernel { kTile, kLanes, kGeneric };
+enum class Kernel { kTile, kRuns, kLanes, kGeneric };
 
 struct Plan {
   Kernel kernel;
@@ -1321,23 +1376,27 @@ inline unsigned int host_payload_tiles(unsigned long long n, bool per_plane,
 }
 
 // tile_ok: every wave's 1024 words lie in one block (block words a multiple of
-// 1024) and the code table is dword aligned.
-Plan make_plan(bool geometry_fast, bool tile_ok, bool sequential) {
+// 1024) and the code table is dword aligned. runs_ok: the run geometry, with such a
+// table. The tile kernels where both hold: a wave's address is then scalar.
+Plan make_plan(bool geometry_fast, bool tile_ok, bool runs_ok, bool sequential) {
   Plan p;
   p.sequential = sequential;
   p.tile_shift = kTileShift;
+  p.per_plane = geometry_fast;
   if (geometry_fast && tile_ok && !sequential) {
     p.kernel = Kernel::kTile;
+  } else if (runs_ok && !sequential) {
+    p.kernel = Kernel::kRuns;
+    p.per_plane = true;
   } else {
     p.kernel = geometry_fast ? Kernel::kLanes : Kernel::kGeneric;
   }
-  p.per_plane = geometry_fast;
   return p;
 }
 
 // Decode tiles every payload per plane.
-Plan make_decode_plan(bool geometry_fast, bool tile_ok) {
-  Plan p = make_plan(geometry_fast, tile_ok, false);
+Plan make_decode_plan(bool geometry_fast, bool tile_ok, bool runs_ok) {
+  Plan p = make_plan(geometry_fast, tile_ok, runs_ok, false);
   p.per_plane = true;
   return p;
 }
@@ -1386,6 +1445,14 @@ long long launch_encode(LaunchArgs& a, const EncodeGeom& g, const Plan& p, hipSt
         hipLaunchKernelGGL((top16_encode_tile<false, false, false>), dim3(a.total_tiles), block,
                            0, stream, a, g);
       }
+      break;
+    case Kernel::kRuns:
+      if (a.ids)
+        hipLaunchKernelGGL((top16_encode_tile<true, false, false, true>), dim3(a.total_tiles),
+                           block, 0, stream, a, g);
+      else
+        hipLaunchKernelGGL((top16_encode_tile<false, false, false, true>), dim3(a.total_tiles),
+                           block, 0, stream, a, g);
       break;
     case Kernel::kLanes:
       hipLaunchKernelGGL((top16_encode_lanes<true, false>), dim3(a.total_tiles), block, 0, stream,
@@ -1481,6 +1548,12 @@ long long launch_decode(LaunchArgs& a, const EncodeGeom& g, const Plan& p, hipSt
       else
         hipLaunchKernelGGL(top16_decode_tile<false>, dim3(a.total_tiles), block, 0, stream, a, g);
       break;
+    case Kernel::kRuns:
+      if (a.ids)
+        hipLaunchKernelGGL(top16_decode_runs<true>, dim3(a.total_tiles), block, 0, stream, a, g);
+      else
+        hipLaunchKernelGGL(top16_decode_runs<false>, dim3(a.total_tiles), block, 0, stream, a, g);
+      break;
     case Kernel::kLanes:
       hipLaunchKernelGGL(top16_decode_lanes, dim3(a.total_tiles), block, 0, stream, a, g);
       break;
@@ -1565,20 +1638,28 @@ extern "C" long long kvq_splitzip_bf16_encode_top16(unsigned long long src_ptr,
   // the source (the first 512 of each tile after the tile kernel, the whole body
   // after the lanes kernels, whose tiles need 64 words for the staging); otherwise
   // one workgroup walks the tiles in order.
-  Plan plan = make_plan(geometry_fast, tile_ok, false);
+  // (halves of whole 16-word lanes too, so that a buffer with room for the lanes
+  // kernels' workspace has room for the same number of tiles)
+  const bool runs_ok = geometry_fast && tables_ptr % 4 == 0 &&
+                       run_geometry(src_ptr, count / 2, 0, count / 2);
+  Plan plan = make_plan(geometry_fast, tile_ok, runs_ok, false);
   unsigned int tiles = host_payload_tiles(count, plan.per_plane, plan.tile_shift);
   const unsigned long long ws_offset = align_up(dst_ptr + encoded, 16) - dst_ptr;
   const unsigned long long ws_bytes = workspace_words(tiles) * 4;
   if (tiles > 1 && ws_offset + ws_bytes <= capacity) {
     a.workspace = reinterpret_cast<unsigned int*>(dst_ptr + ws_offset);
   } else {
+    if (plan.kernel == Kernel::kRuns) {  // its tiles need a workspace
+      plan = make_plan(geometry_fast, tile_ok, false, false);
+      tiles = host_payload_tiles(count, plan.per_plane, plan.tile_shift);
+    }
     const unsigned long long tile_words = 1ull << plan.tile_shift;
     const unsigned long long span = plan.per_plane ? count / 2 : count;
     const unsigned long long last = span % tile_words ? span % tile_words : tile_words;
     if (tiles > 1 && std::min(last, span) >= 64) {
       a.inbody_slots = kInBodySlots;  // 512 bytes: count + 127 escapes
     } else {
-      plan = make_plan(geometry_fast, tile_ok, true);
+      plan = make_plan(geometry_fast, tile_ok, false, true);
       tiles = host_payload_tiles(count, plan.per_plane, plan.tile_shift);
     }
   }
@@ -1623,8 +1704,10 @@ long long decode_top16_one(unsigned long long src_ptr, unsigned long long encode
   a.p[0].block_count = (unsigned int)block_count;
   const bool geometry_fast = block_words % 16 == 0 && dst_ptr % 16 == 0 && plane_stride % 8 == 0 &&
                              block_stride % 8 == 0 && (count_words >> 1) <= 0xFFFFFFFFULL;
-  const Plan plan = make_decode_plan(geometry_fast, tables_ptr % 4 == 0 && block_words % 1024 == 0 &&
-                                                        (count_words >> 1) < kTilePlaneLimit);
+  const bool small = tables_ptr % 4 == 0 && (count_words >> 1) < kTilePlaneLimit;
+  const Plan plan =
+      make_decode_plan(geometry_fast, small && block_words % 1024 == 0,
+                       small && run_geometry(dst_ptr, plane_stride, block_stride, block_words));
   apply_plan(a, plan);
   a.total_tiles = host_payload_tiles(count_words, true, plan.tile_shift);
   InlineBlocks table{};
@@ -1811,8 +1894,9 @@ long long encode_top16_paged_impl(
   if (workspace_ptr % 4 != 0) return 0;
 
   const PagedGeometry pg{kv_ptr, plane_stride, block_stride, block_words, block_ids_ptr};
-  const Plan plan =
-      make_plan(paged_fast(pg), tables_ptr % 4 == 0 && block_words % 1024 == 0, false);
+  const Plan plan = make_plan(
+      paged_fast(pg), tables_ptr % 4 == 0 && block_words % 1024 == 0,
+      tables_ptr % 4 == 0 && run_geometry(kv_ptr, plane_stride, block_stride, block_words), false);
   const unsigned long long dir_tiles =
       kvq_splitzip_top16_paged_directory_bytes(block_words, block_offsets, payload_count) /
       kDirBytesPerTile;
@@ -2012,9 +2096,10 @@ extern "C" long long kvq_splitzip_bf16_decode_top16_paged(
     max_plane = std::max(max_plane, n >> 1);
   }
   const PagedGeometry pg{kv_ptr, plane_stride, block_stride, block_words, block_ids_ptr};
-  const Plan plan = make_decode_plan(
-      paged_fast(pg),
-      tables_ptr % 4 == 0 && block_words % 1024 == 0 && max_plane < kTilePlaneLimit);
+  const bool small = tables_ptr % 4 == 0 && max_plane < kTilePlaneLimit;
+  const Plan plan =
+      make_decode_plan(paged_fast(pg), small && block_words % 1024 == 0,
+                       small && run_geometry(kv_ptr, plane_stride, block_stride, block_words));
   const unsigned long long dir_tiles =
       kvq_splitzip_top16_paged_directory_bytes(block_words, block_offsets, payload_count) /
       kDirBytesPerTile;

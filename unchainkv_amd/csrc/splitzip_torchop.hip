@@ -23,10 +23,10 @@
 // codes LSB-first with zero padding bits). The host reads the plans' sizes between
 // the plan and the encode to lay the payloads out.
 //
-// Kernels: `*_tile` for layers whose block words are a multiple of 1024 (a
-// 1024-word wave chunk lies in one block; one workgroup per 4096-word tile of the
-// launch, XCD-remapped, lanes own two 8-word runs so that every section access of
-// a wave instruction is one contiguous span), `*_generic` for any other geometry
+// Kernels: `*_tile` for layers whose block words are a multiple of 8 (one workgroup
+// per 4096-word tile of the launch, XCD-remapped, lanes own two 8-word runs so that
+// every section access of a wave instruction is one contiguous span), `*_generic` for
+// any other geometry
 // (workgroup (x, y): words [4096 x, 4096 x + 4096) of payload y, 16 consecutive
 // words per thread, byte-granular section accesses). A launch of the tile kernels
 // covers up to 256 payloads (TileArgs), of the generic ones 64; the plan kernel runs
@@ -35,6 +35,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "splitzip_common.h"
 
@@ -566,10 +567,11 @@ __global__ __launch_bounds__(kThreads) void torchop_encode_generic(LaunchArgs a,
 }
 
 // ---------------------------------------------------------------------------
-// tile kernels: block words a multiple of 1024 (a 1024-word wave chunk lies in one
-// block), the layer 16-byte aligned. Workgroup (x, y): words [4096 x, 4096 x +
-// 4096) of payload y; wave w owns the chunk at 4096 x + 1024 w (its block found
-// with scalar loads), lane l the two 8-word runs at 8 l and 512 + 8 l of it. Every
+// tile kernels: block words a multiple of 8, the layer 16-byte aligned. One workgroup
+// per 4096-word tile of a payload; wave w owns the chunk at word 1024 w of it, lane l
+// the two 8-word runs at 8 l and 512 + 8 l of that. Where block words are a multiple
+// of 1024 a chunk lies in one block, found with scalar loads; otherwise (run geometry,
+// kRuns) each lane finds the blocks, and planes, of its runs. Every
 // section access of a wave instruction is then one contiguous span: the run's 16
 // source bytes, its 8 low bytes, its sign byte and its w code bytes (w-bit codes of
 // 8 words fill whole bytes) at the section offset of word i, w * i / 8. Payload
@@ -639,6 +641,8 @@ struct TileArgs {
   unsigned int begin[kMax];    // tile_begin of each payload, 0xFFFFFFFF past the last
   TilePayload p[kMax];
 };
+template <typename Args>
+constexpr unsigned int kPayloads = sizeof(std::decay_t<Args>::p) / sizeof(TilePayload);
 constexpr unsigned int kTilePayloadsSmall = kWave;
 constexpr unsigned int kTilePayloads = 4 * kWave;
 
@@ -660,7 +664,8 @@ __device__ __forceinline__ unsigned int tile_payload(const TileArgs<kMax>& a, un
   return uniform(count - 1u);
 }
 
-// Element offset in the layer of the wave chunk starting at payload word c.
+// Element offset in the layer of payload word c, the first of a wave chunk (uniform)
+// or of a lane's 8-word run.
 template <unsigned int kMax>
 __device__ __forceinline__ unsigned long long chunk_source(const TileArgs<kMax>& a,
                                                            const TilePayload& d,
@@ -676,13 +681,65 @@ __device__ __forceinline__ unsigned long long chunk_source(const TileArgs<kMax>&
   return uniform64(plane * a.plane_stride + blk * a.block_stride + within);
 }
 
+template <unsigned int kMax>
+__device__ __forceinline__ unsigned long long run_source(const TileArgs<kMax>& a,
+                                                         const TilePayload& d,
+                                                         unsigned long long n,
+                                                         unsigned long long i) {
+  const EncodeGeom& geo = a.geo;
+  const unsigned long long half = n >> 1;
+  const unsigned int plane = i >= half ? 1u : 0u;
+  const unsigned int in_plane = (unsigned int)(i - plane * half);
+  const unsigned int j = div_u32(in_plane, geo.bw_magic, geo.bw);
+  const unsigned int within = in_plane - j * geo.bw;
+  const unsigned long long blk = (unsigned long long)a.ids[d.ids_offset + j];
+  return plane * a.plane_stride + blk * a.block_stride + within;
+}
+
+// A lane's two runs of the wave chunk at payload word c, in words from c: 8 * lane and
+// 512 + 8 * lane. In the run geometry a payload may end on any run, and a lane without
+// a second run takes its first one for it (loads need no branch; nothing is stored
+// twice, see each kernel).
+struct LaneRuns {
+  unsigned int at[2];
+  bool active;    // the first run lies in the payload
+  bool active_b;  // the second one does
+};
+
+template <bool kRuns>
+__device__ __forceinline__ LaneRuns lane_runs(unsigned int lane, unsigned long long n,
+                                              unsigned long long c) {
+  LaneRuns r;
+  r.at[0] = 8 * lane;
+  r.at[1] = 512 + 8 * lane;
+  r.active = kRuns ? c + r.at[0] < n : c < n;
+  r.active_b = kRuns ? c + r.at[1] < n : r.active;
+  if (kRuns && !r.active_b) r.at[1] = r.at[0];
+  return r;
+}
+
+// The words of a lane's two active runs.
+template <bool kRuns, unsigned int kMax>
+__device__ __forceinline__ void load_runs(const TileArgs<kMax>& a, const TilePayload& d,
+                                          unsigned long long n, unsigned long long c,
+                                          const LaneRuns& r, u32x4& v0, u32x4& v1) {
+  if (kRuns) {
+    v0 = load_stream16(a.kv + run_source(a, d, n, c + r.at[0]));
+    v1 = load_stream16(a.kv + run_source(a, d, n, c + r.at[1]));
+  } else {
+    const uint16_t* src = a.kv + chunk_source(a, d, n, c);
+    v0 = load_stream16(src + r.at[0]);
+    v1 = load_stream16(src + r.at[1]);
+  }
+}
+
 // Codes k = 0..7 of a run, `width` bits each, LSB-first.
 __device__ __forceinline__ unsigned int run_code(unsigned long long codes, unsigned int width,
                                                  int k) {
   return (unsigned int)(codes >> (width * k)) & ((1u << width) - 1u);
 }
 
-template <unsigned int kMax>
+template <unsigned int kMax, bool kRuns>
 __global__ __launch_bounds__(kThreads) void torchop_presence_tile(TileArgs<kMax> a) {
   __shared__ unsigned char s_high[256];
   __shared__ unsigned int s_nib;
@@ -693,19 +750,16 @@ __global__ __launch_bounds__(kThreads) void torchop_presence_tile(TileArgs<kMax>
   const unsigned long long n = 2ull * d.block_count * a.geo.bw;
   const unsigned long long c =
       (unsigned long long)(tile - d.tile_begin) * kTorchopTile + wave * 1024ull;
-  const bool active = c < n;
+  const LaneRuns runs = lane_runs<kRuns>(lane, n, c);
+  const bool active = runs.active;
   u32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
-  if (active) {
-    const uint16_t* src = a.kv + chunk_source(a, d, n, c);
-    v0 = load_stream16(src + 8 * lane);
-    v1 = load_stream16(src + 512 + 8 * lane);
-  }
+  if (active) load_runs<kRuns>(a, d, n, c, runs, v0, v1);
   if (tid < 64) reinterpret_cast<unsigned int*>(s_high)[tid] = 0;
   if (tid == 0) s_nib = 0;
   __syncthreads();
+  unsigned int nib = 0;
   if (active) {
     const uint32_t x[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-    unsigned int nib = 0;
 #pragma unroll
     for (int k = 0; k < 8; ++k) {
       s_high[(x[k] >> 8) & 0xFF] = 1;
@@ -713,10 +767,10 @@ __global__ __launch_bounds__(kThreads) void torchop_presence_tile(TileArgs<kMax>
       nib |= (1u << (x[k] & 15)) | (1u << (16 + ((x[k] >> 4) & 15)));
       nib |= (1u << ((x[k] >> 16) & 15)) | (1u << (16 + ((x[k] >> 20) & 15)));
     }
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) nib |= __shfl_xor(nib, off, kWave);
-    if (lane == 0) atomicOr(&s_nib, nib);
   }
+#pragma unroll
+  for (int off = kWave / 2; off > 0; off >>= 1) nib |= __shfl_xor(nib, off, kWave);
+  if (lane == 0 && nib) atomicOr(&s_nib, nib);
   __syncthreads();
   unsigned int* rec = a.records + (unsigned long long)kTorchopRecordWords * tile;
   const unsigned long long high = __ballot(s_high[tid] != 0);
@@ -727,7 +781,7 @@ __global__ __launch_bounds__(kThreads) void torchop_presence_tile(TileArgs<kMax>
   if (tid == 0) rec[8] = s_nib;
 }
 
-template <unsigned int kMax>
+template <unsigned int kMax, bool kRuns>
 __global__ __launch_bounds__(kThreads) void torchop_encode_tile(TileArgs<kMax> a) {
   __shared__ unsigned char s_rank[256];
   const unsigned int tid = threadIdx.x;
@@ -738,14 +792,11 @@ __global__ __launch_bounds__(kThreads) void torchop_encode_tile(TileArgs<kMax> a
   const unsigned long long n = 2ull * d.block_count * a.geo.bw;
   const unsigned int local = tile - d.tile_begin;
   const unsigned long long c = (unsigned long long)local * kTorchopTile + wave * 1024ull;
-  const bool active = c < n;
+  const LaneRuns runs = lane_runs<kRuns>(lane, n, c);
+  const bool active = runs.active;
   // the words first: the plan's round trip overlaps with theirs
   u32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
-  if (active) {
-    const uint16_t* src = a.kv + chunk_source(a, d, n, c);
-    v0 = load_stream16(src + 8 * lane);
-    v1 = load_stream16(src + 512 + 8 * lane);
-  }
+  if (active) load_runs<kRuns>(a, d, n, c, runs, v0, v1);
   unsigned char* out = a.buf + d.buf_offset;
   const EncodeFields f = encode_prologue(a.plans + r, n, d.encoded, out, s_rank, local == 0);
   if (!f.ok) return;  // the whole workgroup
@@ -754,8 +805,9 @@ __global__ __launch_bounds__(kThreads) void torchop_encode_tile(TileArgs<kMax> a
   const uint32_t x[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
 #pragma unroll
   for (int run = 0; run < 2; ++run) {
+    if (kRuns && run && !runs.active_b) break;
     const uint32_t* xr = x + 4 * run;
-    const unsigned long long i = c + 512 * run + 8 * lane;  // the run's first word
+    const unsigned long long i = c + runs.at[run];  // the run's first word
     if (f.mode == 1) {
       unsigned long long at = 69;
 #pragma unroll
@@ -802,7 +854,7 @@ __global__ __launch_bounds__(kThreads) void torchop_encode_tile(TileArgs<kMax> a
   }
 }
 
-template <unsigned int kMax>
+template <unsigned int kMax, bool kRuns>
 __global__ __launch_bounds__(kThreads) void torchop_decode_tile(TileArgs<kMax> a) {
   __shared__ unsigned char s_pal[256];
   const unsigned int tid = threadIdx.x;
@@ -814,7 +866,7 @@ __global__ __launch_bounds__(kThreads) void torchop_decode_tile(TileArgs<kMax> a
   const unsigned char* payload = a.buf + d.buf_offset;
   const unsigned long long c =
       (unsigned long long)(tile - d.tile_begin) * kTorchopTile + wave * 1024ull;
-  // a payload of these kernels holds at least 2048 words; a shorter size fails its
+  // a payload of these kernels holds at least 16 words; a shorter size fails its
   // header check below, and the header reads stay inside 16 bytes of the payload
   if (size < 16) return;
   // header bytes 0-7 from the aligned dwords that cover them (scalar loads, in
@@ -825,8 +877,19 @@ __global__ __launch_bounds__(kThreads) void torchop_decode_tile(TileArgs<kMax> a
   const unsigned long long lo64 = hw[0] | ((unsigned long long)hw[1] << 32);
   const unsigned long long first8 =
       sh ? (lo64 >> sh) | ((unsigned long long)hw[2] << (64 - sh)) : lo64;
-  const bool active = c < n;
-  uint16_t* dst = active ? a.kv + chunk_source(a, d, n, c) : nullptr;
+  const LaneRuns runs = lane_runs<kRuns>(lane, n, c);
+  const bool active = runs.active;
+  uint16_t* dst[2] = {nullptr, nullptr};  // of this lane's two runs
+  if (active) {
+    if (kRuns) {
+#pragma unroll
+      for (int run = 0; run < 2; ++run) dst[run] = a.kv + run_source(a, d, n, c + runs.at[run]);
+    } else {
+      uint16_t* chunk = a.kv + chunk_source(a, d, n, c);
+#pragma unroll
+      for (int run = 0; run < 2; ++run) dst[run] = chunk + runs.at[run];
+    }
+  }
   const TorchopHeader h = parse_header(first8, size, n);
   if (!h.ok) return;  // the whole workgroup
   // the palette bytes first, then every section load of both runs, so that the
@@ -840,7 +903,7 @@ __global__ __launch_bounds__(kThreads) void torchop_decode_tile(TileArgs<kMax> a
   if (active) {
 #pragma unroll
     for (int run = 0; run < 2; ++run) {
-      const unsigned long long i = c + 512 * run + 8 * lane;
+      const unsigned long long i = c + runs.at[run];
       if (h.mode == 1) {
 #pragma unroll
         for (int q = 0; q < 4; ++q)
@@ -885,9 +948,9 @@ __global__ __launch_bounds__(kThreads) void torchop_decode_tile(TileArgs<kMax> a
     o[run].w = (word[6] & 0xFFFFu) | (word[7] << 16);
   }
   // write-through stores after the last load (the compiler's waits do not see them)
-  asm volatile("" ::"v"(o[0]), "v"(o[1]));
-  store_through16(dst + 8 * lane, o[0]);
-  store_through16(dst + 512 + 8 * lane, o[1]);
+  asm volatile("" ::"v"(o[0]), "v"(o[1]), "v"(dst[0]), "v"(dst[1]));
+  store_through16(dst[0], o[0]);
+  if (!kRuns || runs.active_b) store_through16(dst[1], o[1]);
 }
 
 }  // namespace
@@ -901,13 +964,6 @@ unsigned long long torchop_tiles(unsigned long long n) {
   return (n + kTorchopTile - 1) / kTorchopTile;
 }
 
-// The tile kernels' geometry: 1024-word wave chunks inside one block, 16-byte
-// aligned runs of the layer.
-bool torchop_tile_geometry(unsigned long long kv_ptr, unsigned long long plane_stride,
-                           unsigned long long block_stride, unsigned long long block_words) {
-  return block_words % 1024 == 0 && kv_ptr % 16 == 0 && plane_stride % 8 == 0 &&
-         block_stride % 8 == 0;
-}
 
 // Queues a tile kernel over payloads [0, payload_count), at most kMax per launch:
 // launch(a, first, before) with the arguments of the payloads from `first` on filled in
@@ -996,12 +1052,15 @@ extern "C" long long kvq_splitzip_bf16_decode_torchop_paged(
     total += 2 * n;
   }
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
-  if (torchop_tile_geometry(kv_ptr, plane_stride, block_stride, block_words)) {
+  if (run_geometry(kv_ptr, plane_stride, block_stride, block_words)) {
     const hipError_t st = tile_launches(
         kv_ptr, plane_stride, block_stride, block_words, block_ids_ptr, block_offsets, src_offsets,
         encoded_bytes, payload_count, [&](auto& a, unsigned long long, unsigned long long) {
           a.buf = reinterpret_cast<unsigned char*>(src_ptr);
-          torchop_decode_tile<<<dim3(a.total_tiles), dim3(kThreads), 0, stream>>>(a);
+          if (block_words % 1024 == 0)
+            torchop_decode_tile<kPayloads<decltype(a)>, false><<<dim3(a.total_tiles), dim3(kThreads), 0, stream>>>(a);
+          else
+            torchop_decode_tile<kPayloads<decltype(a)>, true><<<dim3(a.total_tiles), dim3(kThreads), 0, stream>>>(a);
         });
     return st != hipSuccess ? fail("torchop_decode", st) : (long long)total;
   }
@@ -1114,13 +1173,16 @@ extern "C" long long kvq_splitzip_bf16_plan_torchop_paged(
       kvq_splitzip_torchop_workspace_bytes(block_words, block_offsets, payload_count);
   if (need == 0 || workspace_bytes < need) return 0;
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
-  const bool tiles = torchop_tile_geometry(kv_ptr, plane_stride, block_stride, block_words);
+  const bool tiles = run_geometry(kv_ptr, plane_stride, block_stride, block_words);
   if (tiles) {
     const hipError_t st = tile_launches(
         kv_ptr, plane_stride, block_stride, block_words, block_ids_ptr, block_offsets, nullptr,
         nullptr, payload_count, [&](auto& a, unsigned long long, unsigned long long before) {
           a.records = reinterpret_cast<unsigned int*>(workspace_ptr) + kTorchopRecordWords * before;
-          torchop_presence_tile<<<dim3(a.total_tiles), dim3(kThreads), 0, stream>>>(a);
+          if (block_words % 1024 == 0)
+            torchop_presence_tile<kPayloads<decltype(a)>, false><<<dim3(a.total_tiles), dim3(kThreads), 0, stream>>>(a);
+          else
+            torchop_presence_tile<kPayloads<decltype(a)>, true><<<dim3(a.total_tiles), dim3(kThreads), 0, stream>>>(a);
         });
     if (st != hipSuccess) return fail("torchop_presence", st);
   }
@@ -1182,13 +1244,16 @@ extern "C" long long kvq_splitzip_bf16_encode_torchop_paged(
     total += size;
   }
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
-  if (torchop_tile_geometry(kv_ptr, plane_stride, block_stride, block_words)) {
+  if (run_geometry(kv_ptr, plane_stride, block_stride, block_words)) {
     const hipError_t st = tile_launches(
         kv_ptr, plane_stride, block_stride, block_words, block_ids_ptr, block_offsets, out_offsets,
         encoded_bytes, payload_count, [&](auto& a, unsigned long long first, unsigned long long) {
           a.buf = reinterpret_cast<unsigned char*>(out_ptr);
           a.plans = reinterpret_cast<const TorchopPlan*>(plans_ptr) + first;
-          torchop_encode_tile<<<dim3(a.total_tiles), dim3(kThreads), 0, stream>>>(a);
+          if (block_words % 1024 == 0)
+            torchop_encode_tile<kPayloads<decltype(a)>, false><<<dim3(a.total_tiles), dim3(kThreads), 0, stream>>>(a);
+          else
+            torchop_encode_tile<kPayloads<decltype(a)>, true><<<dim3(a.total_tiles), dim3(kThreads), 0, stream>>>(a);
         });
     return st != hipSuccess ? fail("torchop_encode", st) : (long long)total;
   }
