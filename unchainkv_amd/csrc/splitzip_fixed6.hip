@@ -86,9 +86,10 @@ __global__ __launch_bounds__(kThreads) void palette_presence_tile(LaunchArgs a, 
   if (active) {
     if (kRuns) {
       // (a lane without a second run reads its first one twice: the same mask)
-      v0 = load_stream16(a.kv + run_source<kIds>(a, t, geo, in_plane + 8 * lane));
-      v1 = load_stream16(a.kv + run_source<kIds>(a, t, geo, in_plane + (active_b ? 512 : 0) +
-                                                                8 * lane));
+      unsigned long long run_a, run_b;
+      run_sources<kIds>(a, t, geo, in_plane, lane, active_b ? 512u : 0u, run_a, run_b);
+      v0 = load_stream16(a.kv + run_a);
+      v1 = load_stream16(a.kv + run_b);
     } else {
       const uint16_t* src = a.kv + wave_source<kIds>(a, t, geo, in_plane);
       v0 = load_stream16(src + 8 * lane);
@@ -223,9 +224,12 @@ __global__ __launch_bounds__(kThreads) void palette_encode_tile(LaunchArgs a, En
   uint32_t x[8];
   if (kRuns) {
     u32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
-    if (active) v0 = load_stream16(a.kv + run_source<kIds>(a, t, geo, in_plane + 8 * lane));
-    if (active_b)
-      v1 = load_stream16(a.kv + run_source<kIds>(a, t, geo, in_plane + 512 + 8 * lane));
+    if (active) {
+      unsigned long long run_a, run_b;
+      run_sources<kIds>(a, t, geo, in_plane, lane, active_b ? 512u : 0u, run_a, run_b);
+      v0 = load_stream16(a.kv + run_a);
+      v1 = load_stream16(a.kv + run_b);
+    }
     x[0] = v0.x; x[1] = v0.y; x[2] = v0.z; x[3] = v0.w;
     x[4] = v1.x; x[5] = v1.y; x[6] = v1.z; x[7] = v1.w;
   } else if (active) {
@@ -350,13 +354,12 @@ __device__ __forceinline__ void palette_decode_tile_body(const LaunchArgs& a,
     low_a = load_stream8(low + 8 * lane);
     low_b = load_stream8(low + second + 8 * lane);
     if (kRuns) {
-#pragma unroll
-      for (int run = 0; run < 2; ++run) {
-        const unsigned int word = in_plane + (run ? second : 0u) + 8 * lane;
-        const unsigned int j = div_u32(word, geo.bw_magic, geo.bw);
-        dst[run] = a.kv + t.plane * a.plane_stride + block_of(t, j) * a.block_stride +
-                   (word - j * geo.bw);
-      }
+      unsigned long long run_a, run_b;
+      run_offsets(geo, in_plane, t.blocks - 1, lane, second, [&](unsigned int j) {
+        return t.plane * a.plane_stride + block_of(t, j) * a.block_stride;
+      }, run_a, run_b);
+      dst[0] = a.kv + run_a;
+      dst[1] = a.kv + run_b;
     } else {
       dst[0] = a.kv + 8 * lane +
                wave_offset_by(a, t, geo, in_plane, [&](unsigned int j) { return block_of(t, j); });

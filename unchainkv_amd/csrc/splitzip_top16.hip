@@ -659,9 +659,13 @@ __global__ __launch_bounds__(kThreads) void top16_encode_tile(LaunchArgs a, Enco
   uint32_t x[8];
   if (kRuns) {
     u32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
-    if (active_a) v0 = load_stream16(a.kv + run_source<kIds>(a, t, geo, in_plane + 8 * lane));
-    if (active_b)
-      v1 = load_stream16(a.kv + run_source<kIds>(a, t, geo, in_plane + 512 + 8 * lane));
+    if (active_a) {
+      // (a lane without a second run reads its first one twice)
+      unsigned long long run_a, run_b;
+      run_sources<kIds>(a, t, geo, in_plane, lane, active_b ? 512u : 0u, run_a, run_b);
+      v0 = load_stream16(a.kv + run_a);
+      v1 = load_stream16(a.kv + run_b);
+    }
     x[0] = v0.x; x[1] = v0.y; x[2] = v0.z; x[3] = v0.w;
     x[4] = v1.x; x[5] = v1.y; x[6] = v1.z; x[7] = v1.w;
   } else if (active) {
@@ -864,7 +868,7 @@ __global__ __launch_bounds__(kThreads) void top16_decode_tile_inline(LaunchArgs 
 // The same over the run geometry, with a destination per lane and run. A 65.6 MB layer
 // of 12 requests with 7680-word blocks (6 heads of 80): the 16-word lanes of the
 // lanes kernels store and load 32-byte strides and realign their sections by
-// shuffles; encode + decode call 68.8 us with those, 61.4 us with runs.
+// shuffles; encode + decode call 68.8 us with those, 58.1 us with runs.
 template <bool kIds>
 __global__ __launch_bounds__(kThreads) void top16_decode_runs(LaunchArgs a, EncodeGeom geo) {
   const unsigned int lane = threadIdx.x & (kWave - 1);
@@ -886,8 +890,11 @@ __global__ __launch_bounds__(kThreads) void top16_decode_runs(LaunchArgs a, Enco
   const u32x2 body_b = load_stream8(pbody + second + 8 * lane);
   const uint32_t code_a = load_stream4(pcode + 4 * lane);
   const uint32_t code_b = load_stream4(pcode + second / 2 + 4 * lane);
-  uint16_t* dst_a = a.kv + run_source<kIds>(a, t, geo, in_plane + 8 * lane);
-  uint16_t* dst_b = a.kv + run_source<kIds>(a, t, geo, in_plane + second + 8 * lane);
+  __builtin_amdgcn_sched_barrier(0);
+  unsigned long long run_a, run_b;
+  run_sources<kIds>(a, t, geo, in_plane, lane, second, run_a, run_b);
+  uint16_t* const dst_a = a.kv + run_a;
+  uint16_t* const dst_b = a.kv + run_b;
   const u32x4 out_a = decode_run8(body_a, code_a, cb);
   const u32x4 out_b = decode_run8(body_b, code_b, cb);
   asm volatile("" ::"v"(out_a), "v"(out_b), "v"(dst_a), "v"(dst_b));

@@ -664,8 +664,7 @@ __device__ __forceinline__ unsigned int tile_payload(const TileArgs<kMax>& a, un
   return uniform(count - 1u);
 }
 
-// Element offset in the layer of payload word c, the first of a wave chunk (uniform)
-// or of a lane's 8-word run.
+// Element offset in the layer of the wave chunk starting at payload word c.
 template <unsigned int kMax>
 __device__ __forceinline__ unsigned long long chunk_source(const TileArgs<kMax>& a,
                                                            const TilePayload& d,
@@ -681,19 +680,20 @@ __device__ __forceinline__ unsigned long long chunk_source(const TileArgs<kMax>&
   return uniform64(plane * a.plane_stride + blk * a.block_stride + within);
 }
 
+// Element offsets of a lane's two runs at payload words c + 8 * lane and at_b more: the
+// payload's blocks are its K blocks, then its V blocks, so that runs on both sides of
+// the planes' border (tiles cover [0, n) as one range) need nothing of their own.
 template <unsigned int kMax>
-__device__ __forceinline__ unsigned long long run_source(const TileArgs<kMax>& a,
-                                                         const TilePayload& d,
-                                                         unsigned long long n,
-                                                         unsigned long long i) {
-  const EncodeGeom& geo = a.geo;
-  const unsigned long long half = n >> 1;
-  const unsigned int plane = i >= half ? 1u : 0u;
-  const unsigned int in_plane = (unsigned int)(i - plane * half);
-  const unsigned int j = div_u32(in_plane, geo.bw_magic, geo.bw);
-  const unsigned int within = in_plane - j * geo.bw;
-  const unsigned long long blk = (unsigned long long)a.ids[d.ids_offset + j];
-  return plane * a.plane_stride + blk * a.block_stride + within;
+__device__ __forceinline__ void run_sources(const TileArgs<kMax>& a, const TilePayload& d,
+                                            unsigned int c, unsigned int lane, unsigned int at_b,
+                                            unsigned long long& run_a,
+                                            unsigned long long& run_b) {
+  run_offsets(a.geo, c, 2 * d.block_count - 1, lane, at_b, [&](unsigned int j) {
+    const bool v = j >= d.block_count;
+    const unsigned long long blk =
+        (unsigned long long)a.ids[d.ids_offset + (v ? j - d.block_count : j)];
+    return (v ? a.plane_stride : 0ull) + blk * a.block_stride;
+  }, run_a, run_b);
 }
 
 // A lane's two runs of the wave chunk at payload word c, in words from c: 8 * lane and
@@ -722,10 +722,13 @@ __device__ __forceinline__ LaneRuns lane_runs(unsigned int lane, unsigned long l
 template <bool kRuns, unsigned int kMax>
 __device__ __forceinline__ void load_runs(const TileArgs<kMax>& a, const TilePayload& d,
                                           unsigned long long n, unsigned long long c,
-                                          const LaneRuns& r, u32x4& v0, u32x4& v1) {
+                                          unsigned int lane, const LaneRuns& r, u32x4& v0,
+                                          u32x4& v1) {
   if (kRuns) {
-    v0 = load_stream16(a.kv + run_source(a, d, n, c + r.at[0]));
-    v1 = load_stream16(a.kv + run_source(a, d, n, c + r.at[1]));
+    unsigned long long run_a, run_b;
+    run_sources(a, d, (unsigned int)c, lane, r.at[1] - r.at[0], run_a, run_b);
+    v0 = load_stream16(a.kv + run_a);
+    v1 = load_stream16(a.kv + run_b);
   } else {
     const uint16_t* src = a.kv + chunk_source(a, d, n, c);
     v0 = load_stream16(src + r.at[0]);
@@ -753,7 +756,7 @@ __global__ __launch_bounds__(kThreads) void torchop_presence_tile(TileArgs<kMax>
   const LaneRuns runs = lane_runs<kRuns>(lane, n, c);
   const bool active = runs.active;
   u32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
-  if (active) load_runs<kRuns>(a, d, n, c, runs, v0, v1);
+  if (active) load_runs<kRuns>(a, d, n, c, lane, runs, v0, v1);
   if (tid < 64) reinterpret_cast<unsigned int*>(s_high)[tid] = 0;
   if (tid == 0) s_nib = 0;
   __syncthreads();
@@ -796,7 +799,7 @@ __global__ __launch_bounds__(kThreads) void torchop_encode_tile(TileArgs<kMax> a
   const bool active = runs.active;
   // the words first: the plan's round trip overlaps with theirs
   u32x4 v0 = {0, 0, 0, 0}, v1 = {0, 0, 0, 0};
-  if (active) load_runs<kRuns>(a, d, n, c, runs, v0, v1);
+  if (active) load_runs<kRuns>(a, d, n, c, lane, runs, v0, v1);
   unsigned char* out = a.buf + d.buf_offset;
   const EncodeFields f = encode_prologue(a.plans + r, n, d.encoded, out, s_rank, local == 0);
   if (!f.ok) return;  // the whole workgroup
@@ -882,8 +885,10 @@ __global__ __launch_bounds__(kThreads) void torchop_decode_tile(TileArgs<kMax> a
   uint16_t* dst[2] = {nullptr, nullptr};  // of this lane's two runs
   if (active) {
     if (kRuns) {
-#pragma unroll
-      for (int run = 0; run < 2; ++run) dst[run] = a.kv + run_source(a, d, n, c + runs.at[run]);
+      unsigned long long run_a, run_b;
+      run_sources(a, d, (unsigned int)c, lane, runs.at[1] - runs.at[0], run_a, run_b);
+      dst[0] = a.kv + run_a;
+      dst[1] = a.kv + run_b;
     } else {
       uint16_t* chunk = a.kv + chunk_source(a, d, n, c);
 #pragma unroll
