@@ -476,6 +476,15 @@ long long kvq_splitzip_top16_writeback_paged(
 unsigned long long kvq_splitzip_top16_decode_attention_workspace_bytes(
     unsigned long long batch, unsigned long long kv_heads, unsigned long long max_ctx);
 
+/* 1 when every sequence's payload (its context in whole blocks) lies inside a buffer of
+ * payload_bytes bytes; *workspace_bytes then receives the workspace the call needs. 0
+ * otherwise, or for arguments the call declines. Host arrays; nothing is launched. */
+int kvq_splitzip_top16_decode_attention_fits(
+    const unsigned long long* payload_offsets, const unsigned long long* context_tokens,
+    unsigned long long batch, unsigned long long block_tokens, unsigned long long kv_heads,
+    unsigned long long head_dim, unsigned long long payload_bytes,
+    unsigned long long* workspace_bytes);
+
 long long kvq_splitzip_top16_decode_attention(
     unsigned long long q_ptr, unsigned long long out_ptr, unsigned long long payloads_ptr,
     const unsigned long long* payload_offsets, const unsigned long long* context_tokens,

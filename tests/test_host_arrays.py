@@ -1,0 +1,47 @@
+"""The host module's conversion of per-request numbers to u64 arrays, and the attention
+call's bounds check in the library: the same answers as the plain Python forms."""
+
+import ctypes
+
+import numpy as np
+import pytest
+
+from unchainkv_amd import codec_format, splitzip_cuda as sz
+
+
+@pytest.mark.parametrize("values", [
+    [0, 1, (1 << 64) - 1], [3], [True, 7], [], [5.9, 2], [-1, 4], [1 << 64, 3],
+    np.array([4, 9], dtype=np.int64), np.array([4.5, 9.0]), bytes(range(16)), (8, 16)])
+def test_u64_array(values):
+    want = (ctypes.c_ulonglong * len(values))(*map(int, values))
+    got = sz._u64_array(values)
+    assert len(got) == len(want) and list(got) == list(want)
+
+
+def fits(offsets, contexts, block_tokens, heads, size, head_dim=128):
+    lib = sz._load()
+    need = ctypes.c_ulonglong(123)
+    ok = lib.kvq_splitzip_top16_decode_attention_fits(
+        sz._u64_array(offsets), sz._u64_array(contexts), len(offsets), block_tokens, heads,
+        head_dim, size, ctypes.byref(need))
+    return bool(ok), need.value
+
+
+@pytest.mark.parametrize("contexts", [[1], [16, 17], [300, 5, 4096], [32768]])
+@pytest.mark.parametrize("heads,block_tokens", [(1, 16), (3, 8), (8, 32)])
+def test_attention_bounds(contexts, heads, block_tokens):
+    if not sz.available():
+        pytest.skip(sz.load_error())
+    offsets, end = [], 11
+    for ctx in contexts:
+        offsets.append(end)
+        span = -(-ctx // block_tokens) * block_tokens
+        end += codec_format.top16_encoded_size(2 * span * heads * 128)
+    assert fits(offsets, contexts, block_tokens, heads, end)[0]
+    assert not fits(offsets, contexts, block_tokens, heads, end - 1)[0]
+    assert not fits(offsets[:-1] + [end + 1], contexts, block_tokens, heads, end)[0]
+    assert not fits([-5] + offsets[1:], contexts, block_tokens, heads, end)[0]
+    assert not fits(offsets, [-3] + contexts[1:], block_tokens, heads, end)[0]
+    assert not fits(offsets, contexts, 0, heads, end)[0]
+    assert not fits(offsets, contexts, block_tokens, 0, end)[0]
+    assert not fits(offsets, contexts, block_tokens, heads, end, head_dim=64)[0]

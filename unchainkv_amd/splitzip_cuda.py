@@ -26,6 +26,7 @@ from __future__ import annotations
 
 import array
 import ctypes
+import operator
 import os
 from pathlib import Path
 
@@ -99,6 +100,8 @@ _SIGNATURES = (
     ("kvq_splitzip_top16_noalloc_scratch_bytes", [], _U64, False),
     ("kvq_splitzip_palette_paged_workspace_bytes", [_U64, _U64P, _U64], _U64, False),
     ("kvq_splitzip_top16_decode_attention_workspace_bytes", [_U64] * 3, _U64, False),
+    ("kvq_splitzip_top16_decode_attention_fits", [_U64P, _U64P, _U64, _U64, _U64, _U64, _U64, _U64P],
+     ctypes.c_int, False),
     ("kvq_splitzip_exponent_histogram_workspace_bytes", [_U64] * 2, _U64, False),
     ("kvq_splitzip_exponent_histogram_paged", [_U64] * 10, ctypes.c_longlong, False),
     (
@@ -232,6 +235,17 @@ def _stream_handle(device, torch) -> int:
         index = device.index if device.index is not None else torch.cuda.current_device()
         return int(raw(index))
     return int(torch.cuda.current_stream(device).cuda_stream)
+
+
+def _u64_array(values):
+    """ctypes u64 array of a sequence of integers. ``array`` converts 64 Python ints in
+    about a microsecond, a ctypes array from ``map(int, values)`` in 3; what it does not
+    take (numbers that ``int()`` truncates, negative ones, which wrap) goes the slow way."""
+    n = len(values)
+    try:
+        return (ctypes.c_ulonglong * n).from_buffer(array.array("Q", values))
+    except (TypeError, OverflowError, ValueError):
+        return (ctypes.c_ulonglong * n)(*map(int, values))
 
 
 # ---------------------------------------------------------------------------
@@ -499,6 +513,7 @@ class PagedBatch:
         self.max_block = max(flat)
         self.unique_blocks = len(set(flat)) == len(flat)
         self._palette = {}
+        self._directory_bytes = None
         self._workspace = None
         self._runs = None
         self._writeback = {}
@@ -530,7 +545,9 @@ class PagedBatch:
         """ctypes u64 array of `values` (the batch's own array when it is the same list)."""
         if values is own:
             return own_array
-        return (ctypes.c_ulonglong * self.payload_count)(*map(int, values))
+        if len(values) != self.payload_count:
+            raise ValueError("one value per request")
+        return _u64_array(values)
 
     @property
     def total_raw_bytes(self) -> int:
@@ -569,12 +586,15 @@ class PagedBatch:
 
     def directory_bytes(self) -> int:
         """Bytes of the batch's escape directory (0 when its block geometry has none:
-        block words not a multiple of 1024)."""
-        lib = _load()
-        query = getattr(lib, "kvq_splitzip_top16_paged_directory_bytes", None) if lib else None
-        if query is None:
-            raise RuntimeError(f"splitzip HIP library unavailable: {load_error()}")
-        return int(query(self.block_words, self._block_offsets, self.payload_count))
+        block words not a multiple of 1024), asked of the library once."""
+        if self._directory_bytes is None:
+            lib = _load()
+            query = getattr(lib, "kvq_splitzip_top16_paged_directory_bytes", None) if lib else None
+            if query is None:
+                raise RuntimeError(f"splitzip HIP library unavailable: {load_error()}")
+            self._directory_bytes = int(query(self.block_words, self._block_offsets,
+                                              self.payload_count))
+        return self._directory_bytes
 
     def new_directory(self, torch=None):
         """Device buffer for the escape directory, or None when the batch has none."""
@@ -665,17 +685,16 @@ def _paged_layout_ok(kv_layer, batch: PagedBatch, torch) -> bool:
     shape = kv_layer.shape
     if len(shape) < 3 or shape[0] != 2 or not kv_layer.is_contiguous():
         return False
-    block_words = 1
-    for extent in shape[2:]:
-        block_words *= extent
-    return block_words == batch.block_words and batch.max_block < shape[1]
+    # (a layer without blocks fails the second test)
+    blocks = shape[1]
+    return kv_layer.numel() == 2 * blocks * batch.block_words and batch.max_block < blocks
 
 
 def _payloads_fit(source, src_offsets, encoded_bytes, batch: PagedBatch) -> bool:
     if len(src_offsets) != batch.payload_count or len(encoded_bytes) != batch.payload_count:
         return False
     size = source.numel() if hasattr(source, "numel") and callable(source.numel) else source.size
-    return all(o + e <= size for o, e in zip(src_offsets, encoded_bytes))
+    return max(map(operator.add, src_offsets, encoded_bytes)) <= size
 
 
 def _byte_buffer_ok(buf, device, nbytes: int, torch) -> bool:
@@ -918,7 +937,7 @@ def encode_bf16_paged(kv_layer, batch: PagedBatch, out, workspace, bits: int = 6
             if first < 0 or 32 * (first + 2 * (-(-(n // 2) // 4096))) > presence.numel():
                 return None
         extra = (int(presence.data_ptr()),
-                 (ctypes.c_ulonglong * batch.payload_count)(*map(int, presence_first)))
+                 _u64_array(presence_first))
     stream = _stream_handle(kv_layer.device, torch)
     encoded = encode(int(kv_layer.data_ptr()), int(kv_layer.stride(0)), int(kv_layer.stride(1)),
                      batch.block_words, int(batch.ids.data_ptr()), batch._block_offsets,
@@ -947,7 +966,7 @@ def _encode_bf16_paged_info(kv_layer, batch, out, bits, palette_info, info_first
     records = palette_info.numel() // PagedBatch.PALETTE_INFO_BYTES
     batch.palette_layout(bits)
     offs = batch._palette[bits][3]
-    firsts = (ctypes.c_ulonglong * batch.payload_count)(*map(int, info_first))
+    firsts = _u64_array(info_first)
     stream = _stream_handle(kv_layer.device, torch)
     encoded = encode(int(kv_layer.data_ptr()), int(kv_layer.stride(0)), int(kv_layer.stride(1)),
                      batch.block_words, int(batch.ids.data_ptr()), batch._block_offsets,
@@ -1074,7 +1093,7 @@ def read_torchop_plans(host_plans) -> list[tuple[int, int]]:
 
     raw = np.asarray(host_plans, dtype=np.uint8).reshape(-1, TORCHOP_PLAN_BYTES)
     sizes = raw[:, 48:56].copy().view(np.uint64).reshape(-1)
-    return [(int(raw[r, 36]), int(sizes[r])) for r in range(raw.shape[0])]
+    return list(zip(raw[:, 36].tolist(), sizes.tolist()))
 
 
 def encode_torchop_paged(kv_layer, batch: PagedBatch, plans, out, out_offsets,
@@ -1135,7 +1154,8 @@ def decode_attention_top16(q, payloads, payload_offsets, context_tokens, kv_head
     128) bf16 output, or ``None`` when the kernel declines."""
     lib = _load()
     attend = getattr(lib, "kvq_splitzip_top16_decode_attention", None) if lib else None
-    if attend is None:
+    fits = getattr(lib, "kvq_splitzip_top16_decode_attention_fits", None) if lib else None
+    if attend is None or fits is None:
         return None
     import torch
 
@@ -1148,11 +1168,14 @@ def decode_attention_top16(q, payloads, payload_offsets, context_tokens, kv_head
         return None
     if block_tokens <= 0:
         return None
-    for off, ctx in zip(payload_offsets, context_tokens):
-        span = -(-int(ctx) // block_tokens) * block_tokens
-        n = 2 * span * kv_heads * head_dim
-        if int(off) < 0 or int(off) + codec_format.top16_encoded_size(n) > payloads.numel():
-            return None
+    if not batch:
+        raise ValueError("no sequences")
+    offs, ctxs = _u64_array(payload_offsets), _u64_array(context_tokens)
+    need = ctypes.c_ulonglong()
+    if not fits(offs, ctxs, batch, int(block_tokens), kv_heads, head_dim, payloads.numel(),
+                ctypes.byref(need)):
+        return None
+    need = need.value
     if tables is None:
         tables = _resolve_tables(layer_index, codebooks, q.device, torch)
     if tables is None:
@@ -1164,12 +1187,8 @@ def decode_attention_top16(q, payloads, payload_offsets, context_tokens, kv_head
     elif out.dtype != torch.bfloat16 or not out.is_contiguous() or out.shape != q.shape or \
             out.device != q.device:
         return None
-    max_ctx = max(int(c) for c in context_tokens)
-    need = int(lib.kvq_splitzip_top16_decode_attention_workspace_bytes(batch, kv_heads, max_ctx))
     if not _byte_buffer_ok(workspace, q.device, need, torch):
         workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=q.device)
-    offs = (ctypes.c_ulonglong * batch)(*map(int, payload_offsets))
-    ctxs = (ctypes.c_ulonglong * batch)(*map(int, context_tokens))
     stream = _stream_handle(q.device, torch)
     got = attend(int(q.data_ptr()), int(out.data_ptr()), int(payloads.data_ptr()), offs, ctxs,
                  int(block_tokens), batch, q_heads, kv_heads, head_dim, int(tables.data_ptr()),
