@@ -12,10 +12,13 @@
 // from run to run; every order decodes to the same words).
 //
 // Kernels (one payload or every request of a paged layer per launch):
-//   palette_presence_tile / _generic   256-bit presence mask of the high bytes, one
-//       mask per 4096-word tile (or per workgroup of a grid-stride pass)
+//   palette_presence_span              256-bit presence mask of the high bytes, one
+//       mask per span of tiles, few enough for the encode to form the palette itself
+//   palette_presence_tile / _generic   the same, one mask per 4096-word tile (or per
+//       workgroup of a grid-stride pass)
 //   palette_reduce                     per payload: OR of its masks -> ascending
-//       palette, rank table and distinct count (PaletteInfo in the workspace)
+//       palette, rank table and distinct count (PaletteInfo in the workspace), after
+//       masks per tile or workgroup
 //   palette_encode_tile / _generic     header + palette, low bytes, packed codes
 //   palette_decode_tile / _generic     decode + scatter (no-op unless byte 0 is the
 //       format's mode byte)
@@ -108,6 +111,95 @@ __global__ __launch_bounds__(kThreads) void palette_presence_tile(LaunchArgs a, 
   presence_flush(s_seen, masks + (unsigned long long)tile * 8);
 }
 
+// Span presence: few, long workgroups of 8 waves, so that a payload has at most
+// kSpanMasks masks and the encode tile kernel can form the palette from them itself
+// (palette_from_masks): no reduce launch between the two. A workgroup covers
+// 2^span_shift consecutive tiles of a payload, a wave every eighth 1024-word chunk of
+// them. Its lanes first look up one chunk's address each (one round trip for all block
+// ids); the walk then has two batches of two chunks in flight and no dependent load.
+// 69 MB of words in 8 requests of 500 to 4096 tokens: 15.0 us (4.6 TB/s) and an encode
+// of 26.1 us, against 14.4 us (a workgroup per tile), 4.5 us (reduce) and 24.0 us: 72.4 ->
+// 69.3 us per encode + decode call; 260 MB in 6 requests 235.9 -> 226.9 us; calls of a
+// few MB, which their launches bound, 24 -> 21 us. With at most 128 masks per payload (longer
+// spans) 69.7 us, with 64 71.6 us.
+constexpr unsigned int kSpanMasks = 256;
+constexpr unsigned int kSpanWaves = 8;
+constexpr unsigned int kSpanMaxShift = 7;  // 128 tiles: 64 chunks per wave, one per lane
+
+template <bool kIds>
+__global__ __launch_bounds__(kSpanWaves * kWave) void palette_presence_span(
+    LaunchArgs a, EncodeGeom geo, unsigned int* masks, unsigned int span_shift) {
+  __shared__ unsigned char s_seen[256];
+  const unsigned int tid = threadIdx.x, lane = tid & (kWave - 1), wave = uniform(tid >> 6);
+  const unsigned int span = group_index();
+  const PayloadDesc d = a.p[find_slot_payload(a, span)];
+  const unsigned int half = (unsigned int)(((unsigned long long)d.block_count * geo.bw) >> 10);
+  const unsigned int per_plane = (half + 3) / 4;  // tiles
+  // the span's tiles in chunks: a plane's last tile may hold fewer than four
+  const unsigned int tile0 = (span - d.slot_group_begin) << span_shift;
+  const unsigned int tile1 = min(tile0 + (1u << span_shift), 2 * per_plane);
+  auto chunk_of = [&](unsigned int tile) {
+    return tile < per_plane ? 4 * tile : min(half + 4 * (tile - per_plane), 2 * half);
+  };
+  const unsigned int q0 = chunk_of(tile0) + wave, q1 = chunk_of(tile1);
+  const unsigned int chunks = q1 > q0 ? (q1 - q0 + kSpanWaves - 1) / kSpanWaves : 0;
+  if (tid < 64) reinterpret_cast<unsigned int*>(s_seen)[tid] = 0;
+  __syncthreads();
+  if (chunks) {
+    // lane i: the element offset of the wave's i-th chunk
+    const unsigned int q = q0 + kSpanWaves * min(lane, chunks - 1);
+    const unsigned int plane = q >= half ? 1u : 0u;
+    const unsigned int in_plane = (q - plane * half) << 10;
+    const unsigned int j = div_u32(in_plane, geo.bw_magic, geo.bw);
+    const unsigned long long blk = kIds ? (unsigned long long)a.ids[d.ids_offset + j]
+                                        : a.block_start + j;
+    const unsigned long long off =
+        plane * a.plane_stride + blk * a.block_stride + (in_plane - j * geo.bw);
+    const unsigned int off_lo = (unsigned int)off, off_hi = (unsigned int)(off >> 32);
+    // chunks i and i + 1 (past the end the last one again: the same bytes)
+    auto load = [&](u32x4 (&v)[4], unsigned int i) {
+#pragma unroll
+      for (unsigned int c = 0; c < 2; ++c) {
+        const unsigned int k = min(i + c, chunks - 1);
+        const unsigned long long at =
+            (unsigned int)__builtin_amdgcn_readlane((int)off_lo, (int)k) |
+            ((unsigned long long)(unsigned int)__builtin_amdgcn_readlane((int)off_hi, (int)k)
+             << 32);
+        v[2 * c] = load_stream16(a.kv + at + 8 * lane);
+        v[2 * c + 1] = load_stream16(a.kv + at + 512 + 8 * lane);
+      }
+    };
+    auto mark = [&](const u32x4 (&v)[4]) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const uint32_t x[4] = {v[c].x, v[c].y, v[c].z, v[c].w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          s_seen[(x[k] >> 8) & 0xFF] = 1;
+          s_seen[x[k] >> 24] = 1;
+        }
+      }
+    };
+    u32x4 v0[4], v1[4];
+    load(v0, 0);
+    for (unsigned int i = 0; i < chunks; i += 4) {
+      load(v1, i + 2);
+      mark(v0);
+      load(v0, i + 4);
+      mark(v1);
+    }
+  }
+  __syncthreads();
+  if (wave < 4) {
+    const unsigned long long bits = __ballot(s_seen[tid] != 0);
+    if (lane == 0) {
+      unsigned int* out = masks + 8ull * span + 2 * wave;
+      out[0] = (unsigned int)bits;
+      out[1] = (unsigned int)(bits >> 32);
+    }
+  }
+}
+
 // Grid-stride presence pass over any geometry: grid = payload_count x groups.
 __global__ __launch_bounds__(kThreads) void palette_presence_generic(LaunchArgs a,
                                                                      unsigned int groups,
@@ -141,6 +233,79 @@ __global__ __launch_bounds__(kThreads) void palette_reduce(LaunchArgs a, unsigne
 
 // ---------------------------------------------------------------------------
 // encode
+
+// OR of `count` (at most kSpanMasks) masks at `masks` as eight scalars, by the whole
+// workgroup: a wave takes a quarter of them (lane l the quads l & 1 of every 32nd mask
+// from its l / 2-th on), merges rows of 16 lanes by rotations that keep the parity and
+// the four rows by scalar reads; the waves' results meet in LDS (s_part; one barrier).
+__device__ __forceinline__ void or_masks(const unsigned int* masks, unsigned int count,
+                                         u32x4 (&s_part)[4][2], unsigned int (&mask)[8]) {
+  const unsigned int lane = threadIdx.x & (kWave - 1), wave = uniform(threadIdx.x >> 6);
+  const u32x4* quads = reinterpret_cast<const u32x4*>(masks);
+  constexpr unsigned int kPer = kSpanMasks / 128;  // quads per lane
+  u32x4 part[kPer];
+#pragma unroll
+  for (unsigned int k = 0; k < kPer; ++k) {
+    // (past the last mask the first one: the OR stays)
+    const unsigned int m = lane / 2 + 32 * (wave + 4 * k);
+    part[k] = quads[m < count ? 2 * m + (lane & 1) : (lane & 1)];
+  }
+  unsigned int v[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (unsigned int k = 0; k < kPer; ++k) {
+    v[0] |= part[k].x;
+    v[1] |= part[k].y;
+    v[2] |= part[k].z;
+    v[3] |= part[k].w;
+  }
+  unsigned int own[8];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    // row_ror by 8, 4 and 2 lanes
+    v[k] |= (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v[k], 0x128, 0xF, 0xF, false);
+    v[k] |= (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v[k], 0x124, 0xF, 0xF, false);
+    v[k] |= (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v[k], 0x122, 0xF, 0xF, false);
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      unsigned int m = 0;
+#pragma unroll
+      for (int row = 0; row < 4; ++row)
+        m |= (unsigned int)__builtin_amdgcn_readlane((int)v[k], 16 * row + q);
+      own[4 * q + k] = m;
+    }
+  }
+  if (lane < 2)
+    s_part[wave][lane] = lane == 0 ? u32x4{own[0], own[1], own[2], own[3]}
+                                   : u32x4{own[4], own[5], own[6], own[7]};
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const u32x4 m = s_part[0][q] | s_part[1][q] | s_part[2][q] | s_part[3][q];
+    mask[4 * q] = uniform(m.x);
+    mask[4 * q + 1] = uniform(m.y);
+    mask[4 * q + 2] = uniform(m.z);
+    mask[4 * q + 3] = uniform(m.w);
+  }
+}
+
+// Rank of high byte tid in the ascending palette of `mask` (0 when absent), whether it
+// is present, and the number of distinct bytes. A wave's 64 bytes are two dwords.
+__device__ __forceinline__ unsigned int rank_in(const unsigned int (&mask)[8], bool& present,
+                                                unsigned int& distinct) {
+  const unsigned int wave = uniform(threadIdx.x >> 6), lane = threadIdx.x & (kWave - 1);
+  unsigned int below = 0, lo = 0, hi = 0;
+  distinct = 0;
+#pragma unroll
+  for (unsigned int w = 0; w < 4; ++w) {
+    const unsigned int c = __popc(mask[2 * w]) + __popc(mask[2 * w + 1]);
+    distinct += c;
+    below += w < wave ? c : 0u;
+    lo = w == wave ? mask[2 * w] : lo;
+    hi = w == wave ? mask[2 * w + 1] : hi;
+  }
+  present = ((lane < 32 ? lo >> lane : hi >> (lane & 31)) & 1u) != 0;
+  return present ? __builtin_amdgcn_mbcnt_hi(hi, __builtin_amdgcn_mbcnt_lo(lo, below)) : 0u;
+}
 
 // Header and palette of a payload (from its info); 255 alone on overflow.
 template <int kBits>
@@ -203,11 +368,16 @@ __device__ __forceinline__ unsigned long long unstage_run(const unsigned char* s
   return bits;
 }
 
-// kIndexed: payload r's palette is info[a.p[r].mask_begin] (palettes computed by a
-// Top-16 probe encode for a larger batch), else info[r].
-template <bool kIds, int kBits, bool kIndexed = false, bool kRuns = false>
+// The palette of payload r: info[r] (kInfo), info[a.p[r].mask_begin] (kIndexed: palettes
+// computed by a Top-16 probe encode for a larger batch), or the OR of its span masks
+// from a.p[r].slot_group_begin on, one per 2^span_shift tiles (kSpans).
+enum class From { kInfo, kIndexed, kSpans };
+
+template <bool kIds, int kBits, From kFrom = From::kInfo, bool kRuns = false>
 __global__ __launch_bounds__(kThreads) void palette_encode_tile(LaunchArgs a, EncodeGeom geo,
-                                                                const PaletteInfo* info) {
+                                                                const PaletteInfo* info,
+                                                                const unsigned int* masks,
+                                                                unsigned int span_shift) {
   using P = Palette<kBits>;
   constexpr unsigned int kWaveCodeBytes = 128 * kBits;  // 1024 words
   __shared__ uint32_t s_rank[64];
@@ -216,7 +386,8 @@ __global__ __launch_bounds__(kThreads) void palette_encode_tile(LaunchArgs a, En
   const unsigned int lane = tid & (kWave - 1);
   const unsigned int wave = uniform(tid >> 6);
   const PlaneTile t = plane_tile<kTileShift>(a, group_index());
-  const PaletteInfo& pi = info[kIndexed ? a.p[t.payload_index].mask_begin : t.payload_index];
+  const PaletteInfo& pi =
+      info[kFrom == From::kIndexed ? a.p[t.payload_index].mask_begin : t.payload_index];
   const unsigned int in_plane = t.in_plane0 + wave * 1024;
   const unsigned long long wstart = t.plane * (t.n >> 1) + in_plane;  // payload word
   const bool active = wave * 1024 + (kRuns ? 8 * lane : 0) < t.words;
@@ -242,9 +413,27 @@ __global__ __launch_bounds__(kThreads) void palette_encode_tile(LaunchArgs a, En
 #pragma unroll
     for (int k = 0; k < 8; ++k) x[k] = 0;
   }
-  if (tid < 64) s_rank[tid] = reinterpret_cast<const uint32_t*>(pi.rank)[tid];
-  const unsigned int distinct = pi.distinct;
-  if (t.local_tile == 0) write_palette_header<kBits>(t.payload, pi);
+  unsigned int distinct;
+  if (kFrom == From::kSpans) {
+    __shared__ u32x4 s_part[4][2];
+    unsigned int mask[8];
+    or_masks(masks + 8ull * a.p[t.payload_index].slot_group_begin,
+             (t.payload_tiles + (1u << span_shift) - 1) >> span_shift, s_part, mask);
+    bool present;
+    const unsigned int r = rank_in(mask, present, distinct);
+    reinterpret_cast<unsigned char*>(s_rank)[tid] = (unsigned char)r;
+    if (t.local_tile == 0) {
+      // the header: palette ascending, zeros after it; 255 alone on overflow
+      const bool over = distinct > (unsigned int)P::kLimit;
+      if (tid == 0) t.payload[0] = over ? 255 : (unsigned char)P::kMode;
+      if (!over && present) t.payload[1 + r] = (unsigned char)tid;
+      if (!over && tid >= distinct && tid < (unsigned int)P::kLimit) t.payload[1 + tid] = 0;
+    }
+  } else {
+    if (tid < 64) s_rank[tid] = reinterpret_cast<const uint32_t*>(pi.rank)[tid];
+    distinct = pi.distinct;
+    if (t.local_tile == 0) write_palette_header<kBits>(t.payload, pi);
+  }
   // overflow: the reference writes byte 0 only (kvq_splitzip_cuda.cu:58-61)
   if (distinct > (unsigned int)P::kLimit) return;
   __syncthreads();  // s_rank ready
@@ -454,6 +643,42 @@ unsigned int tiles_of(unsigned long long n) {
   return 2u * (unsigned int)(((n >> 1) + kTileWords - 1) >> kTileShift);
 }
 
+// Tiles of payload r of a launch.
+unsigned int tiles_in(const LaunchArgs& a, unsigned int r) {
+  return (r + 1 < a.payload_count ? a.p[r + 1].tile_begin : a.total_tiles) - a.p[r].tile_begin;
+}
+
+// log2 of the tiles per presence span, 0 for the tile presence pass and its reduce. The
+// spans are the shortest with which no payload has more than kSpanMasks of them (at
+// least two tiles: one chunk per wave), as long as they are short or enough of them
+// to keep the memory busy: below three quarters of a workgroup per CU the pass takes
+// longer than the reduce launch it saves (two requests of 11 MB: 32.1 us both ways).
+constexpr unsigned int kSpanFill = 192;
+
+unsigned int span_shift(const LaunchArgs& a) {
+  unsigned int most = 0;
+  for (unsigned int r = 0; r < a.payload_count; ++r) most = std::max(most, tiles_in(a, r));
+  unsigned int shift = 1;
+  while (shift <= kSpanMaxShift && ((most + (1u << shift) - 1) >> shift) > kSpanMasks) ++shift;
+  if (shift > kSpanMaxShift) return 0;
+  return shift == 1 || (a.total_tiles >> shift) >= kSpanFill ? shift : 0;
+}
+
+// Sets each payload's first span (slot_group_begin); the number of spans.
+unsigned int set_spans(LaunchArgs& a, unsigned int shift) {
+  unsigned int spans = 0, first = 0;
+  bool uniform_spans = true;
+  for (unsigned int r = 0; r < a.payload_count; ++r) {
+    const unsigned int own = (tiles_in(a, r) + (1u << shift) - 1) >> shift;
+    if (r == 0) first = own;
+    uniform_spans = uniform_spans && own == first;
+    a.p[r].slot_group_begin = spans;
+    spans += own;
+  }
+  a.uniform_slot_groups = uniform_spans ? first : 0;
+  return spans;
+}
+
 // masks_given: `masks` already holds one mask per tile of every payload (from the
 // Top-16 encode), at each payload's mask_begin; the presence pass is skipped.
 template <int kBits>
@@ -463,6 +688,22 @@ long long launch_palette_encode(LaunchArgs& a, const EncodeGeom& g, Layout layou
   const dim3 block(kThreads);
   const bool tiles = layout != Layout::kGeneric;
   const dim3 grid(a.total_tiles);
+  const unsigned int shift = layout == Layout::kTile && !masks_given ? span_shift(a) : 0;
+  if (shift != 0) {
+    const dim3 spans(set_spans(a, shift)), threads(kSpanWaves * kWave);
+    if (a.ids)
+      palette_presence_span<true><<<spans, threads, 0, stream>>>(a, g, masks, shift);
+    else
+      palette_presence_span<false><<<spans, threads, 0, stream>>>(a, g, masks, shift);
+    if (long long rc = check("palette_presence")) return rc;
+    if (a.ids)
+      palette_encode_tile<true, kBits, From::kSpans><<<grid, block, 0, stream>>>(a, g, info, masks,
+                                                                                 shift);
+    else
+      palette_encode_tile<false, kBits, From::kSpans><<<grid, block, 0, stream>>>(a, g, info,
+                                                                                  masks, shift);
+    return check("palette_encode");
+  }
   if (masks_given) {
     presence_groups = 0;
   } else if (layout == Layout::kRuns) {
@@ -485,14 +726,16 @@ long long launch_palette_encode(LaunchArgs& a, const EncodeGeom& g, Layout layou
   if (long long rc = check("palette_reduce")) return rc;
   if (layout == Layout::kRuns) {
     if (a.ids)
-      palette_encode_tile<true, kBits, false, true><<<grid, block, 0, stream>>>(a, g, info);
+      palette_encode_tile<true, kBits, From::kInfo, true><<<grid, block, 0, stream>>>(
+          a, g, info, nullptr, 0);
     else
-      palette_encode_tile<false, kBits, false, true><<<grid, block, 0, stream>>>(a, g, info);
+      palette_encode_tile<false, kBits, From::kInfo, true><<<grid, block, 0, stream>>>(
+          a, g, info, nullptr, 0);
   } else if (tiles) {
     if (a.ids)
-      palette_encode_tile<true, kBits><<<grid, block, 0, stream>>>(a, g, info);
+      palette_encode_tile<true, kBits><<<grid, block, 0, stream>>>(a, g, info, nullptr, 0);
     else
-      palette_encode_tile<false, kBits><<<grid, block, 0, stream>>>(a, g, info);
+      palette_encode_tile<false, kBits><<<grid, block, 0, stream>>>(a, g, info, nullptr, 0);
   } else {
     hipLaunchKernelGGL(palette_encode_generic<kBits>, dim3(a.payload_count * kGenericGroups),
                        block, 0, stream, a, info);
@@ -531,11 +774,11 @@ long long launch_palette_encode_info(LaunchArgs& a, const EncodeGeom& g, const P
                                      hipStream_t stream) {
   const dim3 block(kThreads);
   if (a.ids)
-    hipLaunchKernelGGL((palette_encode_tile<true, kBits, true>), dim3(a.total_tiles), block, 0,
-                       stream, a, g, info);
+    palette_encode_tile<true, kBits, From::kIndexed><<<dim3(a.total_tiles), block, 0, stream>>>(
+        a, g, info, nullptr, 0);
   else
-    hipLaunchKernelGGL((palette_encode_tile<false, kBits, true>), dim3(a.total_tiles), block, 0,
-                       stream, a, g, info);
+    palette_encode_tile<false, kBits, From::kIndexed><<<dim3(a.total_tiles), block, 0, stream>>>(
+        a, g, info, nullptr, 0);
   return check("palette_encode (probe palettes)");
 }
 
