@@ -13,9 +13,9 @@ import oracle
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
-BW = 1024  # a quarter of a tile: 4 blocks per tile and plane
 CASES = {
-    # blocks of each request: tiles per request at most 512 -> spans of two tiles
+    # blocks of 1024 words (four per tile and plane) of each request: at most 512 tiles
+    # -> spans of two tiles
     "two_tiles": [1, 2, 3, 4, 5, 9, 1023, 1024],
     # 514 tiles at most -> four tiles, with enough spans in all
     "four_tiles": [1027] * 2 + [1, 6, 15],
@@ -24,6 +24,9 @@ CASES = {
     # 2050 tiles at most -> sixteen tiles
     "sixteen_tiles": [4099] * 2 + [37],
 }
+# the run geometry: blocks of 1032 words (a chunk in two blocks, planes that end inside
+# a chunk) and of 3848 (most chunks in one)
+BLOCK_WORDS = {1024: CASES, 1032: ["two_tiles", "four_tiles", "tile_pass"], 3848: ["two_tiles"]}
 
 
 @pytest.fixture(scope="module")
@@ -37,14 +40,14 @@ def sz():
 
 
 @pytest.mark.parametrize("bits", [6, 5])
-@pytest.mark.parametrize("name", list(CASES))
-def test_spans(sz, name, bits):
-    print("[case] palette spans", name, bits, flush=True)
+@pytest.mark.parametrize("bw,name", [(bw, n) for bw, names in BLOCK_WORDS.items() for n in names])
+def test_spans(sz, bw, name, bits):
+    print("[case] palette spans", bw, name, bits, flush=True)
     counts = CASES[name]
     limit = 64 if bits == 6 else 32
     rng = np.random.default_rng(len(counts) + bits)
     pool = sum(counts) + 3
-    words = rng.integers(0, 1 << 16, (2, pool, BW), dtype=np.uint16)
+    words = rng.integers(0, 1 << 16, (2, pool, bw), dtype=np.uint16)
     words = ((0x40 + (words >> 8) % (limit - 5)) << 8 | (words & 0xFF)).astype(np.uint16)
     ids = rng.permutation(pool).tolist()
     send, at = [], 0
@@ -62,9 +65,9 @@ def test_spans(sz, name, bits):
             # a request too short for limit - 5 more high bytes overflows by its own
             flat[1:1 + limit - 5] = (0x40 + np.arange(limit - 5)) << 8
             flat[int(rng.integers(n // 2 + 1, n - 1))] = 0xFF00
-        words[:, t] = flat.reshape(2, len(t), BW)
+        words[:, t] = flat.reshape(2, len(t), bw)
     layer = torch.from_numpy(words.view(np.int16)).cuda().view(torch.bfloat16)
-    batch = sz.PagedBatch(send, BW, "cuda")
+    batch = sz.PagedBatch(send, bw, "cuda")
     offsets, sizes, _ = batch.palette_layout(bits)
     out = batch.new_palette_buffer(bits).fill_(0x5A)
     assert sz.encode_bf16_paged(layer, batch, out, batch.new_palette_workspace(), bits) == \
@@ -79,7 +82,7 @@ def test_spans(sz, name, bits):
     recv = [[ids[(b + 1) % pool] for b in range(at - len(t), at)]
             for t, at in zip(send, np.cumsum(counts))]
     target = torch.zeros_like(layer)
-    assert sz.decode_bf16_paged(out, offsets, sizes, target, sz.PagedBatch(recv, BW, "cuda"),
+    assert sz.decode_bf16_paged(out, offsets, sizes, target, sz.PagedBatch(recv, bw, "cuda"),
                                 bits) == batch.total_raw_bytes
     restored = target.view(torch.int16).cpu().numpy().view(np.uint16)
     for r, (t, u) in enumerate(zip(send, recv)):

@@ -381,7 +381,7 @@ __device__ __forceinline__ unsigned long long wave_source(const LaunchArgs& a, c
 // on a multiple of 8 words, so runs, not waves, are active or not. Against the generic
 // palette and torch-op kernels, which take a word (or 16) per thread with 64-bit
 // divisions and byte accesses: fixed6 encode + decode of 64 MB with 7680-word blocks
-// 1386 -> 71.5 us.
+// 1386 -> 65.5 us.
 
 // The layout's share of the rule: whole 16-byte runs of the layer.
 inline bool run_geometry(unsigned long long kv_ptr, unsigned long long plane_stride,
@@ -397,8 +397,7 @@ inline bool run_geometry(unsigned long long kv_ptr, unsigned long long plane_str
 // lane picks one by a compare. Smaller ones: a 24-bit division of the run's distance
 // from the first block and a gathered id load per run. With a 64-bit multiply-high
 // division and a gathered id per run at every size, the Top-16 encode + decode call of
-// 65.6 MB with 7680-word blocks took 61.4 us instead of 58.1, fixed6 over 64 MB 75.0 us
-// instead of 71.5.
+// 65.6 MB with 7680-word blocks took 61.4 us instead of 58.1.
 template <typename BaseOf>
 __device__ __forceinline__ void run_offsets(const EncodeGeom& geo, unsigned int first,
                                             unsigned int last, unsigned int lane,

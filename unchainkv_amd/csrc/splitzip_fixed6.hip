@@ -111,6 +111,13 @@ __global__ __launch_bounds__(kThreads) void palette_presence_tile(LaunchArgs a, 
   presence_flush(s_seen, masks + (unsigned long long)tile * 8);
 }
 
+// Lane k's 64-bit value, given in halves (k uniform).
+__device__ __forceinline__ unsigned long long lane_value(unsigned int lo, unsigned int hi,
+                                                         unsigned int k) {
+  return (unsigned int)__builtin_amdgcn_readlane((int)lo, (int)k) |
+         ((unsigned long long)(unsigned int)__builtin_amdgcn_readlane((int)hi, (int)k) << 32);
+}
+
 // Span presence: few, long workgroups of 8 waves, so that a payload has at most
 // kSpanMasks masks and the encode tile kernel can form the palette from them itself
 // (palette_from_masks): no reduce launch between the two. A workgroup covers
@@ -126,14 +133,19 @@ constexpr unsigned int kSpanMasks = 256;
 constexpr unsigned int kSpanWaves = 8;
 constexpr unsigned int kSpanMaxShift = 7;  // 128 tiles: 64 chunks per wave, one per lane
 
-template <bool kIds>
+// kRuns: the run geometry with blocks of at least 1024 words. A chunk then lies in at
+// most two blocks, so a lane looks up two addresses per chunk, and a plane's last chunk
+// may hold fewer words (64 MB of 7680-word blocks, encode + decode: 71.3 us with masks per
+// tile and a reduce, 65.5 us so).
+template <bool kIds, bool kRuns>
 __global__ __launch_bounds__(kSpanWaves * kWave) void palette_presence_span(
     LaunchArgs a, EncodeGeom geo, unsigned int* masks, unsigned int span_shift) {
   __shared__ unsigned char s_seen[256];
   const unsigned int tid = threadIdx.x, lane = tid & (kWave - 1), wave = uniform(tid >> 6);
   const unsigned int span = group_index();
   const PayloadDesc d = a.p[find_slot_payload(a, span)];
-  const unsigned int half = (unsigned int)(((unsigned long long)d.block_count * geo.bw) >> 10);
+  const unsigned int plane_words = d.block_count * geo.bw;  // below 2^31
+  const unsigned int half = (plane_words + 1023) >> 10;     // chunks per plane
   const unsigned int per_plane = (half + 3) / 4;  // tiles
   // the span's tiles in chunks: a plane's last tile may hold fewer than four
   const unsigned int tile0 = (span - d.slot_group_begin) << span_shift;
@@ -151,22 +163,42 @@ __global__ __launch_bounds__(kSpanWaves * kWave) void palette_presence_span(
     const unsigned int plane = q >= half ? 1u : 0u;
     const unsigned int in_plane = (q - plane * half) << 10;
     const unsigned int j = div_u32(in_plane, geo.bw_magic, geo.bw);
-    const unsigned long long blk = kIds ? (unsigned long long)a.ids[d.ids_offset + j]
-                                        : a.block_start + j;
-    const unsigned long long off =
-        plane * a.plane_stride + blk * a.block_stride + (in_plane - j * geo.bw);
+    const unsigned int within = in_plane - j * geo.bw;
+    auto block_at = [&](unsigned int b) {
+      const unsigned long long blk = kIds ? (unsigned long long)a.ids[d.ids_offset + b]
+                                          : a.block_start + b;
+      return plane * a.plane_stride + blk * a.block_stride;
+    };
+    const unsigned long long off = block_at(j) + within;
     const unsigned int off_lo = (unsigned int)off, off_hi = (unsigned int)(off >> 32);
+    // run geometry: the same for the next block, and packed the chunk's words in the
+    // first block (1024 when it has them all) and its words in all
+    unsigned int next_lo = 0, next_hi = 0, ends = 0;
+    if (kRuns) {
+      const unsigned long long next =
+          block_at(min(j + 1, d.block_count - 1)) + within - geo.bw;
+      next_lo = (unsigned int)next;
+      next_hi = (unsigned int)(next >> 32);
+      ends = min(geo.bw - within, 1024u) | (min(plane_words - in_plane, 1024u) << 16);
+    }
     // chunks i and i + 1 (past the end the last one again: the same bytes)
     auto load = [&](u32x4 (&v)[4], unsigned int i) {
 #pragma unroll
       for (unsigned int c = 0; c < 2; ++c) {
         const unsigned int k = min(i + c, chunks - 1);
-        const unsigned long long at =
-            (unsigned int)__builtin_amdgcn_readlane((int)off_lo, (int)k) |
-            ((unsigned long long)(unsigned int)__builtin_amdgcn_readlane((int)off_hi, (int)k)
-             << 32);
-        v[2 * c] = load_stream16(a.kv + at + 8 * lane);
-        v[2 * c + 1] = load_stream16(a.kv + at + 512 + 8 * lane);
+        const unsigned long long at = lane_value(off_lo, off_hi, k);
+        if (kRuns) {
+          const unsigned long long next = lane_value(next_lo, next_hi, k);
+          const unsigned int e = (unsigned int)__builtin_amdgcn_readlane((int)ends, (int)k);
+          // (a run past the chunk's end is its first one again)
+          const unsigned int xa = 8 * lane < (e >> 16) ? 8 * lane : 0;
+          const unsigned int xb = 512 + 8 * lane < (e >> 16) ? 512 + 8 * lane : 0;
+          v[2 * c] = load_stream16(a.kv + (xa < (e & 0xFFFFu) ? at : next) + xa);
+          v[2 * c + 1] = load_stream16(a.kv + (xb < (e & 0xFFFFu) ? at : next) + xb);
+        } else {
+          v[2 * c] = load_stream16(a.kv + at + 8 * lane);
+          v[2 * c + 1] = load_stream16(a.kv + at + 512 + 8 * lane);
+        }
       }
     };
     auto mark = [&](const u32x4 (&v)[4]) {
@@ -688,21 +720,26 @@ long long launch_palette_encode(LaunchArgs& a, const EncodeGeom& g, Layout layou
   const dim3 block(kThreads);
   const bool tiles = layout != Layout::kGeneric;
   const dim3 grid(a.total_tiles);
-  const unsigned int shift = layout == Layout::kTile && !masks_given ? span_shift(a) : 0;
+  const bool runs = layout == Layout::kRuns;
+  const unsigned int shift =
+      !masks_given && (layout == Layout::kTile || (runs && g.bw >= 1024)) ? span_shift(a) : 0;
   if (shift != 0) {
     const dim3 spans(set_spans(a, shift)), threads(kSpanWaves * kWave);
-    if (a.ids)
-      palette_presence_span<true><<<spans, threads, 0, stream>>>(a, g, masks, shift);
-    else
-      palette_presence_span<false><<<spans, threads, 0, stream>>>(a, g, masks, shift);
-    if (long long rc = check("palette_presence")) return rc;
-    if (a.ids)
-      palette_encode_tile<true, kBits, From::kSpans><<<grid, block, 0, stream>>>(a, g, info, masks,
-                                                                                 shift);
-    else
-      palette_encode_tile<false, kBits, From::kSpans><<<grid, block, 0, stream>>>(a, g, info,
-                                                                                  masks, shift);
-    return check("palette_encode");
+    auto queue = [&](auto presence, auto encode) {
+      presence<<<spans, threads, 0, stream>>>(a, g, masks, shift);
+      if (long long rc = check("palette_presence")) return rc;
+      encode<<<grid, block, 0, stream>>>(a, g, info, masks, shift);
+      return check("palette_encode");
+    };
+    if (runs)
+      return a.ids ? queue(palette_presence_span<true, true>,
+                           palette_encode_tile<true, kBits, From::kSpans, true>)
+                   : queue(palette_presence_span<false, true>,
+                           palette_encode_tile<false, kBits, From::kSpans, true>);
+    return a.ids ? queue(palette_presence_span<true, false>,
+                         palette_encode_tile<true, kBits, From::kSpans>)
+                 : queue(palette_presence_span<false, false>,
+                         palette_encode_tile<false, kBits, From::kSpans>);
   }
   if (masks_given) {
     presence_groups = 0;
