@@ -125,6 +125,21 @@ long long kvq_splitzip_bf16_decode_fixed6_host_blocks(
     unsigned long long block_stride, const long long* host_block_ids,
     unsigned long long stream_ptr);
 
+/* The two host-table entries for the run geometry (block_words a multiple of 8 but not
+ * of 1024, dst and strides aligned for 16-byte runs); 0 for any other, or more blocks. */
+long long kvq_splitzip_bf16_decode_top16_host_runs(
+    unsigned long long src_ptr, unsigned long long encoded_bytes, unsigned long long dst_ptr,
+    unsigned long long count_words, unsigned long long block_count,
+    unsigned long long block_words, unsigned long long plane_stride,
+    unsigned long long block_stride, const long long* host_block_ids,
+    unsigned long long tables_ptr, unsigned long long stream_ptr);
+long long kvq_splitzip_bf16_decode_fixed6_host_runs(
+    unsigned long long src_ptr, unsigned long long encoded_bytes, unsigned long long dst_ptr,
+    unsigned long long count_words, unsigned long long block_count,
+    unsigned long long block_words, unsigned long long plane_stride,
+    unsigned long long block_stride, const long long* host_block_ids,
+    unsigned long long stream_ptr);
+
 /* ------------------------------------------------------------------------------
  * Additions: every request of one paged layer in one launch.
  *

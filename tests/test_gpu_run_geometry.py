@@ -112,6 +112,55 @@ def test_top16(sz, bw, kind):
     assert np.array_equal(got[:, recv[-1]], words_r if want[0] == 5 else np.zeros_like(words_r))
 
 
+@pytest.mark.parametrize("blocks", [2, 256, 257])
+@pytest.mark.parametrize("bw", [24, 1032, 1280])
+def test_dropin_block_table(sz, bw, blocks):
+    """Shuffled tables of up to 256 ids ride in the kernel arguments, longer ones in a
+    device copy: the drop-in decodes of both codecs restore the same words."""
+    print("[case] runs drop-in table", bw, blocks, flush=True)
+    rng = np.random.default_rng(bw + blocks)
+    pool = blocks + 5
+    values = rng.standard_normal((2, blocks, bw)).astype(np.float32)
+    words = (values.view(np.uint32) >> 16).astype(np.uint16)
+    ids = rng.permutation(pool)[:blocks].tolist()
+    if blocks == 2:
+        ids = [pool - 1, 0]
+    book = b""
+    for plane in range(2):
+        count = np.bincount((words[plane].reshape(-1) >> 7) & 0xFF, minlength=256)
+        book += bytes(sorted(range(256), key=lambda e: (-count[e], e))[:16])
+    source = to_gpu(words)
+    lib = sz._load()
+    tab = sz.top16_tables_for(book, source.device, torch)
+    buf = torch.zeros(4 * words.size + (1 << 20), dtype=torch.uint8, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    for codec in ("top16", "fixed6"):
+        size = sz.encode_top16(source, buf, 0, codebooks=book) if codec == "top16" else \
+            sz.encode_bf16(source, buf)
+        if not size:  # too short for fixed6 to be smaller
+            assert codec == "fixed6" and words.size < 300
+            continue
+        target = torch.zeros((2, pool, bw), dtype=torch.bfloat16, device="cuda")
+        payload = buf[:size]
+        got = sz.decode_top16(payload, target, ids, 2 * words.size, 0, codebooks=book) \
+            if codec == "top16" else sz.decode_fixed6(payload, target, ids, 2 * words.size)
+        assert got == 2 * words.size
+        restored = target.view(torch.int16).cpu().numpy().view(np.uint16)
+        assert np.array_equal(restored[:, ids], words), codec
+        rest = sorted(set(range(pool)) - set(ids))
+        assert not restored[:, rest].any()
+        # the entries' own rules: each takes its geometry and at most 256 blocks
+        table = np.array(ids, dtype=np.int64)
+        args = (payload.data_ptr(), size, target.data_ptr(), words.size, blocks, bw,
+                target.stride(0), target.stride(1), table.ctypes.data) + \
+            ((tab.data_ptr(),) if codec == "top16" else ()) + (stream,)
+        tile = getattr(lib, f"kvq_splitzip_bf16_decode_{codec}_host_blocks")
+        runs = getattr(lib, f"kvq_splitzip_bf16_decode_{codec}_host_runs")
+        assert tile(*args) == 0
+        assert runs(*args) == (2 * words.size if blocks <= 256 else 0)
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("bits", [6, 5])
 @pytest.mark.parametrize("bw", BLOCK_WORDS)
 def test_palette(sz, bw, bits):

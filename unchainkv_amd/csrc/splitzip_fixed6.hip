@@ -615,11 +615,11 @@ __global__ __launch_bounds__(kThreads) void palette_decode_tile(LaunchArgs a, En
 }
 
 // One request whose block table rides in the kernel arguments.
-template <int kBits>
+template <int kBits, bool kRuns>
 __global__ __launch_bounds__(kThreads) void palette_decode_tile_inline(LaunchArgs a,
                                                                        EncodeGeom geo,
                                                                        InlineBlocks table) {
-  palette_decode_tile_body<kBits, false>(a, geo, [&](const PlaneTile&, unsigned int j) {
+  palette_decode_tile_body<kBits, kRuns>(a, geo, [&](const PlaneTile&, unsigned int j) {
     return (unsigned long long)table.id[j];
   });
 }
@@ -785,13 +785,15 @@ long long launch_palette_decode(LaunchArgs& a, const EncodeGeom& g, Layout layou
                                 hipStream_t stream, const InlineBlocks* table) {
   const dim3 block(kThreads), grid(a.total_tiles);
   if (layout == Layout::kRuns) {
-    if (a.ids)
+    if (table)
+      palette_decode_tile_inline<kBits, true><<<grid, block, 0, stream>>>(a, g, *table);
+    else if (a.ids)
       palette_decode_tile<true, kBits, true><<<grid, block, 0, stream>>>(a, g);
     else
       palette_decode_tile<false, kBits, true><<<grid, block, 0, stream>>>(a, g);
   } else if (layout == Layout::kTile) {
     if (table)
-      palette_decode_tile_inline<kBits><<<grid, block, 0, stream>>>(a, g, *table);
+      palette_decode_tile_inline<kBits, false><<<grid, block, 0, stream>>>(a, g, *table);
     else if (a.ids)
       palette_decode_tile<true, kBits, false><<<grid, block, 0, stream>>>(a, g);
     else
@@ -828,7 +830,7 @@ long long palette_encode(LaunchArgs& a, const EncodeGeom& g, Layout layout,
                                               masks_given, stream);
 }
 
-// `table`: one request's block table in the kernel arguments (tile kernels only).
+// `table`: one request's block table in the kernel arguments (not the generic kernels).
 long long palette_decode(LaunchArgs& a, const EncodeGeom& g, Layout layout, hipStream_t stream,
                          int bits, const InlineBlocks* table = nullptr) {
   return bits == 6 ? launch_palette_decode<6>(a, g, layout, stream, table)
@@ -948,7 +950,8 @@ long long decode_blocks(unsigned long long src_ptr, unsigned long long encoded_b
                         unsigned long long plane_stride, unsigned long long block_stride,
                         unsigned long long block_start, unsigned long long block_ids_ptr,
                         unsigned long long stream_ptr, int bits,
-                        const long long* host_ids = nullptr) {
+                        const long long* host_ids = nullptr,
+                        Layout host_layout = Layout::kTile) {
   // kvq_splitzip_cuda.cu:351-357
   if (src_ptr == 0 || dst_ptr == 0 || count_words == 0 || block_count == 0 || block_words == 0 ||
       count_words != 2 * block_count * block_words)
@@ -971,10 +974,10 @@ long long decode_blocks(unsigned long long src_ptr, unsigned long long encoded_b
   const Layout layout =
       layout_of(dst_ptr, plane_stride, block_stride, block_words, count_words / 2);
   a.total_tiles = tiles_of(count_words);
-  // a host block table rides in the kernel arguments (chunk geometry only)
+  // a host block table rides in the kernel arguments (in the caller's geometry only)
   InlineBlocks table{};
   if (host_ids) {
-    if (layout != Layout::kTile || block_count > kInlineBlocks) return 0;
+    if (layout != host_layout || block_count > kInlineBlocks) return 0;
     for (unsigned long long j = 0; j < block_count; ++j) {
       if (host_ids[j] < 0 || host_ids[j] > 0xFFFFFFFFll) return 0;
       table.id[j] = (unsigned int)host_ids[j];
@@ -1017,6 +1020,18 @@ extern "C" long long kvq_splitzip_bf16_decode_fixed6_host_blocks(
   if (host_block_ids == nullptr) return 0;
   return decode_blocks(src_ptr, encoded_bytes, dst_ptr, count_words, block_count, block_words,
                        plane_stride, block_stride, 0, 0, stream_ptr, 6, host_block_ids);
+}
+
+extern "C" long long kvq_splitzip_bf16_decode_fixed6_host_runs(
+    unsigned long long src_ptr, unsigned long long encoded_bytes, unsigned long long dst_ptr,
+    unsigned long long count_words, unsigned long long block_count,
+    unsigned long long block_words, unsigned long long plane_stride,
+    unsigned long long block_stride, const long long* host_block_ids,
+    unsigned long long stream_ptr) {
+  if (host_block_ids == nullptr) return 0;
+  return decode_blocks(src_ptr, encoded_bytes, dst_ptr, count_words, block_count, block_words,
+                       plane_stride, block_stride, 0, 0, stream_ptr, 6, host_block_ids,
+                       Layout::kRuns);
 }
 
 // ---------------------------------------------------------------------------

@@ -869,8 +869,9 @@ __global__ __launch_bounds__(kThreads) void top16_decode_tile_inline(LaunchArgs 
 // of 12 requests with 7680-word blocks (6 heads of 80): the 16-word lanes of the
 // lanes kernels store and load 32-byte strides and realign their sections by
 // shuffles; encode + decode call 68.8 us with those, 58.1 us with runs.
-template <bool kIds>
-__global__ __launch_bounds__(kThreads) void top16_decode_runs(LaunchArgs a, EncodeGeom geo) {
+template <typename BlockOf>
+__device__ __forceinline__ void decode_runs(const LaunchArgs& a, const EncodeGeom& geo,
+                                            BlockOf block_of) {
   const unsigned int lane = threadIdx.x & (kWave - 1);
   const unsigned int wave = uniform(threadIdx.x >> 6);
   const PlaneTile t = plane_tile<kTileShift>(a, group_index());
@@ -892,7 +893,9 @@ __global__ __launch_bounds__(kThreads) void top16_decode_runs(LaunchArgs a, Enco
   const uint32_t code_b = load_stream4(pcode + second / 2 + 4 * lane);
   __builtin_amdgcn_sched_barrier(0);
   unsigned long long run_a, run_b;
-  run_sources<kIds>(a, t, geo, in_plane, lane, second, run_a, run_b);
+  run_offsets(geo, in_plane, t.blocks - 1, lane, second, [&](unsigned int j) {
+    return t.plane * a.plane_stride + block_of(t, j) * a.block_stride;
+  }, run_a, run_b);
   uint16_t* const dst_a = a.kv + run_a;
   uint16_t* const dst_b = a.kv + run_b;
   const u32x4 out_a = decode_run8(body_a, code_a, cb);
@@ -901,6 +904,20 @@ __global__ __launch_bounds__(kThreads) void top16_decode_runs(LaunchArgs a, Enco
   if (mode != 5) return;
   store_through16(dst_a, out_a);
   if (active_b) store_through16(dst_b, out_b);
+}
+
+template <bool kIds>
+__global__ __launch_bounds__(kThreads) void top16_decode_runs(LaunchArgs a, EncodeGeom geo) {
+  decode_runs(a, geo, [&](const PlaneTile& t, unsigned int j) {
+    return kIds ? (unsigned long long)t.ids[j] : a.block_start + j;
+  });
+}
+
+__global__ __launch_bounds__(kThreads) void top16_decode_runs_inline(LaunchArgs a, EncodeGeom geo,
+                                                                     InlineBlocks table) {
+  decode_runs(a, geo, [&](const PlaneTile&, unsigned int j) {
+    return (unsigned long long)table.id[j];
+  });
 }
 
 // Replaces the exponent of word w (0..1023) of this wave's chunk, held in run A
@@ -1534,7 +1551,7 @@ long long launch_encode(LaunchArgs& a, const EncodeGeom& g, const Plan& p, hipSt
 }
 
 // `table`: the request's block table in the kernel arguments (one payload on the
-// tile plan) instead of a.ids.
+// tile or run plan) instead of a.ids.
 long long launch_decode(LaunchArgs& a, const EncodeGeom& g, const Plan& p, hipStream_t stream,
                         const InlineBlocks* table = nullptr) {
   const dim3 block(kThreads);
@@ -1556,7 +1573,10 @@ long long launch_decode(LaunchArgs& a, const EncodeGeom& g, const Plan& p, hipSt
         hipLaunchKernelGGL(top16_decode_tile<false>, dim3(a.total_tiles), block, 0, stream, a, g);
       break;
     case Kernel::kRuns:
-      if (a.ids)
+      if (table)
+        hipLaunchKernelGGL(top16_decode_runs_inline, dim3(a.total_tiles), block, 0, stream, a, g,
+                           *table);
+      else if (a.ids)
         hipLaunchKernelGGL(top16_decode_runs<true>, dim3(a.total_tiles), block, 0, stream, a, g);
       else
         hipLaunchKernelGGL(top16_decode_runs<false>, dim3(a.total_tiles), block, 0, stream, a, g);
@@ -1681,15 +1701,15 @@ namespace unchainkv {
 namespace {
 
 // One payload's decode + scatter; the block table from block_ids_ptr (device),
-// host_ids (host, carried in the kernel arguments: tile plan only, else declined),
-// or neither (block_start + j).
+// host_ids (host, carried in the kernel arguments: plan `host_plan` only, else
+// declined), or neither (block_start + j).
 long long decode_top16_one(unsigned long long src_ptr, unsigned long long encoded_bytes,
                            unsigned long long dst_ptr, unsigned long long count_words,
                            unsigned long long block_count, unsigned long long block_words,
                            unsigned long long plane_stride, unsigned long long block_stride,
                            unsigned long long block_start, unsigned long long block_ids_ptr,
                            const long long* host_ids, unsigned long long tables_ptr,
-                           unsigned long long stream_ptr) {
+                           unsigned long long stream_ptr, Kernel host_plan = Kernel::kTile) {
   // Preconditions of kvq_splitzip_cuda.cu:423-432.
   if (src_ptr == 0 || dst_ptr == 0 || tables_ptr == 0 || count_words == 0 || block_count == 0 ||
       block_words == 0 || count_words != 2 * block_count * block_words)
@@ -1719,7 +1739,7 @@ long long decode_top16_one(unsigned long long src_ptr, unsigned long long encode
   a.total_tiles = host_payload_tiles(count_words, true, plan.tile_shift);
   InlineBlocks table{};
   if (host_ids) {
-    if (plan.kernel != Kernel::kTile || block_count > kInlineBlocks) return 0;
+    if (plan.kernel != host_plan || block_count > kInlineBlocks) return 0;
     for (unsigned long long j = 0; j < block_count; ++j) {
       if (host_ids[j] < 0 || host_ids[j] > 0xFFFFFFFFll) return 0;
       table.id[j] = (unsigned int)host_ids[j];
@@ -1757,6 +1777,18 @@ extern "C" long long kvq_splitzip_bf16_decode_top16_host_blocks(
   return decode_top16_one(src_ptr, encoded_bytes, dst_ptr, count_words, block_count, block_words,
                           plane_stride, block_stride, 0, 0, host_block_ids, tables_ptr,
                           stream_ptr);
+}
+
+extern "C" long long kvq_splitzip_bf16_decode_top16_host_runs(
+    unsigned long long src_ptr, unsigned long long encoded_bytes, unsigned long long dst_ptr,
+    unsigned long long count_words, unsigned long long block_count,
+    unsigned long long block_words, unsigned long long plane_stride,
+    unsigned long long block_stride, const long long* host_block_ids,
+    unsigned long long tables_ptr, unsigned long long stream_ptr) {
+  if (host_block_ids == nullptr) return 0;
+  return decode_top16_one(src_ptr, encoded_bytes, dst_ptr, count_words, block_count, block_words,
+                          plane_stride, block_stride, 0, 0, host_block_ids, tables_ptr,
+                          stream_ptr, Kernel::kRuns);
 }
 
 extern "C" long long kvq_splitzip_bf16_decode_top16(

@@ -54,6 +54,8 @@ _SIGNATURES = (
     # the host block table's address travels as a u64
     ("kvq_splitzip_bf16_decode_top16_host_blocks", [_U64] * 11, ctypes.c_longlong, False),
     ("kvq_splitzip_bf16_decode_fixed6_host_blocks", [_U64] * 10, ctypes.c_longlong, False),
+    ("kvq_splitzip_bf16_decode_top16_host_runs", [_U64] * 11, ctypes.c_longlong, False),
+    ("kvq_splitzip_bf16_decode_fixed6_host_runs", [_U64] * 10, ctypes.c_longlong, False),
     ("kvq_splitzip_last_error", [], ctypes.c_char_p, True),
     ("kvq_splitzip_top16_paged_workspace_bytes", [_U64, _U64P, _U64], _U64, False),
     ("kvq_splitzip_top16_paged_directory_bytes", [_U64, _U64P, _U64], _U64, False),
@@ -315,18 +317,26 @@ def _decode_layout(source, out, block_ids, raw_bytes, torch):
 def _decode_with_table(lib, host_name, device_name, block_ids, source, out, count_words,
                        block_words, stream, tail, torch):
     """Decode through a non-contiguous block table: in the kernel arguments when the
-    library takes the host list (up to HOST_TABLE_BLOCKS ids, tile geometry), else
-    from a device copy made asynchronously from pinned memory (recorded on the
+    library takes the host list (up to HOST_TABLE_BLOCKS ids; `host_name` for the tile
+    geometry, its ``_host_runs`` form for block words that are another multiple of
+    8), else from a device copy made asynchronously from pinned memory (recorded on the
     current stream). `tail` = the arguments after the table. Returns the C result,
     or None when no entry point is available."""
     common = (int(source.data_ptr()), int(source.numel()), int(out.data_ptr()), count_words,
               len(block_ids), block_words, int(out.stride(0)), int(out.stride(1)))
-    host_decode = getattr(lib, host_name, None)
-    if host_decode is not None and len(block_ids) <= HOST_TABLE_BLOCKS:
-        table = array.array("q", block_ids)
-        copied = host_decode(*common, table.buffer_info()[0], *tail, stream)
-        if copied != 0:
-            return copied
+    if len(block_ids) <= HOST_TABLE_BLOCKS:
+        table = None
+        for name in (host_name, host_name.replace("_host_blocks", "_host_runs")):
+            host_decode = getattr(lib, name, None)
+            if host_decode is None:
+                continue
+            if table is None:
+                table = array.array("q", block_ids)
+            copied = host_decode(*common, table.buffer_info()[0], *tail, stream)
+            if copied != 0:
+                return copied
+            if block_words % 1024 == 0:
+                break
     device_decode = getattr(lib, device_name, None)
     if device_decode is None:
         return None
