@@ -105,8 +105,8 @@ long long kvq_splitzip_bf16_decode_top16(
  * first, src/unchain_kv/splitzip_cuda.py:226-229). Up to 256 ids, each below 2^32,
  * travel in the kernel arguments, so no host-to-device copy precedes the launch;
  * the table is read before the call returns. Returns 0 (declined: use the
- * device-table entry) for more blocks or a geometry the tile kernels do not take
- * (block_words not a multiple of 1024, dst or strides off alignment). */
+ * device-table entry) for more blocks or a geometry the chunk tile kernels do not
+ * take (block_words not a multiple of 1024, dst or strides off alignment). */
 long long kvq_splitzip_bf16_decode_top16_host_blocks(
     unsigned long long src_ptr, unsigned long long encoded_bytes, unsigned long long dst_ptr,
     unsigned long long count_words, unsigned long long block_count,
