@@ -1,9 +1,10 @@
 """Presence spans of the palette encode (a workgroup's mask covers 2^k tiles, the encode
-forms the palette from a payload's masks): span sizes on both sides of the rule, spans
-that cross from the K to the V plane, planes that end inside a tile, and high bytes
-present in a single word (a request's first, last, plane-border or a random one), which
-a span that skipped a chunk would lose. Payloads byte for byte with the oracle's, a
-payload with one high byte too many as 255 alone, and the decode word for word."""
+forms the palette from a payload's masks): every span length, spans that cross from the K
+to the V plane, planes that end inside a tile, and high bytes present in a single word,
+which a span that skipped a chunk would lose. Short requests: payloads byte for byte with
+the oracle's, a payload with one high byte too many as 255 alone, and the decode word for
+word. Long ones: palette and decoded words, compared on the GPU. And the cost: a layer
+takes no longer in many short requests than in few long ones."""
 
 import numpy as np
 import pytest
@@ -14,12 +15,12 @@ torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
 
 CASES = {
-    # blocks of 1024 words (four per tile and plane) of each request: at most 512 tiles
-    # -> spans of two tiles
+    # blocks of 1024 words (four per tile and plane) of each request. Spans of eight tiles
+    # for requests of 512 tiles and less,
     "two_tiles": [1, 2, 3, 4, 5, 9, 1023, 1024],
-    # 514 tiles at most -> four tiles, with enough spans in all
+    # of 514 tiles beside short ones,
     "four_tiles": [1027] * 2 + [1, 6, 15],
-    # 514 tiles alone -> the tile presence pass and its reduce
+    # and alone
     "tile_pass": [1027],
     # 2050 tiles at most -> sixteen tiles
     "sixteen_tiles": [4099] * 2 + [37],
@@ -88,3 +89,86 @@ def test_spans(sz, bw, name, bits):
     for r, (t, u) in enumerate(zip(send, recv)):
         want = words[:, t] if r != overflow else np.zeros_like(words[:, t])
         assert np.array_equal(restored[:, u], want), r
+
+
+# (block words, blocks, log2 of the tiles per span; 0: more than 32768 tiles, the tile
+# presence pass and its reduce)
+LONG = [(1024, 4096, 3), (1024, 8192, 4), (1024, 16384, 5), (1024, 32768, 6), (1024, 32801, 7),
+        (1024, 65503, 7), (2048, 32803, 0), (1032, 8200, 5), (3848, 8601, 6), (1032, 32603, 7)]
+
+
+@pytest.mark.parametrize("bw,blocks,shift", LONG)
+def test_long_spans(sz, bw, blocks, shift):
+    print("[case] long palette spans", bw, blocks, shift, flush=True)
+    half = bw * blocks
+    chunks = -(-half // 1024)              # of a plane
+    tiles = 2 * -(-half // 4096)
+    if shift:
+        assert tiles <= 256 << shift and (shift == 3 or tiles > 256 << (shift - 1))
+    else:
+        assert tiles > 256 << 7
+    g = torch.Generator(device="cuda")
+    g.manual_seed(bw + blocks)
+    low = torch.randint(0, 256, (2, half), generator=g, device="cuda", dtype=torch.int32)
+    high = torch.randint(0x50, 0x5C, (2, half), generator=g, device="cuda", dtype=torch.int32)
+    # single words of other high bytes: in the first, middle and last chunks that a wave
+    # of a span walks (every eighth chunk of 4 << shift), and at the planes' ends
+    walk = 4 << (shift or 3)
+    places = [(0, 0), (0, half - 1), (1, 0), (1, half - 1), (0, (chunks - 1) * 1024)]
+    for k, lane in enumerate((0, 1, 2, 3, walk // 16, walk // 8 - 2, walk // 8 - 1)):
+        for span in (1, max(1, chunks // walk // 2), chunks // walk - 1):
+            chunk = span * walk + 8 * lane + k
+            places.append((k % 2, min(chunk * 1024 + 37 * k + 512 * (span % 2), half - 1)))
+    singles = [b for b in range(256) if not 0x50 <= b < 0x5C][:len(places)]
+    for (plane, at), b in zip(places, singles):
+        high[plane, at] = b
+    words = (((high << 8) | low) & 0xFFFF).to(torch.int16).view(2, blocks, bw)
+    present = torch.unique(high).tolist()
+    assert len(present) <= 64
+    del low, high
+    ids = torch.randperm(blocks, generator=g, device="cuda")
+    layer = torch.empty_like(words)
+    layer[:, ids] = words
+    batch = sz.PagedBatch([ids.tolist()], bw, "cuda")
+    offsets, sizes, _ = batch.palette_layout(6)
+    out = batch.new_palette_buffer(6)
+    assert sz.encode_bf16_paged(layer.view(torch.bfloat16), batch, out,
+                                batch.new_palette_workspace(), 6) == sizes[0]
+    head = out[offsets[0]:offsets[0] + 65].tolist()
+    assert head[0] == 3 and head[1:] == present + [0] * (64 - len(present))
+    target = torch.zeros_like(words)
+    recv = sz.PagedBatch([list(range(blocks))], bw, "cuda")
+    assert sz.decode_bf16_paged(out, offsets, sizes, target.view(torch.bfloat16), recv, 6) == \
+        batch.total_raw_bytes
+    assert torch.equal(target, words)
+
+
+def time_of(call, n=20):
+    """Median time of a call among n (us)."""
+    times = []
+    for _ in range(7):
+        begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        begin.record()
+        for _ in range(n):
+            call()
+        end.record()
+        torch.cuda.synchronize()
+        times.append(begin.elapsed_time(end) / n * 1e3)
+    return sorted(times)[3]
+
+
+def test_many_requests_cost_no_more_than_few(sz):
+    """128 MiB in 8 and in 64 requests: 70 and 67 us; with spans of one or two chunks per
+    wave the 64 requests took 100 us. A quarter of room for noise."""
+    bw, blocks = 1024, 32768
+    layer = torch.randn((2, blocks, bw), device="cuda").to(torch.bfloat16)
+    times = []
+    for requests in (8, 64):
+        per = blocks // requests
+        batch = sz.PagedBatch([list(range(r * per, (r + 1) * per)) for r in range(requests)], bw,
+                              "cuda")
+        out, workspace = batch.new_palette_buffer(6), batch.new_palette_workspace()
+        assert sz.encode_bf16_paged(layer, batch, out, workspace, 6)
+        times.append(time_of(lambda: sz.encode_bf16_paged(layer, batch, out, workspace, 6)))
+    print("[case] fixed6 encode in 8 and 64 requests", times, flush=True)
+    assert times[1] <= 1.25 * times[0], times

@@ -120,7 +120,7 @@ __device__ __forceinline__ unsigned long long lane_value(unsigned int lo, unsign
 
 // Span presence: few, long workgroups of 8 waves, so that a payload has at most
 // kSpanMasks masks and the encode tile kernel can form the palette from them itself
-// (palette_from_masks): no reduce launch between the two. A workgroup covers
+// (or_masks): no reduce launch between the two. A workgroup covers
 // 2^span_shift consecutive tiles of a payload, a wave every eighth 1024-word chunk of
 // them. Its lanes first look up one chunk's address each (one round trip for all block
 // ids); the walk then has two batches of two chunks in flight and no dependent load.
@@ -680,20 +680,23 @@ unsigned int tiles_in(const LaunchArgs& a, unsigned int r) {
   return (r + 1 < a.payload_count ? a.p[r + 1].tile_begin : a.total_tiles) - a.p[r].tile_begin;
 }
 
-// log2 of the tiles per presence span, 0 for the tile presence pass and its reduce. The
-// spans are the shortest with which no payload has more than kSpanMasks of them (at
-// least two tiles: one chunk per wave), as long as they are short or enough of them
-// to keep the memory busy: below three quarters of a workgroup per CU the pass takes
-// longer than the reduce launch it saves (two requests of 11 MB: 32.1 us both ways).
-constexpr unsigned int kSpanFill = 192;
+// log2 of the tiles per presence span, 0 for the tile presence pass and its reduce (a
+// payload of more than 256 MiB). The spans are the shortest of at least eight tiles with
+// which no payload has more than kSpanMasks of them. Eight tiles give a wave four chunks,
+// the two batches it keeps in flight; shorter spans are workgroups that mostly start and
+// drain. Encode of 64 requests, spans of two / four / eight / sixteen tiles against masks
+// per tile and a reduce: 64 MB 59.0 / 46.5 / 39.2 / 38.8 and 43.8 us, 128 MB 108 / 82 /
+// 69 / 68 and 75 us, 240 MB 192 / 146 / 123 / 122 and 127 us; one request of 1 MB, 16 MB
+// and 64 MB (spans of 8, 8 and 32 tiles, 16 to 256 workgroups) 12.3, 15.2 and 38.7 us
+// against 16.7, 19.0 and 46.9.
+constexpr unsigned int kSpanMinShift = 3;
 
 unsigned int span_shift(const LaunchArgs& a) {
   unsigned int most = 0;
   for (unsigned int r = 0; r < a.payload_count; ++r) most = std::max(most, tiles_in(a, r));
-  unsigned int shift = 1;
+  unsigned int shift = kSpanMinShift;
   while (shift <= kSpanMaxShift && ((most + (1u << shift) - 1) >> shift) > kSpanMasks) ++shift;
-  if (shift > kSpanMaxShift) return 0;
-  return shift == 1 || (a.total_tiles >> shift) >= kSpanFill ? shift : 0;
+  return shift <= kSpanMaxShift ? shift : 0;
 }
 
 // Sets each payload's first span (slot_group_begin); the number of spans.
