@@ -91,8 +91,7 @@ __global__ __launch_bounds__(kThreads) void palette_presence_tile(LaunchArgs a, 
       // (a lane without a second run reads its first one twice: the same mask)
       unsigned long long run_a, run_b;
       run_sources<kIds>(a, t, geo, in_plane, lane, active_b ? 512u : 0u, run_a, run_b);
-      v0 = load_stream16(a.kv + run_a);
-      v1 = load_stream16(a.kv + run_b);
+      load_runs16(geo, a.kv + run_a, a.kv + run_b, v0, v1);
     } else {
       const uint16_t* src = a.kv + wave_source<kIds>(a, t, geo, in_plane);
       v0 = load_stream16(src + 8 * lane);
@@ -430,8 +429,7 @@ __global__ __launch_bounds__(kThreads) void palette_encode_tile(LaunchArgs a, En
     if (active) {
       unsigned long long run_a, run_b;
       run_sources<kIds>(a, t, geo, in_plane, lane, active_b ? 512u : 0u, run_a, run_b);
-      v0 = load_stream16(a.kv + run_a);
-      v1 = load_stream16(a.kv + run_b);
+      load_runs16(geo, a.kv + run_a, a.kv + run_b, v0, v1);
     }
     x[0] = v0.x; x[1] = v0.y; x[2] = v0.z; x[3] = v0.w;
     x[4] = v1.x; x[5] = v1.y; x[6] = v1.z; x[7] = v1.w;
@@ -590,6 +588,7 @@ __device__ __forceinline__ void palette_decode_tile_body(const LaunchArgs& a,
   __syncthreads();
   if (mode != P::kMode || !active) return;  // the reference leaves other payloads untouched
   const unsigned char* stage = reinterpret_cast<const unsigned char*>(s_code) + wave * kWaveCodeBytes;
+  u32x4 words[2];  // run geometry: both runs' words
 #pragma unroll
   for (int run = 0; run < 2; ++run) {
     const unsigned long long bits = unstage_run<kBits>(stage, kBits * (run * 64 + lane));
@@ -603,8 +602,13 @@ __device__ __forceinline__ void palette_decode_tile_body(const LaunchArgs& a,
       const uint32_t h1 = s_pal[(bits >> (kBits * (2 * k + 1))) & kMask];
       out[k] = (lo & 0xFF) | (h0 << 8) | ((lo >> 8) << 16) | (h1 << 24);
     }
-    if (run == 0 || active_b) store_through16(dst[run], u32x4{out[0], out[1], out[2], out[3]});
+    const u32x4 v = {out[0], out[1], out[2], out[3]};
+    if (kRuns)
+      words[run] = v;
+    else
+      store_through16(dst[run], v);
   }
+  if (kRuns) store_runs16(geo, dst[0], words[0], dst[1], words[1], active_b);
 }
 
 template <bool kIds, int kBits, bool kRuns>

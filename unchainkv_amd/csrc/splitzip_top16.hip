@@ -30,8 +30,8 @@
 //       place escapes in ascending order, write the header (the tile kernel
 //       zeroes the escape slots of its span).
 //   top16_decode_tile / top16_decode_runs / top16_decode_lanes / top16_decode_generic
-//       decode + scatter for the tile geometry, the run geometry, 16-word lanes (code
-//       tables or planes past the tile kernels' limits), any geometry.
+//       decode + scatter for the tile geometry, the run geometry, 16-word lanes (short
+//       blocks, and code tables or planes past the tile kernels' limits), any geometry.
 // Global memory takes unaligned vector accesses (the code object's unaligned
 // access mode), so a payload's sections need no alignment: the reference
 // connector's payloads start at a buffer's first byte, their body at byte 5.
@@ -663,8 +663,7 @@ __global__ __launch_bounds__(kThreads) void top16_encode_tile(LaunchArgs a, Enco
       // (a lane without a second run reads its first one twice)
       unsigned long long run_a, run_b;
       run_sources<kIds>(a, t, geo, in_plane, lane, active_b ? 512u : 0u, run_a, run_b);
-      v0 = load_stream16(a.kv + run_a);
-      v1 = load_stream16(a.kv + run_b);
+      load_runs16(geo, a.kv + run_a, a.kv + run_b, v0, v1);
     }
     x[0] = v0.x; x[1] = v0.y; x[2] = v0.z; x[3] = v0.w;
     x[4] = v1.x; x[5] = v1.y; x[6] = v1.z; x[7] = v1.w;
@@ -868,7 +867,7 @@ __global__ __launch_bounds__(kThreads) void top16_decode_tile_inline(LaunchArgs 
 // The same over the run geometry, with a destination per lane and run. A 65.6 MB layer
 // of 12 requests with 7680-word blocks (6 heads of 80): the 16-word lanes of the
 // lanes kernels store and load 32-byte strides and realign their sections by
-// shuffles; encode + decode call 68.8 us with those, 58.1 us with runs.
+// shuffles; encode + decode call 68.8 us with those, 54.6 us with runs.
 template <typename BlockOf>
 __device__ __forceinline__ void decode_runs(const LaunchArgs& a, const EncodeGeom& geo,
                                             BlockOf block_of) {
@@ -902,8 +901,7 @@ __device__ __forceinline__ void decode_runs(const LaunchArgs& a, const EncodeGeo
   const u32x4 out_b = decode_run8(body_b, code_b, cb);
   asm volatile("" ::"v"(out_a), "v"(out_b), "v"(dst_a), "v"(dst_b));
   if (mode != 5) return;
-  store_through16(dst_a, out_a);
-  if (active_b) store_through16(dst_b, out_b);
+  store_runs16(geo, dst_a, out_a, dst_b, out_b, active_b);
 }
 
 template <bool kIds>
@@ -1418,7 +1416,16 @@ Plan make_plan(bool geometry_fast, bool tile_ok, bool runs_ok, bool sequential) 
   return p;
 }
 
-// Decode tiles every payload per plane.
+// Decode tiles every payload per plane. Short blocks that are a multiple of 16 words but
+// not of 64 keep the lanes kernel: it needs half the block ids, and where every line is
+// shared between blocks its stores reach as far. 64 MB in 64 requests with shuffled
+// tables, runs against lanes: 51.8 / 37.9 us (16-word blocks), 35.1 / 30.6 us (48), 30.7 /
+// 28.9 us (80), 28.2 / 27.9 us (144), 27.4 / 27.6 us (176), 26.3 / 26.7 us (224). A host
+// table rides in the kernel arguments for the run kernel only (at most 256 such blocks).
+bool short_lane_blocks(unsigned long long block_words) {
+  return block_words % 16 == 0 && block_words % 64 != 0 && block_words < 160;
+}
+
 Plan make_decode_plan(bool geometry_fast, bool tile_ok, bool runs_ok) {
   Plan p = make_plan(geometry_fast, tile_ok, runs_ok, false);
   p.per_plane = true;
@@ -1734,7 +1741,8 @@ long long decode_top16_one(unsigned long long src_ptr, unsigned long long encode
   const bool small = tables_ptr % 4 == 0 && (count_words >> 1) < kTilePlaneLimit;
   const Plan plan =
       make_decode_plan(geometry_fast, small && block_words % 1024 == 0,
-                       small && run_geometry(dst_ptr, plane_stride, block_stride, block_words));
+                       small && (host_ids || !short_lane_blocks(block_words)) &&
+                           run_geometry(dst_ptr, plane_stride, block_stride, block_words));
   apply_plan(a, plan);
   a.total_tiles = host_payload_tiles(count_words, true, plan.tile_shift);
   InlineBlocks table{};
@@ -2138,7 +2146,8 @@ extern "C" long long kvq_splitzip_bf16_decode_top16_paged(
   const bool small = tables_ptr % 4 == 0 && max_plane < kTilePlaneLimit;
   const Plan plan =
       make_decode_plan(paged_fast(pg), small && block_words % 1024 == 0,
-                       small && run_geometry(kv_ptr, plane_stride, block_stride, block_words));
+                       small && !short_lane_blocks(block_words) &&
+                           run_geometry(kv_ptr, plane_stride, block_stride, block_words));
   const unsigned long long dir_tiles =
       kvq_splitzip_top16_paged_directory_bytes(block_words, block_offsets, payload_count) /
       kDirBytesPerTile;

@@ -728,8 +728,7 @@ __device__ __forceinline__ void load_runs(const TileArgs<kMax>& a, const TilePay
   if (kRuns) {
     unsigned long long run_a, run_b;
     run_sources(a, d, (unsigned int)c, lane, r.at[1] - r.at[0], run_a, run_b);
-    v0 = load_stream16(a.kv + run_a);
-    v1 = load_stream16(a.kv + run_b);
+    load_runs16(a.geo, a.kv + run_a, a.kv + run_b, v0, v1);
   } else {
     const uint16_t* src = a.kv + chunk_source(a, d, n, c);
     v0 = load_stream16(src + r.at[0]);
@@ -1021,8 +1020,12 @@ __global__ __launch_bounds__(kThreads) void torchop_decode_tile(TileArgs<kMax> a
   }
   // write-through stores after the last load (the compiler's waits do not see them)
   asm volatile("" ::"v"(o[0]), "v"(o[1]), "v"(dst[0]), "v"(dst[1]));
-  store_through16(dst[0], o[0]);
-  if (!kRuns || runs.active_b) store_through16(dst[1], o[1]);
+  if (kRuns) {
+    store_runs16(a.geo, dst[0], o[0], dst[1], o[1], runs.active_b);
+  } else {
+    store_through16(dst[0], o[0]);
+    store_through16(dst[1], o[1]);
+  }
 }
 
 }  // namespace
