@@ -24,7 +24,7 @@ def sz():
     return splitzip_cuda
 
 
-def make_batch(sz, kv_heads, contexts, seed):
+def make_batch(sz, kv_heads, contexts, seed, edit=None):
     from unchainkv_amd import workloads
 
     shape = workloads.Shape(layers=1, kv_heads=kv_heads, head_dim=HEAD_DIM)
@@ -32,6 +32,8 @@ def make_batch(sz, kv_heads, contexts, seed):
     kv = workloads.make_kv_layer(torch, shape, sum(blocks), seed=seed, layer=0, device="cuda",
                                  outlier_rate=0.001)
     tables = workloads.random_block_tables(torch, sum(blocks), blocks, seed=seed)
+    if edit:
+        edit(kv, tables)
     books = workloads.fit_codebook(torch, kv, tables)
     batch = sz.PagedBatch(tables, shape.block_words, "cuda")
     payloads = batch.new_payload_buffer()
@@ -86,3 +88,49 @@ def test_workspace_of_the_largest_batch_serves_smaller_ones(sz):
     for heads_rows in (sizes[:5], sizes[5:]):
         for column in zip(*heads_rows):
             assert list(column) == sorted(column)
+
+
+@pytest.mark.parametrize("kv_heads,context", [(8, 1500), (1, 4000), (3, 700)])
+@pytest.mark.parametrize("first,count", [(0, 16), (0, 128), (192, 64), (256, 128)])
+@pytest.mark.parametrize("value", [float("nan"), float("-inf")])
+def test_keys_that_are_not_finite(sz, kv_heads, context, first, count, value):
+    """A NaN in the keys of a head makes its rows NaN, also where the NaN tokens fill whole
+    ranges and splits; tokens whose scores are all -inf have no weight. Other heads keep
+    their results."""
+    print("[case] attention not finite", kv_heads, context, first, count, value, flush=True)
+    head = kv_heads // 2
+
+    def edit(kv, tables):
+        for t in range(first, first + count):
+            kv[0, tables[0][t // 16], t % 16, head, 5] = value
+
+    kv, tables, books, batch, payloads, q = make_batch(sz, kv_heads, [context], 11, edit)
+    q[:, :, 5] = q[:, :, 5].abs() + 0.5
+    assert int(payloads[batch.out_offsets[0]]) == 5
+    out = sz.decode_attention_top16(q, payloads, batch.out_offsets, [context], kv_heads,
+                                    codebooks=books)
+    got = out[0].double()
+    ref = reference(kv, tables[0], context, q[0], kv_heads)
+    rows = range(4 * head, 4 * head + 4)
+    if value != value:
+        assert torch.isnan(ref[rows]).all() and torch.isnan(got[rows]).all()
+        keep = [r for r in range(4 * kv_heads) if r not in rows]
+        got, ref = got[keep], ref[keep]
+    if len(got):
+        err, scale = (got - ref).abs().amax(dim=-1), ref.abs().amax(dim=-1).clamp_min(1e-6)
+        assert (err <= TOL * scale).all(), float((err / scale).max())
+
+
+def test_repeated_calls_give_the_same_bits(sz):
+    """Whatever the workspace and the output held before."""
+    contexts = [1, 300, 2113, 9000]
+    kv, tables, books, batch, payloads, q = make_batch(sz, 2, contexts, 3)
+    need = sz.decode_attention_workspace_bytes(len(contexts), 2, max(contexts))
+    bits = []
+    for fill in (0, 255, 0x7F):
+        workspace = torch.full((need,), fill, dtype=torch.uint8, device="cuda")
+        out = torch.full_like(q, float("nan"))
+        assert sz.decode_attention_top16(q, payloads, batch.out_offsets, contexts, 2,
+                                         codebooks=books, out=out, workspace=workspace) is out
+        bits.append(out.view(torch.int16).clone())
+    assert torch.equal(bits[0], bits[1]) and torch.equal(bits[0], bits[2])

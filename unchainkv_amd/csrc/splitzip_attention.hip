@@ -79,6 +79,11 @@ constexpr int kPartial = kHeadDim + 2;      // m, l, acc[128] per (split, query 
 // Context splits of one sequence at most: four batches of kCombineParts *
 // kCombineBatch partials in the combine kernel.
 constexpr unsigned int kMaxSplits = 256;
+// Running max before any token: the lowest float, not -inf, so that a range whose scores
+// are all -inf has weights exp2(-inf) = 0 and one whose scores are all NaN keeps a NaN sum
+// that reaches the output. (With -inf both gave NaN sums, and the merges took a max of
+// -inf for a range without tokens: a NaN that filled a whole split was left out.)
+constexpr float kNoMax = -3.402823466e38f;
 constexpr int kCheck = 8;                   // escape-order pairs per thread held through the walk
 // Independent accumulator chains of the PV product: one chain keeps the kernel at
 // 125 VGPRs (4 waves per SIMD); two reached 128 with a spill and ran 1 us slower.
@@ -391,7 +396,7 @@ __device__ __forceinline__ void attend_step(const RawShare& cur, unsigned int ts
   }
   float mloc = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
   mloc = max_over_lane_groups(mloc);
-  const float m_new = fmaxf(w.m_run, mloc);  // finite: every step holds a token
+  const float m_new = fmaxf(w.m_run, mloc);
   if (__ballot(m_new > w.m_run) & 0xFull) {
     // a head's max moved: rescale its sum share and its acc row
     const float alpha = __builtin_amdgcn_exp2f(w.m_run - m_new);
@@ -518,7 +523,7 @@ top16_attention_split(AttnArgs a) {
   }
 
   WaveWalk w;
-  w.m_run = -INFINITY;
+  w.m_run = kNoMax;
   w.l_run = 0.f;
 #pragma unroll
   for (int k = 0; k < 2 * kPvChains; ++k) w.acc[k] = f32x4{0, 0, 0, 0};
@@ -639,7 +644,7 @@ top16_attention_split(AttnArgs a) {
     if (hm < hkv) {
       const float* src[kRanges];
       float mr[kRanges];
-      float big = -INFINITY;
+      float big = kNoMax;
 #pragma unroll
       for (int r = 0; r < kRanges; ++r) {
         src[r] = sm + ((m * kRanges + r) * kGroup + j) * kPartial;
@@ -649,15 +654,13 @@ top16_attention_split(AttnArgs a) {
       float l_sum = 0.f, o[kVals];
 #pragma unroll
       for (int k = 0; k < kVals; ++k) o[k] = 0.f;
-      if (big != -INFINITY) {
-        // a wave with no tokens has m = -inf and weight 0
+      // (a wave without tokens has sums of 0)
 #pragma unroll
-        for (int r = 0; r < kRanges; ++r) {
-          const float wr = mr[r] == -INFINITY ? 0.f : exp2f(mr[r] - big);
-          l_sum += src[r][1] * wr;
+      for (int r = 0; r < kRanges; ++r) {
+        const float wr = exp2f(mr[r] - big);
+        l_sum += src[r][1] * wr;
 #pragma unroll
-          for (int k = 0; k < kVals; ++k) o[k] += src[r][2 + d0 + k] * wr;
-        }
+        for (int k = 0; k < kVals; ++k) o[k] += src[r][2 + d0 + k] * wr;
       }
       float* dst = a.partial +
                    (((unsigned long long)item * hkv + hm) * kGroup + j) * kPartial;
@@ -717,7 +720,7 @@ __global__ __launch_bounds__(kHeadDim * kParts) void top16_attention_combine(Att
     float top = big;
 #pragma unroll
     for (int k = 0; k < kCombineBatch; ++k) top = fmaxf(top, m[k]);
-    if (top == -INFINITY) continue;  // no split of this batch holds a token
+    if (top == -INFINITY) continue;  // rejected splits only
     if (big != -INFINITY && top != big) {
       const float r = exp2f(big - top);
       num *= r;
@@ -726,7 +729,7 @@ __global__ __launch_bounds__(kHeadDim * kParts) void top16_attention_combine(Att
     big = top;
 #pragma unroll
     for (int k = 0; k < kCombineBatch; ++k) {
-      if (m[k] == -INFINITY) continue;  // a split with no tokens
+      if (m[k] == -INFINITY) continue;  // past the last split
       const float wgt = exp2f(m[k] - big);
       den += l[k] * wgt;
       num += v[k] * wgt;
