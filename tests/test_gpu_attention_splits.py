@@ -134,3 +134,25 @@ def test_repeated_calls_give_the_same_bits(sz):
                                          codebooks=books, out=out, workspace=workspace) is out
         bits.append(out.view(torch.int16).clone())
     assert torch.equal(bits[0], bits[1]) and torch.equal(bits[0], bits[2])
+
+
+@pytest.mark.parametrize("kv_heads,contexts,least,most", [
+    (8, [256] * 32, 128, 256),       # 2 to 4 workgroups per CU: 16 us; one per CU: 18 us
+    (8, [8192] * 32, 256, 256),      # 4 per CU: 144 us; 3: 150 us, 2: 164 us
+    (1, [16384], 64, 128),           # 2 to 4 steps per range: 14 to 15 us; 1: 16.7 us
+    (8, [32768], 96, 192),           # 2 or 3 per CU: 34 us; 1: 39 us, 4: 41 us
+])
+def test_number_of_splits(sz, kv_heads, contexts, least, most):
+    """The splits a launch takes (partials written to the workspace), within those that
+    measured best."""
+    tokens = sum(contexts)
+    kv, tables, books, batch, payloads, q = make_batch(sz, kv_heads, contexts, 5)
+    need = sz.decode_attention_workspace_bytes(len(contexts), kv_heads, max(contexts))
+    workspace = torch.full((need,), 0x7E, dtype=torch.uint8, device="cuda")
+    assert sz.decode_attention_top16(q, payloads, batch.out_offsets, contexts, kv_heads,
+                                     codebooks=books, workspace=workspace) is not None
+    # a partial starts with its running max, never the filler
+    maxima = workspace.view(torch.int32)[::4 * (HEAD_DIM + 2)]
+    written = int((maxima != 0x7E7E7E7E).sum())
+    print("[case] attention splits", kv_heads, tokens, written / kv_heads, flush=True)
+    assert written % kv_heads == 0 and least <= written // kv_heads <= most

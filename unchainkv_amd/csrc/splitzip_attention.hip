@@ -825,9 +825,10 @@ Shape group_shape(unsigned long long kv_heads) {
 }
 
 // Splits of all sequences of a launch together, at most: two rounds of the resident
-// workgroups and one split per sequence, and no more than one step per wave. Grows
-// with each argument, so a workspace made for the largest batch and context serves
-// the smaller ones.
+// workgroups and one split per sequence, and no more than one step per wave. Grows with
+// the sequences and the context at a given number of kv heads, so that a workspace made
+// for the largest batch and context serves the smaller ones. (Between head counts it goes
+// up and down with the groups: a workspace is sized for its own.)
 unsigned long long max_launch_splits(unsigned long long sequences, unsigned long long kv_heads,
                                      unsigned long long max_ctx) {
   const Shape sh = group_shape(kv_heads);
@@ -836,56 +837,81 @@ unsigned long long max_launch_splits(unsigned long long sequences, unsigned long
                   2 * residency().cus * residency().per_cu / sh.groups + sequences);
 }
 
-// Splits of all sequences together with at most `per_split` tokens in each.
-unsigned long long count_splits(const unsigned long long* ctx, unsigned int count,
-                                unsigned int per_split) {
-  unsigned long long splits = 0;
-  for (unsigned int r = 0; r < count; ++r) splits += ((unsigned int)ctx[r] + per_split - 1) / per_split;
-  return splits;
+// Splits of all sequences together with at most `per_split` tokens in each, from
+// half[r] = the sequence's tokens - 0.5: half * (1 / per_split) is never within its
+// rounding error of a whole number (tokens < 2^24), so that truncation gives
+// (tokens - 1) / per_split exactly, several sequences per instruction.
+unsigned long long count_splits(const double* half, unsigned int count, unsigned int per_split) {
+  const double inverse = 1.0 / per_split;
+  int more = 0;
+  for (unsigned int r = 0; r < count; ++r) more += (int)(half[r] * inverse);
+  return (unsigned long long)more + count;
 }
 
-// Cost of one round of w workgroups per CU whose longest range has s steps, in
-// hundredths of a microsecond: kRoundCost + w * kGroupCost + s * kStepCost[w]. A step
-// of more workgroups takes longer (they share the CU's LDS and the memory), but less
-// than in proportion, and more workgroups pay more start-ups, so that few steps in
-// all are best spread thinly. Fitted to 32 sequences of 8192 tokens, 8 kv heads, at
-// 1, 2, 3 and 4 workgroups per CU: 254, 168, 152 and 146 us per call (128, 64, 43 and
-// 32 steps); one sequence of 32768 tokens: 40, 35, 37 and 41 us (16, 8, 6 and 4); 64
-// sequences of 128 to 32768 tokens, 1 kv head: 68, 45.5, 45 and 47 us.
-constexpr unsigned long long kStepCost[] = {0, 193, 248, 326, 410};
-constexpr unsigned long long kRoundCost = 400, kGroupCost = 350;
+// Time of a launch of `wgs` workgroups whose longest range has `steps` steps, in
+// hundredths of a microsecond, up to a constant: whole rounds of the resident workgroups
+// and a last one of w per CU, each w * kGroupCost (start-up) + steps * (kStepCost[w], for
+// workgroups that share a CU, + kShareCost per workgroup and CU of the chip, for all that
+// share the memory), and the merge: a pass per 64 splits of a sequence, and every split's
+// partials. Fitted by least squares to 6000 timings of 686 batches (1 to 8 kv heads, 1 to
+// 64 sequences, equal and mixed contexts of 16 to 32768 tokens, KV from memory) over their
+// step counts; the step count it chooses is 0.4 % above the best one on average. Examples,
+// us at 1 / 2 / 3 / 4 workgroups per CU: 32 sequences of 8192 tokens, 8 heads 251 / 164 /
+// 147 / 143; one of 32768 39 / 32 / 35 / 41.
+constexpr unsigned long long kStepCost[] = {0, 148, 152, 181, 234};
+constexpr unsigned long long kShareCost = 42, kGroupCost = 96, kMergeCost = 210;
+constexpr unsigned long long kPartialCost = 21;  // of 100 partials
+
+unsigned long long launch_cost(const Residency& res, unsigned long long wgs,
+                               unsigned long long steps, unsigned long long head_splits,
+                               unsigned long long most_splits) {
+  auto round_cost = [&](unsigned long long n) {
+    const unsigned long long w = (n + res.cus - 1) / res.cus;
+    return w * kGroupCost + steps * ((w <= 4 ? kStepCost[w] : kStepCost[4] * w / 4) +
+                                     kShareCost * n / res.cus);
+  };
+  const unsigned long long slots = res.cus * res.per_cu;
+  constexpr unsigned long long kPass = kCombineParts * kCombineBatch;
+  return wgs / slots * round_cost(slots) + round_cost(wgs % slots) +
+         (most_splits + kPass - 1) / kPass * kMergeCost + head_splits * kPartialCost / 100;
+}
 
 // Fills the launch's splits (a.tpw, a.first_split, a.uniform_splits) from the
 // sequences' own context lengths and returns the most of one sequence: a split gives
 // every head `ranges` token ranges, and a sequence takes as many splits as keep its
-// ranges within the launch's number of steps. That number is the smallest whose
-// workgroups fit a round of w workgroups per CU, or several rounds of as many as stay
-// resident, whichever costs least. Sized for the longest sequence instead, with equal
+// ranges within the launch's number of steps: the smallest whose workgroups fit half the
+// CUs, or 1, 2, ... per CU, whichever costs least. Sized for the longest sequence instead, with equal
 // splits per sequence, a batch of mixed lengths left most of its workgroups empty: 64
-// sequences of 128 to 32768 tokens, one kv head, 117 -> 45 us per call (185 MB of
-// packed KV); one 1500-token sequence of 8 kv heads, 18.4 -> 12.8 us (8 -> 47 splits).
+// sequences of 128 to 32768 tokens, one kv head, 117 -> 42 us per call (185 MB of packed
+// KV). (With a start-up of 3.5 us per workgroup in the cost, 32 sequences of 256 tokens, 8
+// heads, took 2 splits each instead of 4, 18.0 us instead of 16.3, and one of 16384 tokens,
+// 1 head, 256 splits instead of 128, 16.7 us instead of 14.0.)
 unsigned int plan_splits(AttnArgs& a, const Shape& sh, const unsigned long long* ctx,
                          unsigned int count, unsigned long long max_ctx) {
   const Residency res = residency();
   const unsigned long long groups = sh.groups;
-  const unsigned long long limit = max_launch_splits(count, a.kv_heads, max_ctx);
+  const unsigned long long limit =
+      std::max<unsigned long long>(max_launch_splits(count, a.kv_heads, max_ctx), count);
   const unsigned int round = sh.ranges * kStep;  // tokens of a split with one step per range
+  double half[kMaxSeqs];
   unsigned long long total = 0;
-  for (unsigned int r = 0; r < count; ++r) total += ctx[r];
+  for (unsigned int r = 0; r < count; ++r) {
+    half[r] = (double)ctx[r] - 0.5;
+    total += ctx[r];
+  }
   // steps per range: with one split per sequence, and with the most splits
   const unsigned int most = (unsigned int)((max_ctx + round - 1) / round);
   const unsigned int least = (most + kMaxSplits - 1) / kMaxSplits;
   unsigned int best = most;
   unsigned long long best_cost = ~0ull;
-  // k rounds of w workgroups per CU: w = 1, 2, ... for one round, then k = 2, 3
-  for (unsigned long long c = 1; c < res.per_cu + 3; ++c) {
-    const unsigned long long w = std::min(c, res.per_cu);
-    const unsigned long long k0 = std::max<unsigned long long>(
-        1, (count * groups + res.cus * w - 1) / (res.cus * w));
-    const unsigned long long k = k0 + (c - w);
-    if (w < res.per_cu && k > 1) continue;
+  // k workgroups per CU, from half the CUs (k = 0) or one split per sequence up to two
+  // rounds more
+  const unsigned long long k0 = count * groups <= res.cus / 2
+                                    ? 0
+                                    : (count * groups + res.cus - 1) / res.cus;
+  for (unsigned long long k = k0; k <= k0 + 2 * res.per_cu; ++k) {
     const unsigned long long fit =
-        std::min(k * res.cus * w / groups, std::max<unsigned long long>(limit, count));
+        std::min((k ? k * res.cus : res.cus / 2) / groups, limit);
     // smallest number of steps per range whose splits fit: between the even share of
     // all tokens and that of all but one split per sequence
     unsigned int lo = std::max<unsigned int>(
@@ -897,18 +923,20 @@ unsigned int plan_splits(AttnArgs& a, const Shape& sh, const unsigned long long*
     }
     while (lo < hi) {
       const unsigned int mid = lo + (hi - lo) / 2;
-      if (count_splits(ctx, count, mid * round) <= fit)
+      if (count_splits(half, count, mid * round) <= fit)
         hi = mid;
       else
         lo = mid + 1;
     }
-    const unsigned long long step_cost =
-        w < sizeof(kStepCost) / sizeof(kStepCost[0]) ? kStepCost[w] : kStepCost[4] * w / 4;
-    const unsigned long long cost = k * (kRoundCost + w * kGroupCost + lo * step_cost);
+    if (lo == best && best_cost != ~0ull) continue;  // more workgroups than there are splits
+    const unsigned long long splits = count_splits(half, count, lo * round);
+    const unsigned long long cost = launch_cost(res, splits * groups, lo, splits * a.kv_heads,
+                                                (most + lo - 1) / lo);
     if (cost < best_cost) {
       best_cost = cost;
       best = lo;
     }
+    if (lo == least || fit == limit) break;
   }
   // even ranges within each sequence
   unsigned int splits = 0, largest = 0, smallest = ~0u;
