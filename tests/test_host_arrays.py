@@ -45,3 +45,37 @@ def test_attention_bounds(contexts, heads, block_tokens):
     assert not fits(offsets, contexts, 0, heads, end)[0]
     assert not fits(offsets, contexts, block_tokens, 0, end)[0]
     assert not fits(offsets, contexts, block_tokens, heads, end, head_dim=64)[0]
+
+
+class RecordingLibrary:
+    """Stands in for the C library: notes which entry is called, with what result."""
+
+    def __init__(self, results):
+        self.results, self.calls = results, []
+
+    def __getattr__(self, name):
+        if name not in self.results:
+            raise AttributeError(name)
+
+        def entry(*args):
+            self.calls.append(name)
+            return self.results[name]
+
+        return entry
+
+
+@pytest.mark.parametrize("block_words,blocks,entries", [
+    (1024, 3, ["tile"]), (16384, 256, ["tile"]), (640, 3, ["runs"]), (8, 256, ["runs"]),
+    (1032, 2, ["runs"]), (12, 3, []), (1024, 257, []), (640, 257, [])])
+@pytest.mark.parametrize("answer", [64, 0, -1])
+def test_one_host_table_entry_per_geometry(block_words, blocks, entries, answer):
+    """A host block table is offered to the entry of its geometry and to no other."""
+    torch = pytest.importorskip("torch")
+    name = {"tile": "decode_x_host_blocks", "runs": "decode_x_host_runs"}
+    lib = RecordingLibrary({n: answer for n in name.values()})
+    source, out = torch.zeros(4, dtype=torch.uint8), torch.zeros((2, 4, 4), dtype=torch.bfloat16)
+    got = sz._decode_with_table(lib, name["tile"], "decode_x_blocks", list(range(blocks))[::-1],
+                                source, out, 2 * blocks * block_words, block_words, 0, (), torch)
+    assert lib.calls == [name[e] for e in entries]
+    # (a decline goes on to the device table, which this library does not have)
+    assert got == (answer if entries and answer else None)

@@ -324,19 +324,15 @@ def _decode_with_table(lib, host_name, device_name, block_ids, source, out, coun
     or None when no entry point is available."""
     common = (int(source.data_ptr()), int(source.numel()), int(out.data_ptr()), count_words,
               len(block_ids), block_words, int(out.stride(0)), int(out.stride(1)))
-    if len(block_ids) <= HOST_TABLE_BLOCKS:
-        table = None
-        for name in (host_name, host_name.replace("_host_blocks", "_host_runs")):
-            host_decode = getattr(lib, name, None)
-            if host_decode is None:
-                continue
-            if table is None:
-                table = array.array("q", block_ids)
-            copied = host_decode(*common, table.buffer_info()[0], *tail, stream)
-            if copied != 0:
-                return copied
-            if block_words % 1024 == 0:
-                break
+    # (one entry per geometry: the other one would only decline)
+    if block_words % 1024:
+        host_name = host_name.replace("_host_blocks", "_host_runs")
+    host_decode = getattr(lib, host_name, None) if block_words % 8 == 0 else None
+    if host_decode is not None and len(block_ids) <= HOST_TABLE_BLOCKS:
+        table = array.array("q", block_ids)
+        copied = host_decode(*common, table.buffer_info()[0], *tail, stream)
+        if copied != 0:
+            return copied
     device_decode = getattr(lib, device_name, None)
     if device_decode is None:
         return None
