@@ -79,3 +79,20 @@ def test_one_host_table_entry_per_geometry(block_words, blocks, entries, answer)
     assert lib.calls == [name[e] for e in entries]
     # (a decline goes on to the device table, which this library does not have)
     assert got == (answer if entries and answer else None)
+
+
+@pytest.mark.parametrize("offset,context", [
+    (1 << 64, 16), ((1 << 64) + 11, 16), (11 - (1 << 64), 16), (-1, 16),
+    (11, (1 << 64) + 16), (11, 16 - (1 << 64)), (11.0, 1e30)])
+def test_attention_declines_numbers_outside_64_bits(monkeypatch, offset, context):
+    """They reach the library neither as they are nor modulo 2^64."""
+    torch = pytest.importorskip("torch")
+    lib = RecordingLibrary({"kvq_splitzip_top16_decode_attention": 1,
+                            "kvq_splitzip_top16_decode_attention_fits": 1})
+    monkeypatch.setattr(sz, "_load", lambda: lib)
+    monkeypatch.setattr(sz, "_is_cuda", lambda tensor: True)
+    q = torch.zeros((2, 4, 128), dtype=torch.bfloat16)
+    payloads = torch.zeros(1 << 16, dtype=torch.uint8)
+    got = sz.decode_attention_top16(q, payloads, [11, offset], [16, context], 1,
+                                    tables=torch.zeros(544, dtype=torch.uint8))
+    assert got is None and lib.calls == []

@@ -239,15 +239,19 @@ def _stream_handle(device, torch) -> int:
     return int(torch.cuda.current_stream(device).cuda_stream)
 
 
-def _u64_array(values):
+def _u64_array(values, wrap=True):
     """ctypes u64 array of a sequence of integers. ``array`` converts 64 Python ints in
-    about a microsecond, a ctypes array from ``map(int, values)`` in 3; what it does not
-    take (numbers that ``int()`` truncates, negative ones, which wrap) goes the slow way."""
+    about a microsecond, a ctypes array from ``map(int, values)`` in 6; what it does not
+    take (numbers that ``int()`` truncates, ones outside 64 bits) goes the slow way. The
+    latter wrap, or without ``wrap`` give ``None``."""
     n = len(values)
     try:
         return (ctypes.c_ulonglong * n).from_buffer(array.array("Q", values))
     except (TypeError, OverflowError, ValueError):
-        return (ctypes.c_ulonglong * n)(*map(int, values))
+        whole = list(map(int, values))
+        if not wrap and not all(0 <= v < 1 << 64 for v in whole):
+            return None
+        return (ctypes.c_ulonglong * n)(*whole)
 
 
 # ---------------------------------------------------------------------------
@@ -1176,10 +1180,11 @@ def decode_attention_top16(q, payloads, payload_offsets, context_tokens, kv_head
         return None
     if not batch:
         raise ValueError("no sequences")
-    offs, ctxs = _u64_array(payload_offsets), _u64_array(context_tokens)
+    offs, ctxs = _u64_array(payload_offsets, False), _u64_array(context_tokens, False)
     need = ctypes.c_ulonglong()
-    if not fits(offs, ctxs, batch, int(block_tokens), kv_heads, head_dim, payloads.numel(),
-                ctypes.byref(need)):
+    if offs is None or ctxs is None or \
+            not fits(offs, ctxs, batch, int(block_tokens), kv_heads, head_dim, payloads.numel(),
+                     ctypes.byref(need)):
         return None
     need = need.value
     if tables is None:
