@@ -1,9 +1,9 @@
 """Layers whose block words are a multiple of 8 but not of 1024 (the run geometry of the
 tile kernels): every codec's payloads byte for byte with the oracle's and the decode
 into other blocks word for word. Requests end on both sides of a 512-word run row, a
-1024-word wave and a 4096-word tile; exponents are natural, escape-dense (tiles past
-the staged escapes are scanned again) or overflow the Top-16 capacity. Blocks of the
-layer outside the requests stay untouched."""
+1024-word wave and a 4096-word tile; exponents are natural, escape-dense (a tile of each
+plane past the staged escapes is scanned again) or overflow the Top-16 capacity. Blocks
+of the layer outside the requests stay untouched."""
 
 import numpy as np
 import pytest
@@ -32,17 +32,11 @@ def sz():
 def make(bw, kind, seed):
     """(layer words, sender tables, receiver tables, codebook)."""
     rng = np.random.default_rng(seed)
-    counts = [max(3, t // bw) for t in (500, 1024, 4096, 4608, 13000)]
+    # 'dense': a longest request with room for more escapes than one tile stages
+    counts = [max(3, t // bw) for t in (500, 1024, 4096, 4608, 64000 if kind == "dense" else 13000)]
     pool = sum(counts) + 4
     values = rng.standard_normal((2, pool, bw)).astype(np.float32)
     words = (values.view(np.uint32) >> 16).astype(np.uint16)
-    if kind != "natural":
-        # 'dense': one request's words in one tile-long stretch all off the codebook
-        # (still within the payload's capacity only for the long requests)
-        flat = words.reshape(-1)
-        share = 0.003 if kind == "dense" else 0.05
-        hit = rng.random(flat.size) < share
-        flat[hit] = (rng.integers(0x60, 0x7F, hit.sum()) << 8).astype(np.uint16)
 
     def tables():
         ids, at, out = rng.permutation(pool).tolist(), 0, []
@@ -52,16 +46,33 @@ def make(bw, kind, seed):
         return out
 
     send, recv = tables(), tables()
+    if kind != "natural":
+        hit = rng.random(words.shape) < (0.003 if kind == "dense" else 0.05)
+        if kind == "dense":
+            hit[:, send[-1]] = False
+        words[hit] = (rng.integers(0x60, 0x7F, hit.sum()) << 8).astype(np.uint16)
     if kind == "dense":
-        # 150 escapes in a row in the longest request: more than a tile stages, within
-        # its capacity where the request is long enough
-        words[0, send[-1][0], :min(bw, 150)] = 0x7F00
+        # one tile of each plane with more escapes than are staged, in two places of it
+        request = words[:, send[-1]].reshape(2, -1)
+        request[:, 4096 + 300:4096 + 400] = 0x7F00
+        request[:, 4096 + 3900:4096 + 3980] = 0xFF00
+        words[:, send[-1]] = request.reshape(2, -1, bw)
     book = b""
     for plane in range(2):
         count = np.bincount((words[plane].reshape(-1) >> 7) & 0xFF, minlength=256)
         count[0xC0:] = 0
         book += bytes(sorted(range(256), key=lambda e: (-count[e], e))[:16])
     return words, send, recv, book
+
+
+def escapes_of_tiles(words, book):
+    """Escapes of every 4096-word tile of a request (2, words of a plane)."""
+    counts = []
+    for plane in range(2):
+        miss = ~np.isin((words[plane] >> 7) & 0xFF, np.frombuffer(book[16 * plane:16 * plane + 16],
+                                                                  dtype=np.uint8))
+        counts += [int(miss[at:at + 4096].sum()) for at in range(0, miss.size, 4096)]
+    return counts
 
 
 def to_gpu(words):
@@ -97,6 +108,9 @@ def test_top16(sz, bw, kind):
         assert bytes(host[a:a + batch.encoded_bytes[r]]) == bytes(want), r
         ok.append(want[0] == 5)
     assert (host[:batch.out_offsets[0]] == 0x5A).all()
+    if kind == "dense":
+        # scanned again and placed: more escapes than a tile stages (128), no overflow
+        assert max(escapes_of_tiles(words[:, send[-1]].reshape(2, -1), book)) > 128 and ok[-1]
     target = torch.zeros_like(layer)
     assert sz.decode_top16_paged(out, batch.out_offsets, batch.encoded_bytes, target,
                                  sz.PagedBatch(recv, bw, "cuda"), codebooks=book) == \
@@ -281,3 +295,31 @@ def test_short_blocks_decode_no_slower_than_they_encode(sz, bw):
     times = time_of(encode), time_of(decode)
     print("[case] runs short blocks", bw, "encode, decode (us)", times, flush=True)
     assert times[1] <= 1.25 * times[0], times
+
+
+@pytest.mark.parametrize("bw", [24, 48, 640, 1024])
+def test_code_table_off_four_byte_alignment(sz, bw):
+    """Such a table takes the 16-word lanes (block words a multiple of 16) or the generic
+    kernels."""
+    print("[case] code table at byte offset 1", bw, flush=True)
+    words, send, recv, book = make(bw, "natural", bw + 3)
+    layer = to_gpu(words)
+    batch = sz.PagedBatch(send, bw, "cuda")
+    room = torch.zeros(545, dtype=torch.uint8, device="cuda")
+    tables = room[1:]
+    tables.copy_(sz.top16_tables_for(book, layer.device, torch))
+    assert tables.data_ptr() % 4 == 1
+    out = batch.new_payload_buffer().fill_(0x5A)
+    assert sz.encode_top16_paged(layer, batch, out, batch.new_workspace(), tables=tables) == \
+        batch.total_encoded_bytes
+    host = out.cpu().numpy()
+    tab = oracle.top16_tables(book)
+    for r, t in enumerate(send):
+        a = batch.out_offsets[r]
+        want = oracle.top16_encode(words[:, t].reshape(-1), tab)
+        assert want[0] == 5 and bytes(host[a:a + batch.encoded_bytes[r]]) == bytes(want), r
+    target = torch.zeros_like(layer)
+    assert sz.decode_top16_paged(out, batch.out_offsets, batch.encoded_bytes, target,
+                                 sz.PagedBatch(recv, bw, "cuda"), tables=tables) == \
+        batch.total_raw_bytes
+    check_restored(words, send, recv, target, [True] * len(send))
