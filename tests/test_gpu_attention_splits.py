@@ -156,3 +156,27 @@ def test_number_of_splits(sz, kv_heads, contexts, least, most):
     written = int((maxima != 0x7E7E7E7E).sum())
     print("[case] attention splits", kv_heads, tokens, written / kv_heads, flush=True)
     assert written % kv_heads == 0 and least <= written // kv_heads <= most
+
+
+def test_rejected_payloads_with_more_splits_than_one_merge_pass(sz):
+    """An overflowed payload and an escape list out of order make all rows of their own
+    sequences NaN, also where four thread groups merge a sequence's splits."""
+    heads, contexts = 2, [9000, 9000, 9000]
+    kv, tables, books, batch, payloads, q = make_batch(sz, heads, contexts, 17)
+    payloads[batch.out_offsets[0]] = 255
+    at, n = batch.out_offsets[2], batch.count_words[2]
+    count = int.from_bytes(bytes(payloads[at + 1:at + 5].cpu().numpy()), "little")
+    assert count > 100
+    last = at + 5 + n + n // 2 + 5 * (count - 2)  # the last two entries swapped
+    pair = payloads[last:last + 10].clone()
+    payloads[last:last + 5], payloads[last + 5:last + 10] = pair[5:], pair[:5]
+    need = sz.decode_attention_workspace_bytes(len(contexts), heads, max(contexts))
+    workspace = torch.full((need,), 0x7E, dtype=torch.uint8, device="cuda")
+    out = sz.decode_attention_top16(q, payloads, batch.out_offsets, contexts, heads,
+                                    codebooks=books, workspace=workspace)
+    written = int((workspace.view(torch.int32)[::4 * (HEAD_DIM + 2)] != 0x7E7E7E7E).sum())
+    assert written > 16 * heads * len(contexts)  # splits of a sequence: more than one pass
+    assert torch.isnan(out[0]).all() and torch.isnan(out[2]).all()
+    ref = reference(kv, tables[1], contexts[1], q[1], heads)
+    err, scale = (out[1].double() - ref).abs().amax(dim=-1), ref.abs().amax(dim=-1)
+    assert (err <= TOL * scale).all()
