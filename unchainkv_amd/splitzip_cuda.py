@@ -328,10 +328,13 @@ def _decode_with_table(lib, host_name, device_name, block_ids, source, out, coun
     or None when no entry point is available."""
     common = (int(source.data_ptr()), int(source.numel()), int(out.data_ptr()), count_words,
               len(block_ids), block_words, int(out.stride(0)), int(out.stride(1)))
-    # (one entry per geometry: the other one would only decline)
+    host_decode = getattr(lib, host_name, None)
     if block_words % 1024:
-        host_name = host_name.replace("_host_blocks", "_host_runs")
-    host_decode = getattr(lib, host_name, None) if block_words % 8 == 0 else None
+        # one entry per geometry, the other one would only decline (a library without the
+        # second entry is asked as it always was)
+        runs = getattr(lib, host_name.replace("_host_blocks", "_host_runs"), None)
+        if runs is not None:
+            host_decode = runs if block_words % 8 == 0 else None
     if host_decode is not None and len(block_ids) <= HOST_TABLE_BLOCKS:
         table = array.array("q", block_ids)
         copied = host_decode(*common, table.buffer_info()[0], *tail, stream)
