@@ -8,10 +8,12 @@
 // LDS, patches the step's escapes there, and runs QK^T and PV on the MFMA units
 // with an online softmax.
 //
-// Work split (flash-decoding): one workgroup per (sequence, context split, pair of
-// kv heads); waves 0-1 walk two consecutive token ranges of the split for the first
-// head, waves 2-3 the same ranges for the second (the two heads' rows of a token
-// are adjacent in the payload and are read together), with a workgroup barrier
+// Work split (flash-decoding): every sequence has the context splits its own length
+// needs; one workgroup of four waves per (sequence, context split, pair of kv heads),
+// or one head where the head count is odd. With a pair, waves 0-1 walk two consecutive
+// token ranges of the split for the first head, waves 2-3 the same ranges for the
+// second (the two heads' rows of a token are adjacent in the payload and are read
+// together); with one head the waves walk four ranges. The waves meet at a barrier
 // every second step. Per 16-token step a wave decodes K and V into its LDS (lane l:
 // tokens l/8 and l/8 + 8, dims 16*(l%8) .. +15, so 8 lanes read a token's row),
 // patches the step's escapes there, and then:
@@ -812,8 +814,10 @@ Residency residency() {
 // workgroups of `heads` kv heads and `ranges` token ranges each. Pairs of heads where
 // they come out even (above); with an odd count the last pair would leave two waves
 // of its workgroups idle, which costs more than reading code lines that two heads
-// share twice: 27 sequences of about 17000 tokens, 3 kv heads, 135 -> 117 us per call;
-// one sequence of 32768 tokens, 1 head, 21.6 -> 19.6 us.
+// share twice: 16 sequences of 16384 tokens, 3 kv heads, 77.6 us in pairs, 62.9 us so; one
+// of 8192 tokens, 1 head, 15.7 and 12.5 us. Over contexts of 64 to 32768 tokens and 1 to 64
+// sequences: 3 heads 7 % on average, 1 head 4 %, 7 heads 3 %, 5 heads 1 % (large equal
+// batches of five heads would be 3 to 8 % faster in pairs).
 struct Shape {
   unsigned long long groups;
   unsigned int heads, ranges;

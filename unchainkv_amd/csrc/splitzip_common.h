@@ -381,7 +381,9 @@ __device__ __forceinline__ unsigned long long wave_source(const LaunchArgs& a, c
 // on a multiple of 8 words, so runs, not waves, are active or not. Against the generic
 // palette and torch-op kernels, which take a word (or 16) per thread with 64-bit
 // divisions and byte accesses: fixed6 encode + decode of 64 MB with 7680-word blocks
-// 1386 -> 65.5 us.
+// 975 -> 63.2 us, with 512-word blocks 522 -> 68 us; against the lanes kernels (16 words
+// per lane), Top-16 of 64 MB with 512-word blocks: encode 30.8 -> 24.8, decode 26.8 -> 25.9
+// us, with 640-word ones 30.7 -> 25.0 and 26.1 -> 25.8.
 
 // The layout's share of the rule: whole 16-byte runs of the layer.
 inline bool run_geometry(unsigned long long kv_ptr, unsigned long long plane_stride,
@@ -397,7 +399,8 @@ inline bool run_geometry(unsigned long long kv_ptr, unsigned long long plane_str
 // lane picks one by a compare. Smaller ones: a 24-bit division of the run's distance
 // from the first block and a gathered id load per run. With a 64-bit multiply-high
 // division and a gathered id per run at every size, the Top-16 encode + decode call of
-// 65.6 MB with 7680-word blocks took 61.4 us instead of 58.1.
+// 65.6 MB with 7680-word blocks took 61.4 us instead of 58.1 (54.6 with both runs' loads
+// in one branch, load_runs16).
 template <typename BaseOf>
 __device__ __forceinline__ void run_offsets(const EncodeGeom& geo, unsigned int first,
                                             unsigned int last, unsigned int lane,

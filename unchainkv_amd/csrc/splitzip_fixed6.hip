@@ -134,8 +134,8 @@ constexpr unsigned int kSpanMaxShift = 7;  // 128 tiles: 64 chunks per wave, one
 
 // kRuns: the run geometry with blocks of at least 1024 words. A chunk then lies in at
 // most two blocks, so a lane looks up two addresses per chunk, and a plane's last chunk
-// may hold fewer words (64 MB of 7680-word blocks, encode + decode: 71.3 us with masks per
-// tile and a reduce, 65.5 us so).
+// may hold fewer words (64 MB of 7680-word blocks in 4 requests, encode: 43.9 us with masks
+// per tile and a reduce, 41.1 us so).
 template <bool kIds, bool kRuns>
 __global__ __launch_bounds__(kSpanWaves * kWave) void palette_presence_span(
     LaunchArgs a, EncodeGeom geo, unsigned int* masks, unsigned int span_shift) {
