@@ -487,7 +487,9 @@ long long kvq_splitzip_top16_writeback_paged(
  * fails.
  * ---------------------------------------------------------------------------- */
 
-/* Workspace bytes kvq_splitzip_top16_decode_attention needs (split partials). */
+/* Workspace bytes kvq_splitzip_top16_decode_attention needs (split partials). Grows with
+ * batch and max_ctx at a given kv_heads, not with kv_heads: a workspace for the largest
+ * batch and context serves smaller ones of its own head count. */
 unsigned long long kvq_splitzip_top16_decode_attention_workspace_bytes(
     unsigned long long batch, unsigned long long kv_heads, unsigned long long max_ctx);
 

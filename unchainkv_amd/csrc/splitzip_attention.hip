@@ -886,7 +886,7 @@ unsigned long long launch_cost(const Residency& res, unsigned long long wgs,
 // ranges within the launch's number of steps: the smallest whose workgroups fit half the
 // CUs, or 1, 2, ... per CU, whichever costs least. Sized for the longest sequence instead, with equal
 // splits per sequence, a batch of mixed lengths left most of its workgroups empty: 64
-// sequences of 128 to 32768 tokens, one kv head, 117 -> 42 us per call (185 MB of packed
+// sequences of 128 to 32768 tokens, one kv head, 117 -> 41 us per call (185 MB of packed
 // KV). (With a start-up of 3.5 us per workgroup in the cost, 32 sequences of 256 tokens, 8
 // heads, took 2 splits each instead of 4, 18.0 us instead of 16.3, and one of 16384 tokens,
 // 1 head, 256 splits instead of 128, 16.7 us instead of 14.0.)
