@@ -269,9 +269,9 @@ __global__ __launch_bounds__(kThreads) void palette_reduce(LaunchArgs a, unsigne
 // of them, lane l the quads l & 1 of every 32nd mask from its l / 2-th on. Issued before
 // the tile's words, so that the OR and the palette (rotations, scalar reads, a barrier, a
 // rank per byte) run while those are in flight; after them, behind a wait for both, a
-// fixed5 encode of 200 MB in 40 requests took 107.8 us instead of 105.8 (its kernel is the
-// longer one of two), of 64 MB in 60 requests 38.4 instead of 37.4, and a fixed6 encode of
-// 200 MB in 40 requests 106.7 instead of 103.3 (1024-word blocks).
+// fixed5 encode of 200 MB in 40 requests took 107.8 us instead of 105.8, of 64 MB in 60
+// requests 38.4 instead of 37.4, and a fixed6 encode of 200 MB in 40 requests 106.7
+// instead of 103.3 (1024-word blocks).
 constexpr unsigned int kMaskQuads = kSpanMasks / 128;
 __device__ __forceinline__ void load_masks(const unsigned int* masks, unsigned int count,
                                            u32x4 (&part)[kMaskQuads]) {
